@@ -1,0 +1,592 @@
+// chp_kernels.h -- the kernels of libcannon_hip.so.  The narrowphase resolvers, which take most of
+// the compile time, are instantiated in chp_narrow_kernels.hip (one object per precision); every
+// other kernel in chp_api.hip.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "../../include/cannon_hip.h"
+#include "chp_build.h"
+#include "chp_stages.h"
+#include "chp_events.h"
+#include "chp_query.h"
+#include "chp_split.h"
+
+namespace chp {
+
+// One kernel per stage, one workgroup per listed world.  The batched path launches each stage
+// once over every world of the batch; the plain path launches them for one world at a time.
+#define CHP_WORLD_PROLOGUE                                          \
+  const DevWorld<R>& W = worlds[list[blockIdx.x]];                  \
+  if (block_bcast(W.counters[C_STATUS], sh) != 0) return;
+
+// gravity / solve mass / AABBs, broadphase and the collideConnected filter.  One kernel per
+// broadphase kind (each holds only its code and registers), each skipping the other kind's
+// worlds.  Dynamic LDS holds the naive broadphase's body data of worlds with at most lds_nb
+// bodies.
+template <typename R, bool SAP>
+__global__ __launch_bounds__(256) void k_bp(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                            int lds_nb) {
+  __shared__ int sh[256];
+  extern __shared__ double lds_d[];
+  CHP_WORLD_PROLOGUE
+  if ((W.broadphase == CHP_BROADPHASE_SAP) != SAP) return;
+  if (threadIdx.x == 0) {
+    W.counters[C_STAGING] = 0;
+    if (W.ev_mask) W.ev_ctl[EV_JT] = 0;
+  }
+  if (W.nb >= BP_BIG) return;  // the grid-wide kernels below take large worlds
+  st_prestep<R, SAP>(W);
+  __syncthreads();
+  bool ok;
+  if constexpr (SAP) {
+    ok = st_bp_sap(W, sh);
+  } else {
+    BpLds<R> L;
+    if (W.nb <= lds_nb) {
+      L.carve(lds_d, lds_nb);
+      ok = st_bp_naive<R, true>(W, sh, L);
+    } else {
+      ok = st_bp_naive<R, false>(W, sh, L);
+    }
+  }
+  if (ok) st_filter(W);
+}
+
+// large worlds (at least BP_BIG bodies): prestep, SAP sort and pair passes over the grid.
+// spans: (list index, first row) per BP_SPAN rows; tiles: (list index, first position) per
+// SAP_TILE keys of the SAP worlds; bigw: list indices of the large worlds.
+#define CHP_SPAN_PROLOGUE(tab)                                      \
+  const int2 sp = tab[blockIdx.x];                                  \
+  const DevWorld<R>& W = worlds[list[sp.x]];                        \
+  if (W.counters[C_STATUS] != 0) return;
+
+template <typename R>
+__global__ __launch_bounds__(64) void k_big_prestep(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                    const int2* __restrict__ spans) {
+  CHP_SPAN_PROLOGUE(spans)
+  const int i = sp.y + threadIdx.x;
+  if (i < W.nb) prestep_body(W, i);
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_sap_tile(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                  const int2* __restrict__ tiles, int apply) {
+  __shared__ unsigned long long lk[SAP_TILE];
+  __shared__ int lord[SAP_TILE];
+  CHP_SPAN_PROLOGUE(tiles)
+  sap_tile(W, sp.y, lk, lord, apply != 0);
+}
+template <typename R>
+__global__ __launch_bounds__(64) void k_sap_merge(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                  const int2* __restrict__ spans, int w, int src, int apply) {
+  CHP_SPAN_PROLOGUE(spans)
+  const int g = sp.y + threadIdx.x;
+  if (W.broadphase == CHP_BROADPHASE_SAP && g < W.nb) sap_merge(W, g, w, src, apply != 0);
+}
+// pass 0 counts the pairs of each row into cnt; pass 1 writes them from the scanned offsets.
+// Four workgroups per span, BP_ROWS rows each, one wave per row.
+constexpr int BP_ROWS = BP_SPAN / 4;
+template <typename R>
+__global__ __launch_bounds__(256) void k_big_rows(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                  const int2* __restrict__ spans, int emit) {
+  const int2 sp = spans[blockIdx.x >> 2];
+  const DevWorld<R>& W = worlds[list[sp.x]];
+  if (W.counters[C_STATUS] != 0) return;
+  const int r0 = sp.y + BP_ROWS * (int)(blockIdx.x & 3), end = min(r0 + BP_ROWS, W.nb);
+  for (int k = r0 + (int)(threadIdx.x >> 6); k < end; k += 4) {
+    if (emit) {
+      big_row(W, k, true, W.cnt[k]);
+    } else {
+      int c = big_row(W, k, false, 0);
+      if ((threadIdx.x & 63) == 0) W.cnt[k] = c;
+    }
+  }
+}
+template <typename R>
+__global__ __launch_bounds__(1024) void k_big_scan(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                   const int* __restrict__ bigw) {
+  __shared__ int sh[1024];
+  const DevWorld<R>& W = worlds[list[bigw[blockIdx.x]]];
+  if (block_bcast(W.counters[C_STATUS], sh) != 0) return;
+  const int P = array_exscan(W.cnt, W.nb, sh);
+  if (threadIdx.x == 0) {
+    W.counters[C_PAIRS] = P;
+    if (P > W.pair_cap) ws_fail(W.counters, WS_PAIRS);
+  }
+}
+
+// narrowphase class counts and queue placement of a large world's pairs: the world's spans are
+// its K workers, worker k takes pairs k * 256 + t, stride K * 256.  Counts add into the world's
+// qcls entries (zeroed by k_narrow_count); placement reserves each class range per workgroup.
+template <typename R>
+__device__ __forceinline__ void big_pair_classes(const DevWorld<R>& W, int2 sp, int* sh, bool mark_filtered) {
+  const int K = (W.nb + BP_SPAN - 1) / BP_SPAN, k = sp.y / BP_SPAN, P = W.counters[C_PAIRS];
+  for (int p = k * 256 + (int)threadIdx.x; p < P; p += K * 256) {
+    int bi = W.pair_i[p], bj = W.pair_j[p];
+    if (bi < 0) {
+      if (mark_filtered) pair_counts(W, p, 0, 0);
+      continue;
+    }
+    atomicAdd(&sh[pair_class(W, bi, bj)], 1);
+  }
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_big_ncount(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                    const int2* __restrict__ spans, int* __restrict__ qcls, int n) {
+  __shared__ int sh[NP_NCLS];
+  CHP_SPAN_PROLOGUE(spans)
+  if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = 0;
+  __syncthreads();
+  big_pair_classes(W, sp, sh, true);
+  __syncthreads();
+  if (threadIdx.x < NP_NCLS && sh[threadIdx.x]) atomicAdd(&qcls[threadIdx.x * n + sp.x], sh[threadIdx.x]);
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_big_nplace(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                    const int2* __restrict__ spans, int* __restrict__ qcls,
+                                                    int2* __restrict__ q, int n) {
+  __shared__ int sh[NP_NCLS];
+  CHP_SPAN_PROLOGUE(spans)
+  if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = 0;
+  __syncthreads();
+  big_pair_classes(W, sp, sh, false);
+  __syncthreads();
+  if (threadIdx.x < NP_NCLS)
+    sh[threadIdx.x] = sh[threadIdx.x] ? atomicAdd(&qcls[threadIdx.x * n + sp.x], sh[threadIdx.x]) : 0;
+  __syncthreads();
+  const int K = (W.nb + BP_SPAN - 1) / BP_SPAN, k = sp.y / BP_SPAN, P = W.counters[C_PAIRS], wid = list[sp.x];
+  for (int p = k * 256 + (int)threadIdx.x; p < P; p += K * 256) {
+    int bi = W.pair_i[p], bj = W.pair_j[p];
+    if (bi < 0) continue;
+    q[atomicAdd(&sh[pair_class(W, bi, bj)], 1)] = make_int2(wid, p);
+  }
+}
+
+// rows of a large world: the offsets and counters in one workgroup per world, then the rows of
+// its pairs and constraints over its spans (worker k of K as above)
+template <typename R>
+__global__ __launch_bounds__(1024) void k_big_rowscan(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                      const int* __restrict__ bigw) {
+  __shared__ int sh[1024];
+  const DevWorld<R>& W = worlds[list[bigw[blockIdx.x]]];
+  if (block_bcast(W.counters[C_STATUS], sh) != 0) return;
+  const int P = W.counters[C_PAIRS];
+  const int F = array_exscan(W.pf_cnt, P, sh);
+  const int C = array_exscan(W.pc_off, P, sh);
+  const int E = F + C + W.ncrows;
+  if (threadIdx.x == 0) {
+    if (E > W.row_cap) {
+      W.counters[C_ROWS] = E;
+      ws_fail(W.counters, WS_ROWS);
+    } else {
+      rows_done(W, P, F, C, E);
+    }
+  }
+}
+
+
+// integration of a large world's bodies over its spans; a non-finite pose is noted in
+// C_POSTFAIL and raised by k_post, which also advances the step counter
+template <typename R>
+__global__ __launch_bounds__(64) void k_big_post(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                 const int2* __restrict__ spans, double dt) {
+  CHP_SPAN_PROLOGUE(spans)
+  const int i = sp.y + threadIdx.x;
+  if (i < W.nb && !post_body(W, i, (R)dt, W.counters[C_ROWS], post_qn(W))) W.counters[C_POSTFAIL] = 1;
+}
+
+// narrowphase: per-class pair counts per world, class-major offsets, placement in the queue,
+// then one pair per thread over the thread classes and one pair per wave over the wave class,
+// each grid-wide over the whole batch.  qcls: class-major, qcls[c * n + list index]; bounds:
+// NP_NCLS + 1 ints, then the wave classes' NP_NTICKET pair tickets.
+template <typename R>
+__global__ __launch_bounds__(256) void k_narrow_count(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                      int* __restrict__ qcls, int n) {
+  __shared__ int sh[64];
+  int* cnt = qcls + blockIdx.x;
+  const DevWorld<R>& W = worlds[list[blockIdx.x]];
+  if (block_bcast(W.counters[C_STATUS], sh) != 0 || W.nb >= BP_BIG) {  // large worlds: k_big_ncount
+    if (threadIdx.x < NP_NCLS) cnt[threadIdx.x * n] = 0;
+    return;
+  }
+  st_narrow_count(W, cnt, n, sh);
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_narrow(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                const int* __restrict__ qcls, int2* __restrict__ q, int n) {
+  __shared__ int sh[64];
+  CHP_WORLD_PROLOGUE
+  if (W.nb >= BP_BIG) return;  // k_big_nplace
+  st_narrow_place(W, list[blockIdx.x], qcls + blockIdx.x, n, q, sh);
+}
+// classes whose resolvers clip polygons (convex-convex, and the mixed class) hold the clip
+// polygons of the block's 64 lanes in LDS
+constexpr bool cls_clips(int c) { return c == NP_CC || c == NP_OTHER; }
+template <typename R, int CLS>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_narrow_cls(const DevWorld<R>* __restrict__ worlds, const int2* __restrict__ q,
+                                                   const int* __restrict__ bounds, double dt) {
+  __shared__ f3 cb[cls_clips(CLS) ? 2 * CLIP_THREAD * 64 : 1];
+  st_narrow_class<R, CLS>(worlds, q, bounds, (R)dt, cb);
+}
+template <typename R, int CLS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_narrow_wave(const DevWorld<R>* __restrict__ worlds, const int2* __restrict__ q,
+                                                     int* __restrict__ bounds, double dt) {
+  __shared__ f3 ws[4][NPCtx<R, true>::WS_F3];            // one LDS workspace per wave
+  __shared__ ContactRec<R> loc[4][WAVE_KMAX];             // and one contact buffer
+  constexpr unsigned kinds = CLS == NP_WHC ? (NK_CC | NK_HC | NK_SH) : NK_ALL;
+  st_narrow_wave<R, kinds>(worlds, q + bounds[CLS], bounds[CLS + 1] - bounds[CLS], bounds + NP_NCLS + 1 + (CLS - NP_WHC),
+                           (R)dt, ws[threadIdx.x >> 6],
+                           loc[threadIdx.x >> 6], WAVE_KMAX);
+}
+
+
+// equations: the row offsets per world (large worlds: k_big_rowscan), then the friction and
+// contact rows of every queued pair (one pair per thread over the whole batch), then the joint
+// rows (one workgroup per world)
+template <typename R>
+__global__ __launch_bounds__(128) void k_rows(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list) {
+  __shared__ int sh[128];
+  CHP_WORLD_PROLOGUE
+  if (W.nb >= BP_BIG) return;
+  st_rowscan(W, sh);
+}
+// MODE ROWS_AB: the rows' body pairs only (before the level schedule); ROWS_GS: the rows
+// themselves, as GS records at their level-order positions (after it)
+template <typename R, int MODE>
+__global__ __launch_bounds__(64) void k_pair_rows(const DevWorld<R>* __restrict__ worlds, const int2* __restrict__ q,
+                                                  const int* __restrict__ bounds, double dt, int keep) {
+  const int n = bounds[NP_NCLS];
+  const int g = (int)(blockIdx.x * blockDim.x + threadIdx.x), ng = (int)(gridDim.x * blockDim.x);
+  for (int i = g; i < n; i += ng) {
+    const int2 e = q[i];
+    const DevWorld<R>& W = worlds[e.x];
+    if (W.counters[C_STATUS] != 0) continue;
+    pair_rows<R, MODE>(W, e.y, W.counters[C_FROWS], (R)dt, keep != 0);
+  }
+}
+template <typename R, int MODE>
+__global__ __launch_bounds__(64) void k_joint_rows(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                   double dt, int keep) {
+  const DevWorld<R>& W = worlds[list[blockIdx.x]];
+  if (W.ncons == 0 || W.counters[C_STATUS] != 0) return;
+  const int F = W.counters[C_FROWS], C = W.counters[C_CROWS];
+  for (int c = threadIdx.x; c < W.ncons; c += blockDim.x)
+    constraint_rows<R, MODE>(W, c, F + C + W.c_row_off[c], (R)dt, keep != 0);
+}
+
+// Levels and GS sweeps run one large world per workgroup (the first nbig entries of the list)
+// and one small world (at most SMALL_NB bodies) per wave, blockDim / 64 of them per workgroup.
+constexpr int SMALL_NB = 128;        // bodies of a world run by one wave
+constexpr int LS_BIG = 2048, LS_SMALL = 1024;   // level starts kept in LDS
+constexpr int LS_LEVELS = 4096;                  // the level histogram of a large world's level stage
+// bodies of a large world whose GS / level state fits in LDS: at least 512, up to the largest
+// large world of the launch (the launch's dynamic LDS is sized for it), at most what a
+// workgroup's LDS holds beside the level starts and the static arrays (4 KiB kept free)
+constexpr int BIG_NB_LDS_MIN = 512;
+static int big_lds_cap(int nbig, int max_nb, size_t max_lds) {
+  const int most = (int)((max_lds - 4096 - (size_t)LS_BIG * sizeof(int)) / (8 * sizeof(float)));
+  return nbig ? std::max(BIG_NB_LDS_MIN, std::min(max_nb, most)) : BIG_NB_LDS_MIN;
+}
+
+// bodies of a large world whose level walk keeps each body's last level in LDS (4 bytes per
+// body): up to the largest large world of the launch, at most what a workgroup's LDS holds beside
+// the level histogram and the static arrays (4 KiB kept free)
+static int levels_lds_cap(int nbig, int max_nb, size_t max_lds) {
+  const int most = (int)((max_lds - 4096 - (size_t)LS_LEVELS * sizeof(int)) / sizeof(int));
+  return nbig ? std::max(BIG_NB_LDS_MIN, std::min(max_nb, most)) : BIG_NB_LDS_MIN;
+}
+
+// dynamic LDS of k_levels / k_gs for a workgroup of bd threads (big_cap: as levels_lds_cap /
+// big_lds_cap)
+static size_t lds_levels(int bd, int big_cap) {
+  size_t big = (size_t)(big_cap + LS_LEVELS) * sizeof(int), small = (size_t)(SMALL_NB + LS_SMALL) * sizeof(int);
+  return std::max(big, (bd / 64) * small);
+}
+static size_t lds_gs(int bd, int big_cap) {
+  size_t big = (size_t)big_cap * 8 * sizeof(float) + LS_BIG * sizeof(int);
+  size_t small = (size_t)SMALL_NB * 8 * sizeof(float) + LS_SMALL * sizeof(int);
+  return std::max(big, (bd / 64) * small);
+}
+
+// the world of this workgroup (large) or of this wave (small); -1: none / quarantined
+template <typename R>
+__device__ __forceinline__ int group_world(const DevWorld<R>* worlds, const int* list, int nbig, int n, int* sh,
+                                           int& wave) {
+  if ((int)blockIdx.x < nbig) {
+    wave = -1;
+    int id = list[blockIdx.x];
+    return block_bcast(worlds[id].counters[C_STATUS], sh) != 0 ? -1 : id;
+  }
+  wave = threadIdx.x >> 6;
+  int idx = nbig + ((int)blockIdx.x - nbig) * (int)(blockDim.x >> 6) + wave;
+  if (idx >= n) return -1;
+  int id = list[idx];
+  return worlds[id].counters[C_STATUS] != 0 ? -1 : id;
+}
+
+// GS dependency levels of the step's rows and the level-ordered GS records
+template <typename R>
+__global__ __launch_bounds__(256) void k_levels(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                int nbig, int n, int big_cap, int gather) {
+  __shared__ int sh[256];
+  extern __shared__ int lds_i[];
+  int wave;
+  int id = group_world(worlds, list, nbig, n, sh, wave);
+  if (id < 0) return;
+  const DevWorld<R>& W = worlds[id];
+  if (W.solver_kind == CHP_SOLVER_SPLIT) return;   // k_split_prep orders its rows
+  if (wave < 0) {
+    if (W.nb <= big_cap) st_levels<R, GBlock, true>(W, GBlock(), sh, lds_i, lds_i + big_cap, LS_LEVELS, gather != 0);
+    else st_levels<R, GBlock, false>(W, GBlock(), sh, W.tmp, nullptr, 0, gather != 0);
+  } else {
+    int* base = lds_i + wave * (SMALL_NB + LS_SMALL);
+    if (W.nb <= SMALL_NB) st_levels<R, GWave, true>(W, GWave(), sh, base, base + SMALL_NB, LS_SMALL, gather != 0);
+    else st_levels<R, GWave, false>(W, GWave(), sh, W.tmp, nullptr, 0, gather != 0);
+  }
+}
+
+// GS sweeps of the worlds of at most GS_SUB_MAX_NB bodies run G lanes per world, 64 / G worlds
+// per wave (a level of such a world is rarely wider than a few dozen rows, and the sweep is a
+// chain of dependent steps: packing worlds into a wave divides the instructions issued for the
+// same rows by 64 / G).  Their vlambda / wlambda and level starts live in LDS.
+#ifndef CHP_GS_SUB_MAX_NB
+#define CHP_GS_SUB_MAX_NB 512
+#endif
+constexpr int GS_SUB_MAX_NB = CHP_GS_SUB_MAX_NB;
+__host__ __device__ constexpr int gs_group(int nb) { return nb <= 64 ? 16 : nb <= 128 ? 32 : nb <= GS_SUB_MAX_NB ? 64 : 0; }
+__host__ __device__ constexpr int gs_sub_nb(int G) { return G == 16 ? 64 : G == 32 ? 128 : GS_SUB_MAX_NB; }
+__host__ __device__ constexpr int gs_sub_ls(int G) { return G == 16 ? 512 : G == 32 ? 1024 : 2048; }
+constexpr size_t gs_sub_bytes(int G) {
+  return (size_t)(64 / G) * (8 * gs_sub_nb(G) * sizeof(float) + gs_sub_ls(G) * sizeof(int));
+}
+// whether k_gs_sub runs the world (else k_gs does)
+template <typename R> __device__ __forceinline__ bool gs_sub_fits(const DevWorld<R>& W, int L) {
+  const int G = gs_group(W.nb);
+  return G != 0 && L + 1 <= gs_sub_ls(G);
+}
+
+// the list positions of a list sorted by body count (largest first): [0, blk) over
+// GS_SUB_MAX_NB bodies, [blk, s32) G = 64, [s32, s16) G = 32, [s16, n) G = 16
+struct GsSegs {
+  int blk = 0, s32 = 0, s16 = 0;
+};
+
+// the group's world: list position lo + (block b of the segment) * (64 / G) + group
+template <typename R, int G>
+__device__ __forceinline__ void gs_sub_run(const DevWorld<R>* worlds, const int* list, int lo, int hi, int b,
+                                           float* lds, int keep) {
+  const int sub = ((int)threadIdx.x & 63) / G;
+  const int idx = lo + b * (64 / G) + sub;
+  if (idx >= hi) return;
+  const DevWorld<R>& W = worlds[list[idx]];
+  if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;
+  if (gs_group(W.nb) != G || !gs_sub_fits(W, W.counters[C_LEVELS])) return;
+  float* base = lds + sub * (8 * gs_sub_nb(G) + gs_sub_ls(G));
+  st_gs<R, GSub<G>, true>(W, GSub<G>(), nullptr, nullptr, base, (int*)(base + 8 * gs_sub_nb(G)), keep != 0);
+}
+// one wave per workgroup; the workgroups are dealt to the three segments (G = 64 first: their
+// worlds have the longest chains), so that all of them run in one launch
+template <typename R>
+__global__ __launch_bounds__(64) void k_gs_sub(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                               GsSegs g, int n, int keep) {
+  extern __shared__ float4 lds_f4[];
+  float* lds = (float*)lds_f4;
+  const int b = (int)blockIdx.x;
+  const int n64 = g.s32 - g.blk, n32 = (g.s16 - g.s32 + 1) / 2;
+  if (b < n64) gs_sub_run<R, 64>(worlds, list, g.blk, g.s32, b, lds, keep);
+  else if (b < n64 + n32) gs_sub_run<R, 32>(worlds, list, g.s32, g.s16, b - n64, lds, keep);
+  else gs_sub_run<R, 16>(worlds, list, g.s16, n, b - n64 - n32, lds, keep);
+}
+
+// GS iterations of the rest.  GLOBAL = false: the worlds over GS_SUB_MAX_NB bodies whose body
+// velocities and level starts fit in LDS, one per workgroup; GLOBAL = true: every world that
+// neither this nor k_gs_sub runs, from global memory (a separate kernel, so that the common LDS
+// form keeps its own, smaller register count)
+template <typename R, bool GLOBAL>
+__global__ __launch_bounds__(256) void k_gs(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                            int nbig, int n, int big_cap, int keep) {
+  __shared__ int sh[256];
+  __shared__ double shd[256];
+  extern __shared__ float4 lds_f4[];
+  int wave;
+  int id = group_world(worlds, list, nbig, n, sh, wave);
+  if (id < 0) return;
+  const DevWorld<R>& W = worlds[id];
+  if (W.solver_kind == CHP_SOLVER_SPLIT) return;   // k_split_gs solves its islands
+  float* lds = (float*)lds_f4;
+  const int L = W.counters[C_LEVELS];
+  if (wave < 0) {
+    const bool fits = W.nb <= big_cap && L + 1 <= LS_BIG;
+    if constexpr (!GLOBAL) {
+      if (fits) st_gs<R, GBlock, true>(W, GBlock(), shd, sh, lds, (int*)(lds + 8 * big_cap), keep != 0);
+    } else {
+      if (!fits) st_gs<R, GBlock, false>(W, GBlock(), shd, sh, W.vw, nullptr, keep != 0);
+    }
+  } else {
+    if constexpr (GLOBAL) {
+      if (!gs_sub_fits(W, L)) st_gs<R, GWave, false>(W, GWave(), shd, sh, W.vw, nullptr, keep != 0);
+    }
+  }
+}
+
+// the GS stage of a list (the level schedule and the GS records are in place)
+template <typename R>
+static void launch_gs(const DevWorld<R>* dw, const int* d_list, int n, const GsSegs& g, int bcap, int bd, int keep,
+                      hipStream_t st) {
+  if (g.blk) k_gs<R, false><<<g.blk, bd, lds_gs(bd, bcap), st>>>(dw, d_list, g.blk, g.blk, bcap, keep);
+  const int nsub = (g.s32 - g.blk) + (g.s16 - g.s32 + 1) / 2 + (n - g.s16 + 3) / 4;
+  if (nsub) {
+    size_t bytes = 0;
+    if (g.s32 > g.blk) bytes = std::max(bytes, gs_sub_bytes(64));
+    if (g.s16 > g.s32) bytes = std::max(bytes, gs_sub_bytes(32));
+    if (n > g.s16) bytes = std::max(bytes, gs_sub_bytes(16));
+    k_gs_sub<R><<<nsub, 64, bytes, st>>>(dw, d_list, g, n, keep);
+  }
+  const int per = bd / 64;
+  k_gs<R, true><<<g.blk + (n - g.blk + per - 1) / per, bd, 0, st>>>(dw, d_list, g.blk, n, bcap, keep);
+}
+
+// World.step(dt, timeSinceLastCalled): the interpolated poses and World.time += the elapsed time
+template <typename R>
+__global__ __launch_bounds__(256) void k_interp(const DevWorld<R>* __restrict__ worlds, int id, double t, double elapsed) {
+  const DevWorld<R>& W = worlds[id];
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i == 0) W.wtime[0] += elapsed;
+  if (i < W.nb) interp_body(W, i, (R)t);
+}
+
+// queries: the preparation (AABBs, SAP axis list), the AABB query, the ray passes
+template <typename R>
+__global__ __launch_bounds__(1024) void k_query_prep(const DevWorld<R>* __restrict__ worlds, int id) {
+  st_query_prep(worlds[id]);
+}
+template <typename R>
+__global__ __launch_bounds__(1024) void k_aabb_query(const DevWorld<R>* __restrict__ worlds, int id, f3 lo, f3 hi,
+                                                     int* __restrict__ out, int cap, int* __restrict__ total) {
+  __shared__ int sh[1024];
+  const DevWorld<R>& W = worlds[id];
+  int carry = 0;
+  for (int k0 = 0; k0 < W.nb; k0 += blockDim.x) {
+    const int k = k0 + (int)threadIdx.x;
+    const int b = k < W.nb ? query_body(W, k) : 0;
+    const int hit = (k < W.nb && aabb_overlaps(F3<R>(W.aabb_lo, b), F3<R>(W.aabb_hi, b), lo, hi)) ? 1 : 0;
+    int t;
+    const int r = tile_exscan(hit, sh, &t);
+    if (hit && carry + r < cap) out[carry + r] = b;
+    carry += t;
+  }
+  if (threadIdx.x == 0) *total = carry;
+}
+template <typename R, int PASS>
+__global__ __launch_bounds__(64) void k_rays(const DevWorld<R>* __restrict__ worlds, int id, const chp_ray* __restrict__ rays,
+                                             int nr, int4* __restrict__ probe, int* __restrict__ cnt,
+                                             const int* __restrict__ off, chp_ray_hit* __restrict__ out) {
+  st_rays<R, PASS>(worlds[id], rays, nr, probe, cnt, off, out);
+}
+
+// SplitSolver: ids, islands and row positions (after the rows' body pairs), then the islands'
+// Gauss-Seidel (after the rows)
+template <typename R>
+__global__ __launch_bounds__(1024) void k_split_prep(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list) {
+  __shared__ int sh[1024];
+  CHP_WORLD_PROLOGUE
+  if (W.solver_kind != CHP_SOLVER_SPLIT) return;
+  st_split_prep(W, sh);
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_split_gs(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                  int keep) {
+  __shared__ int sh[256];
+  CHP_WORLD_PROLOGUE
+  if (W.solver_kind != CHP_SOLVER_SPLIT) return;
+  st_split_gs(W, keep != 0);
+}
+
+// contact-event bookkeeping after the narrowphase (worlds with events on); seed: only the key
+// sets, from the contacts the slab holds
+template <typename R>
+__global__ __launch_bounds__(1024) void k_events(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                 int seed) {
+  __shared__ int sh[1024];
+  CHP_WORLD_PROLOGUE
+  if (!W.ev_mask) return;
+  st_events(W, seed != 0, sh);
+}
+
+// the wake-up pass after the narrowphase (worlds that may hold sleeping bodies)
+template <typename R>
+__global__ __launch_bounds__(256) void k_wake(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list) {
+  __shared__ int sh[256];
+  CHP_WORLD_PROLOGUE
+  st_wake(W);
+}
+
+// velocities, damping, integration, clearForces
+template <typename R>
+__global__ __launch_bounds__(256) void k_post(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                              double dt) {
+  __shared__ int sh[256];
+  CHP_WORLD_PROLOGUE
+  if (W.nb >= BP_BIG) {  // k_big_post integrated the bodies
+    if (threadIdx.x == 0) {
+      if (W.counters[C_POSTFAIL]) {
+        W.counters[C_POSTFAIL] = 0;
+        ws_fail(W.counters, WS_NONFINITE);
+      }
+      step_done(W, dt);
+    }
+    return;
+  }
+  st_post(W, dt);
+}
+
+// broadphase only (Broadphase.collisionPairs on the current state)
+template <typename R>
+__global__ __launch_bounds__(CHP_BLOCK) void k_broadphase(const DevWorld<R>* __restrict__ worlds, int wid) {
+  __shared__ int sh[CHP_BLOCK];
+  const DevWorld<R>& W = worlds[wid];
+  if (W.broadphase == CHP_BROADPHASE_SAP) {
+    for (int i = threadIdx.x; i < W.nb; i += blockDim.x)
+      if (W.flags[i] & BF_AABB_DIRTY) { body_aabb(W, i); W.flags[i] &= ~BF_AABB_DIRTY; }
+    __syncthreads();
+    st_bp_sap(W, sh);
+  } else {
+    BpLds<R> L;
+    st_bp_naive<R, false>(W, sh, L);
+  }
+}
+
+// Narrowphase slot: contacts for the pairs in the world's pair slab, then the equations
+template <typename R>
+__global__ __launch_bounds__(64) void k_np_slot(const DevWorld<R>* __restrict__ worlds, int id, double dt,
+                                                chp_equation* __restrict__ out, int cap) {
+  __shared__ int sh[64];
+  __shared__ f3 cb[2 * CLIP_THREAD * 64];
+  const DevWorld<R>& W = worlds[id];
+  st_narrow(W, (R)dt, cb);
+  st_equations(W, (R)dt, out, cap, sh);
+}
+
+// Solver slot: rows from given equations; then k_levels / k_gs; then the velocity update
+template <typename R>
+__global__ __launch_bounds__(256) void k_solve_rows(const DevWorld<R>* __restrict__ worlds, int id,
+                                                    const chp_equation* __restrict__ eq, int n, double dt) {
+  st_solve_rows(worlds[id], eq, n, (R)dt);
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_solve_finish(const DevWorld<R>* __restrict__ worlds, int id) {
+  st_solve_finish(worlds[id]);
+}
+
+// the kernels instantiated in chp_narrow_kernels.hip
+#define CHP_NARROW_KERNELS(X, R)                                                                       \
+  X void k_narrow_cls<R, NP_SS>(const DevWorld<R>*, const int2*, const int*, double);                  \
+  X void k_narrow_cls<R, NP_SP>(const DevWorld<R>*, const int2*, const int*, double);                  \
+  X void k_narrow_cls<R, NP_SB>(const DevWorld<R>*, const int2*, const int*, double);                  \
+  X void k_narrow_cls<R, NP_SC>(const DevWorld<R>*, const int2*, const int*, double);                  \
+  X void k_narrow_cls<R, NP_PC>(const DevWorld<R>*, const int2*, const int*, double);                  \
+  X void k_narrow_cls<R, NP_CC>(const DevWorld<R>*, const int2*, const int*, double);                  \
+  X void k_narrow_cls<R, NP_OTHER>(const DevWorld<R>*, const int2*, const int*, double);               \
+  X void k_narrow_wave<R, NP_WHC>(const DevWorld<R>*, const int2*, int*, double);                      \
+  X void k_narrow_wave<R, NP_WAVE>(const DevWorld<R>*, const int2*, int*, double);
+
+}  // namespace chp
