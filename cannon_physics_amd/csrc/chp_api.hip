@@ -30,10 +30,70 @@ __global__ __launch_bounds__(1024) void k_narrow_scan(int* __restrict__ qcls, in
   st_narrow_scan(qcls, n, bounds, sh);
 }
 
-__global__ void k_gather_status(const int* const* counters, int n, int* out) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    for (int k = 0; k < C_COUNT; k++) out[i * C_COUNT + k] = counters[i][k];
+// counter words of the listed worlds; the pointers and the words are in pinned host memory
+__global__ __launch_bounds__(256) void k_gather_status(const int* const* __restrict__ counters, int n, int* __restrict__ out) {
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < n * C_COUNT) out[i] = counters[i / C_COUNT][i % C_COUNT];
+}
+
+// ---- a world's state to and from the caller's records ---------------------------------------------
+// chp_body_state is 38 words; the bodies of a workgroup are turned between their arrays and their
+// records in LDS, and one contiguous run of words goes to (PACK) or comes from the pinned host
+// buffer.  A state of a few hundred bodies is a few tens of kilobytes, so a transfer is bound by
+// latency: one launch and one wait, where a copy per array cost twelve round trips (a step and
+// the state of a 217-body world 600 -> 423 us; 60 steps of 2048 worlds and all their states
+// 439 -> 147 ms).
+struct StateArrays {
+  float* f[9];        // in record order: pos, quat, vel, avel, force, torque, iiw, aabb_lo, aabb_hi
+  int *flags, *sleep;
+  double* tls;
+  int* status;
+};
+constexpr int STATE_WORDS = sizeof(chp_body_state) / 4, STATE_BODIES = 64;
+static_assert(sizeof(chp_body_state) == 152 && offsetof(chp_body_state, aabb_needs_update) == 136 &&
+              offsetof(chp_body_state, time_last_sleepy) == 144, "the record layout k_state writes");
+template <bool PACK>
+__global__ __launch_bounds__(256) void k_state(StateArrays A, uint2* __restrict__ host, int first, int n) {
+  __shared__ uint2 rec2[STATE_BODIES * STATE_WORDS / 2];
+  unsigned* rec = (unsigned*)rec2;
+  const int b0 = (int)blockIdx.x * STATE_BODIES, cnt = min(STATE_BODIES, n - b0), tid = (int)threadIdx.x;
+  const size_t g0 = (size_t)first + b0;
+  uint2* h = host + (size_t)b0 * (STATE_WORDS / 2);
+  if constexpr (!PACK) {
+    for (int t = tid; t < cnt * (STATE_WORDS / 2); t += 256) rec2[t] = h[t];
+    if (blockIdx.x == 0 && tid == 0) *A.status = 0;   // a fresh state clears a quarantine
+    __syncthreads();
+  }
+  int off = 0;
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    const int w = k == 1 ? 4 : k == 6 ? 9 : 3;
+    unsigned* d = (unsigned*)A.f[k] + g0 * w;
+    for (int t = tid; t < cnt * w; t += 256) {
+      unsigned& r = rec[(t / w) * STATE_WORDS + off + t % w];
+      if constexpr (PACK) r = d[t];
+      else d[t] = r;
+    }
+    off += w;
+  }
+  if (tid < cnt) {
+    unsigned* r = rec + tid * STATE_WORDS + off;
+    const size_t i = g0 + tid;
+    if constexpr (PACK) {
+      const unsigned long long t = (unsigned long long)__double_as_longlong(A.tls[i]);
+      r[0] = (A.flags[i] & BF_AABB_DIRTY) ? 1u : 0u;
+      r[1] = (unsigned)A.sleep[i];
+      r[2] = (unsigned)t;
+      r[3] = (unsigned)(t >> 32);
+    } else {
+      A.flags[i] = (A.flags[i] & ~BF_AABB_DIRTY) | (r[0] ? BF_AABB_DIRTY : 0);
+      A.sleep[i] = (int)r[1];
+      A.tls[i] = __longlong_as_double((long long)((unsigned long long)r[2] | ((unsigned long long)r[3] << 32)));
+    }
+  }
+  if constexpr (PACK) {
+    __syncthreads();
+    for (int t = tid; t < cnt * (STATE_WORDS / 2); t += 256) h[t] = rec2[t];
   }
 }
 
@@ -206,9 +266,10 @@ struct chp_ctx {
   ListState second;          // the second stream's list state (see ListState)
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   bool keep_rows = false;   // steps also write row records (the capture reads them)
-  int* d_status = nullptr;
-  const int** d_cptrs = nullptr;
-  size_t d_status_cap = 0;
+  // pinned host staging of the state transfers and the status words; every user waits for its
+  // kernel before it returns, so the next one finds it free
+  char* h_stage = nullptr;
+  size_t h_stage_cap = 0;
   std::string err;
   std::mutex mu;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;  // bracket the last chp_step / chp_step_plain on the stream
@@ -664,22 +725,29 @@ template <typename R> static int prepare(chp_ctx* ctx, const uint32_t* ids, uint
   return CHP_OK;
 }
 
+// the staging buffer at least this large (powers of two from 64 KiB)
+static int ensure_stage(chp_ctx* ctx, size_t bytes) {
+  if (ctx->h_stage_cap >= bytes) return CHP_OK;
+  size_t cap = 65536;
+  while (cap < bytes) cap <<= 1;
+  if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
+  ctx->h_stage = nullptr;
+  ctx->h_stage_cap = 0;
+  HIPCHK(ctx, hipHostMalloc((void**)&ctx->h_stage, cap, hipHostMallocDefault));
+  ctx->h_stage_cap = cap;
+  return CHP_OK;
+}
+
 static int read_status(chp_ctx* ctx, const uint32_t* ids, uint32_t n, std::vector<int>& out) {
-  if (ctx->d_status_cap < n) {
-    if (ctx->d_status) (void)hipFree(ctx->d_status);
-    if (ctx->d_cptrs) (void)hipFree(ctx->d_cptrs);
-    HIPCHK(ctx, hipMalloc(&ctx->d_status, (size_t)n * C_COUNT * sizeof(int)));
-    HIPCHK(ctx, hipMalloc(&ctx->d_cptrs, (size_t)n * sizeof(int*)));
-    ctx->d_status_cap = n;
-  }
-  std::vector<const int*> ptrs(n);
+  const size_t words = (size_t)n * C_COUNT * sizeof(int);
+  int r = ensure_stage(ctx, words + (size_t)n * sizeof(int*));
+  if (r != CHP_OK) return r;
+  const int** ptrs = (const int**)(ctx->h_stage + words);
   for (uint32_t k = 0; k < n; k++) ptrs[k] = (const int*)((char*)ctx->worlds[ids[k]].mem + ctx->worlds[ids[k]].off_counters);
-  HIPCHK(ctx, hipMemcpyAsync(ctx->d_cptrs, ptrs.data(), n * sizeof(int*), hipMemcpyHostToDevice, ctx->stream));
-  k_gather_status<<<(n + 255) / 256, 256, 0, ctx->stream>>>(ctx->d_cptrs, (int)n, ctx->d_status);
+  k_gather_status<<<(n * C_COUNT + 255) / 256, 256, 0, ctx->stream>>>(ptrs, (int)n, (int*)ctx->h_stage);
   HIPCHK(ctx, hipGetLastError());
-  out.resize((size_t)n * C_COUNT);
-  HIPCHK(ctx, hipMemcpyAsync(out.data(), ctx->d_status, out.size() * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  out.assign((const int*)ctx->h_stage, (const int*)ctx->h_stage + (size_t)n * C_COUNT);
   return CHP_OK;
 }
 
@@ -1301,70 +1369,44 @@ template <typename R> static int set_capacity_t(chp_ctx* ctx, uint32_t id, uint3
 // C-ABI
 // ---------------------------------------------------------------------------------------------
 
+// bodies per transfer of a state: the staging buffer stays under 4 MiB however large the world
+constexpr int STATE_CHUNK = 16384;
 template <typename R> static int state_io(chp_ctx* ctx, uint32_t id, chp_body_state* buf, uint32_t n, bool download) {
   WorldSlot& S = ctx->worlds[id];
   DevWorld<R>& D = dev_of<R>(S);
   if (n < (uint32_t)S.nb) return fail(ctx, CHP_E_CAPACITY, "state buffer smaller than the body count");
-  int nb = S.nb;
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  std::vector<float> pos(3 * nb), quat(4 * nb), vel(3 * nb), avel(3 * nb), force(3 * nb), torque(3 * nb), iiw(9 * nb),
-      lo(3 * nb), hi(3 * nb);
-  std::vector<int> flags(nb), sleep(nb);
-  std::vector<double> tls(nb);
-  struct F { std::vector<float>* v; float* d; } fs[] = {{&pos, D.pos}, {&quat, D.quat}, {&vel, D.vel}, {&avel, D.avel},
-                                                       {&force, D.force}, {&torque, D.torque}, {&iiw, D.iiw},
-                                                       {&lo, D.aabb_lo}, {&hi, D.aabb_hi}};
-  if (download) {
-    for (auto& f : fs) HIPCHK(ctx, hipMemcpy(f.v->data(), f.d, f.v->size() * 4, hipMemcpyDeviceToHost));
-    HIPCHK(ctx, hipMemcpy(flags.data(), D.flags, nb * 4, hipMemcpyDeviceToHost));
-    HIPCHK(ctx, hipMemcpy(sleep.data(), D.sleep_state, nb * 4, hipMemcpyDeviceToHost));
-    HIPCHK(ctx, hipMemcpy(tls.data(), D.sleep_tls, nb * 8, hipMemcpyDeviceToHost));
+  const int nb = S.nb;
+  bool asleep = false;
+  if (!download)
     for (int i = 0; i < nb; i++) {
-      chp_body_state& s = buf[i];
-      memset(&s, 0, sizeof(s));
-      memcpy(s.position, &pos[3 * i], 12); memcpy(s.quaternion, &quat[4 * i], 16);
-      memcpy(s.velocity, &vel[3 * i], 12); memcpy(s.angular_velocity, &avel[3 * i], 12);
-      memcpy(s.force, &force[3 * i], 12); memcpy(s.torque, &torque[3 * i], 12);
-      memcpy(s.inv_inertia_world, &iiw[9 * i], 36);
-      memcpy(s.aabb_lower, &lo[3 * i], 12); memcpy(s.aabb_upper, &hi[3 * i], 12);
-      s.aabb_needs_update = (flags[i] & BF_AABB_DIRTY) ? 1 : 0;
-      s.sleep_state = sleep[i];
-      s.time_last_sleepy = tls[i];
-    }
-  } else {
-    for (uint32_t i = 0; i < (uint32_t)nb; i++)
       if (buf[i].sleep_state < CHP_SLEEP_AWAKE || buf[i].sleep_state > CHP_SLEEP_SLEEPING)
         return fail(ctx, CHP_E_INVALID, "body " + std::to_string(i) + ": sleep_state is not a CHP_SLEEP_* value");
-    HIPCHK(ctx, hipMemcpy(flags.data(), D.flags, nb * 4, hipMemcpyDeviceToHost));
-    bool asleep = false;
-    for (int i = 0; i < nb; i++) {
-      const chp_body_state& s = buf[i];
-      sleep[i] = s.sleep_state;
-      tls[i] = s.time_last_sleepy;
-      asleep = asleep || s.sleep_state == CHP_SLEEP_SLEEPING;
-      memcpy(&pos[3 * i], s.position, 12); memcpy(&quat[4 * i], s.quaternion, 16);
-      memcpy(&vel[3 * i], s.velocity, 12); memcpy(&avel[3 * i], s.angular_velocity, 12);
-      memcpy(&force[3 * i], s.force, 12); memcpy(&torque[3 * i], s.torque, 12);
-      memcpy(&iiw[9 * i], s.inv_inertia_world, 36);
-      memcpy(&lo[3 * i], s.aabb_lower, 12); memcpy(&hi[3 * i], s.aabb_upper, 12);
-      flags[i] = (flags[i] & ~BF_AABB_DIRTY) | (s.aabb_needs_update ? BF_AABB_DIRTY : 0);
+      asleep = asleep || buf[i].sleep_state == CHP_SLEEP_SLEEPING;
     }
-    for (auto& f : fs) HIPCHK(ctx, hipMemcpy(f.d, f.v->data(), f.v->size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(ctx, hipMemcpy(D.flags, flags.data(), nb * 4, hipMemcpyHostToDevice));
-    HIPCHK(ctx, hipMemcpy(D.sleep_state, sleep.data(), nb * 4, hipMemcpyHostToDevice));
-    HIPCHK(ctx, hipMemcpy(D.sleep_tls, tls.data(), nb * 8, hipMemcpyHostToDevice));
+  int r = ensure_stage(ctx, (size_t)std::min(nb, STATE_CHUNK) * sizeof(chp_body_state));
+  if (r != CHP_OK) return r;
+  StateArrays A{{D.pos, D.quat, D.vel, D.avel, D.force, D.torque, D.iiw, D.aabb_lo, D.aabb_hi},
+                D.flags, D.sleep_state, D.sleep_tls, D.counters + C_STATUS};
+  for (int b0 = 0; b0 == 0 || b0 < nb; b0 += STATE_CHUNK) {
+    const int m = std::min(STATE_CHUNK, nb - b0), blocks = std::max(1, (m + STATE_BODIES - 1) / STATE_BODIES);
+    const size_t bytes = (size_t)m * sizeof(chp_body_state);
+    if (!download) memcpy(ctx->h_stage, buf + b0, bytes);
+    if (download) k_state<true><<<blocks, 256, 0, ctx->stream>>>(A, (uint2*)ctx->h_stage, b0, m);
+    else k_state<false><<<blocks, 256, 0, ctx->stream>>>(A, (uint2*)ctx->h_stage, b0, m);
+    HIPCHK(ctx, hipGetLastError());
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    if (download) memcpy(buf + b0, ctx->h_stage, bytes);
+  }
+  if (!download) {
     const bool may = D.allow_sleep != 0 || asleep;
     if (may != S.may_sleep) {   // the step's wake-up pass is launched per list
       S.may_sleep = may;
       invalidate_lists(ctx);
     }
-    int zero = 0;  // a fresh state clears a quarantine
-    HIPCHK(ctx, hipMemcpy(D.counters + C_STATUS, &zero, 4, hipMemcpyHostToDevice));
   }
   return CHP_OK;
 }
 
-// the sleeping-body count and World.time of a world
 template <typename R> static int sleep_stats_t(chp_ctx* ctx, uint32_t id, chp_step_stats* out) {
   WorldSlot& S = ctx->worlds[id];
   DevWorld<R>& D = dev_of<R>(S);
@@ -1912,8 +1954,7 @@ int chp_ctx_destroy(chp_ctx* ctx) {
   if (ctx->d_worlds) (void)hipFree(ctx->d_worlds);
   if (ctx->d_big) (void)hipFree(ctx->d_big);
   if (ctx->d_list) (void)hipFree(ctx->d_list);
-  if (ctx->d_status) (void)hipFree(ctx->d_status);
-  if (ctx->d_cptrs) (void)hipFree(ctx->d_cptrs);
+  if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
   if (ctx->d_eq) (void)hipFree(ctx->d_eq);
   if (ctx->d_qbuf) (void)hipFree(ctx->d_qbuf);
   if (ctx->d_q) (void)hipFree(ctx->d_q);
