@@ -460,10 +460,10 @@ static int build_slot(chp_ctx* ctx, WorldSlot& S, const HostWorld<R>& H, int pai
   SCR(contacts, ContactRec<R>, contact_cap);
   SCR(rows, RowRec<R>, row_cap);
   SCR(level, int, row_cap); SCR(sched, int, row_cap); SCR(lvl_start, int, row_cap + 2);
-  SCR(row_ab, int, 2 * row_cap); SCR(rpos, int, row_cap + 1); SCR(absdl, R, row_cap + 1); SCR(glam, R, row_cap + 1);
-  fix.emplace_back((void**)(void*)&D.gsr, L.add<R>((size_t)4 * GS_GROUPS * row_cap));
-  SCR(vw, float, 8 * nb);
-  SCR(last_level, int, std::max(nb, row_cap + 1));
+  SCR(row_ab, int, 2 * row_cap); SCR(rpos, int, row_cap + 1); SCR(glam, R, 2 * ((size_t)row_cap + 1));
+  fix.emplace_back((void**)(void*)&D.gsr, L.add<R>((size_t)4 * GS_GROUPS * ((size_t)row_cap + 1)));
+  SCR(vw, float, 8 * ((size_t)nb + 1));
+  SCR(last_level, int, std::max(nb, row_cap + 1) + 16);   // also the GS step table (gs_steps + 1)
   SCR(sort_keys, unsigned long long, np2 + nb);  // the grid-wide SAP sort merges between two halves
   {  // SplitSolver: the persistent ids state (carried over from a previous slab) and the scratch
     const bool split = H.wd.solver == CHP_SOLVER_SPLIT;
@@ -826,9 +826,11 @@ static int upload_list(chp_ctx* ctx, const std::vector<int>& list) {
       while (k < n && (int)ctx->worlds[list[k]].nb > nb_over) k++;
       return (int)k;
     };
-    ctx->gsg.blk = lead(GS_SUB_MAX_NB);
-    ctx->gsg.s32 = lead(128);
-    ctx->gsg.s16 = lead(64);
+    GsSegs& g = ctx->gsg;
+    g.blk = lead(GS_SUB_MAX_NB);
+    g.wave = lead(GS_WAVE_NB);
+    g.nb_sub = g.wave > g.blk ? ctx->worlds[list[g.blk]].nb : 0;
+    g.nb_wave = (int)n > g.wave ? ctx->worlds[list[g.wave]].nb : 0;
   }
   std::vector<int> spans, tiles, bigw;
   int max_tiles = 1;
@@ -940,7 +942,7 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
   const DevWorld<R>* dw = (const DevWorld<R>*)V.worlds;
   const int* d_list = V.list;
   auto groups = [&](int bd) { return nbig + (n - nbig + bd / 64 - 1) / (bd / 64); };
-  const int bcap = big_lds_cap(nbig, max_nb, ctx->max_lds), lcap = levels_lds_cap(nbig, max_nb, ctx->max_lds);
+  const int lcap = levels_lds_cap(nbig, max_nb, ctx->max_lds);
   hipStream_t st = ctx->stream;
   if (ev) HIPCHK(ctx, hipEventRecord(ev[0], st));
   {
@@ -1004,7 +1006,7 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
       k_levels<R><<<groups(b), b, lds_levels(b, lcap), st>>>(dw, d_list, nbig, n, lcap, 0);
       build_rows();   // at the positions this schedule gave (the order inside a level may differ)
       HIPCHK(ctx, hipEventRecord(ctx->tev[3 * c + 1], st));
-      launch_gs<R>(dw, d_list, n, V.gsg, bcap, b, keep, st);
+      launch_gs<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, b, keep, 0, st);
       HIPCHK(ctx, hipEventRecord(ctx->tev[3 * c + 2], st));
     }
     if (ev) {
@@ -1018,7 +1020,7 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
     if (ev) HIPCHK(ctx, hipEventRecord(ev[4], st));
     build_rows();
     if (ev) HIPCHK(ctx, hipEventRecord(ev[5], st));
-    launch_gs<R>(dw, d_list, n, V.gsg, bcap, bg, keep, st);
+    launch_gs<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, bg, keep, 0, st);
     if (ev) HIPCHK(ctx, hipEventRecord(ev[6], st));
   }
   if (V.n_split) k_split_gs<R><<<n, 256, 0, st>>>(dw, d_list, keep);
@@ -1306,8 +1308,9 @@ template <typename R> static int step_noalloc_t(chp_ctx* ctx, uint32_t id, doubl
   V.n_events = S.ev.mask ? 1 : 0;
   V.n_split = S.split ? 1 : 0;
   V.gsg.blk = S.nb > GS_SUB_MAX_NB ? 1 : 0;
-  V.gsg.s32 = S.nb > 128 ? 1 : 0;
-  V.gsg.s16 = S.nb > 64 ? 1 : 0;
+  V.gsg.wave = S.nb > GS_WAVE_NB ? 1 : 0;
+  V.gsg.nb_sub = V.gsg.wave > V.gsg.blk ? S.nb : 0;
+  V.gsg.nb_wave = V.gsg.wave ? 0 : S.nb;
   V.qcls = (int*)(base + o_qcls);
   V.q = (int2*)(base + o_q);
   V.qcap = (size_t)S.pair_cap;
@@ -1703,8 +1706,10 @@ static int solve_t(chp_ctx* ctx, uint32_t id, const chp_equation* eqs, uint32_t 
   if (n > (uint32_t)S.row_cap)
     return fail(ctx, CHP_E_CAPACITY, "more equations than the world's row slab (" + std::to_string(S.row_cap) +
                                          "); raise it with chp_world_set_capacity");
+  int self = 0;   // an equation of one body with itself
   for (uint32_t k = 0; k < n; k++) {
     const chp_equation& e = eqs[k];
+    if (e.body_i == e.body_j) self = 1;
     if (e.body_i < 0 || e.body_j < 0 || e.body_i >= S.nb || e.body_j >= S.nb || e.kind < CHP_ROW_FRICTION ||
         e.kind > CHP_ROW_MOTOR)
       return fail(ctx, CHP_E_INVALID, "equation " + std::to_string(k) + " is malformed");
@@ -1721,9 +1726,9 @@ static int solve_t(chp_ctx* ctx, uint32_t id, const chp_equation* eqs, uint32_t 
   const int bl = ctx->levels_block, bg = ctx->solve_block, nbig = S.nb > SMALL_NB ? 1 : 0;
   hipStream_t st = ctx->stream;
   k_solve_rows<R><<<1, 256, 0, st>>>(dw, (int)id, ctx->d_eq, (int)n, dt);
-  const int bcap = big_lds_cap(nbig, S.nb, ctx->max_lds), lcap = levels_lds_cap(nbig, S.nb, ctx->max_lds);
+  const int lcap = levels_lds_cap(nbig, S.nb, ctx->max_lds);
   k_levels<R><<<1, bl, lds_levels(bl, lcap), st>>>(dw, ctx->d_list, nbig, 1, lcap, 1);
-  launch_gs<R>(dw, ctx->d_list, 1, ctx->gsg, bcap, bg, 1, st);
+  launch_gs<R>(dw, ctx->d_list, 1, ctx->gsg, S.nb, ctx->max_lds, bg, 1, self, st);
   k_solve_finish<R><<<1, 256, 0, st>>>(dw, (int)id);
   HIPCHK(ctx, hipGetLastError());
   HIPCHK(ctx, hipStreamSynchronize(st));

@@ -4,6 +4,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "../../include/cannon_hip.h"
 #include "chp_build.h"
 #include "chp_stages.h"
@@ -273,37 +275,24 @@ __global__ __launch_bounds__(64) void k_joint_rows(const DevWorld<R>* __restrict
     constraint_rows<R, MODE>(W, c, F + C + W.c_row_off[c], (R)dt, keep != 0);
 }
 
-// Levels and GS sweeps run one large world per workgroup (the first nbig entries of the list)
-// and one small world (at most SMALL_NB bodies) per wave, blockDim / 64 of them per workgroup.
+// The level stage runs one large world per workgroup (the first nbig entries of the list) and one
+// small world (at most SMALL_NB bodies) per wave, blockDim / 64 of them per workgroup.
 constexpr int SMALL_NB = 128;        // bodies of a world run by one wave
-constexpr int LS_BIG = 2048, LS_SMALL = 1024;   // level starts kept in LDS
-constexpr int LS_LEVELS = 4096;                  // the level histogram of a large world's level stage
-// bodies of a large world whose GS / level state fits in LDS: at least 512, up to the largest
-// large world of the launch (the launch's dynamic LDS is sized for it), at most what a
-// workgroup's LDS holds beside the level starts and the static arrays (4 KiB kept free)
-constexpr int BIG_NB_LDS_MIN = 512;
-static int big_lds_cap(int nbig, int max_nb, size_t max_lds) {
-  const int most = (int)((max_lds - 4096 - (size_t)LS_BIG * sizeof(int)) / (8 * sizeof(float)));
-  return nbig ? std::max(BIG_NB_LDS_MIN, std::min(max_nb, most)) : BIG_NB_LDS_MIN;
-}
+constexpr int LS_SMALL = 1024;                  // level histogram of a small world in LDS
+constexpr int LS_LEVELS = 4096;                 // of a large world's level stage
 
 // bodies of a large world whose level walk keeps each body's last level in LDS (4 bytes per
 // body): up to the largest large world of the launch, at most what a workgroup's LDS holds beside
 // the level histogram and the static arrays (4 KiB kept free)
+constexpr int BIG_NB_LDS_MIN = 512;
 static int levels_lds_cap(int nbig, int max_nb, size_t max_lds) {
   const int most = (int)((max_lds - 4096 - (size_t)LS_LEVELS * sizeof(int)) / sizeof(int));
   return nbig ? std::max(BIG_NB_LDS_MIN, std::min(max_nb, most)) : BIG_NB_LDS_MIN;
 }
 
-// dynamic LDS of k_levels / k_gs for a workgroup of bd threads (big_cap: as levels_lds_cap /
-// big_lds_cap)
+// dynamic LDS of k_levels for a workgroup of bd threads (big_cap: as levels_lds_cap)
 static size_t lds_levels(int bd, int big_cap) {
   size_t big = (size_t)(big_cap + LS_LEVELS) * sizeof(int), small = (size_t)(SMALL_NB + LS_SMALL) * sizeof(int);
-  return std::max(big, (bd / 64) * small);
-}
-static size_t lds_gs(int bd, int big_cap) {
-  size_t big = (size_t)big_cap * 8 * sizeof(float) + LS_BIG * sizeof(int);
-  size_t small = (size_t)SMALL_NB * 8 * sizeof(float) + LS_SMALL * sizeof(int);
   return std::max(big, (bd / 64) * small);
 }
 
@@ -344,105 +333,94 @@ __global__ __launch_bounds__(256) void k_levels(const DevWorld<R>* __restrict__ 
   }
 }
 
-// GS sweeps of the worlds of at most GS_SUB_MAX_NB bodies run G lanes per world, 64 / G worlds
-// per wave (a level of such a world is rarely wider than a few dozen rows, and the sweep is a
-// chain of dependent steps: packing worlds into a wave divides the instructions issued for the
-// same rows by 64 / G).  Their vlambda / wlambda and level starts live in LDS.
-#ifndef CHP_GS_SUB_MAX_NB
-#define CHP_GS_SUB_MAX_NB 512
+// GS sweeps.  Worlds of at most GS_WAVE_NB bodies run one per wave, four to a workgroup; those of
+// at most GS_SUB_MAX_NB one per workgroup of four waves, all of them in one launch; larger ones
+// one per workgroup of their own launch.  vlambda / wlambda and the step tables live in LDS where
+// they fit.
+constexpr int GS_SUB_MAX_NB = 512, GS_WAVE_NB = 128;
+constexpr int GS_SS_WAVE = 1024, GS_SS_SUB = 2048, GS_SS_BIG = 4096;   // step table entries in LDS
+#ifndef CHP_GS_DEPTH
+#define CHP_GS_DEPTH 4
 #endif
-constexpr int GS_SUB_MAX_NB = CHP_GS_SUB_MAX_NB;
-__host__ __device__ constexpr int gs_group(int nb) { return nb <= 64 ? 16 : nb <= 128 ? 32 : nb <= GS_SUB_MAX_NB ? 64 : 0; }
-__host__ __device__ constexpr int gs_sub_nb(int G) { return G == 16 ? 64 : G == 32 ? 128 : GS_SUB_MAX_NB; }
-__host__ __device__ constexpr int gs_sub_ls(int G) { return G == 16 ? 512 : G == 32 ? 1024 : 2048; }
-constexpr size_t gs_sub_bytes(int G) {
-  return (size_t)(64 / G) * (8 * gs_sub_nb(G) * sizeof(float) + gs_sub_ls(G) * sizeof(int));
-}
-// whether k_gs_sub runs the world (else k_gs does)
-template <typename R> __device__ __forceinline__ bool gs_sub_fits(const DevWorld<R>& W, int L) {
-  const int G = gs_group(W.nb);
-  return G != 0 && L + 1 <= gs_sub_ls(G);
-}
+template <typename R> constexpr int gs_depth() { return sizeof(R) == 4 ? CHP_GS_DEPTH : 2; }
 
 // the list positions of a list sorted by body count (largest first): [0, blk) over
-// GS_SUB_MAX_NB bodies, [blk, s32) G = 64, [s32, s16) G = 32, [s16, n) G = 16
+// GS_SUB_MAX_NB bodies, [blk, wave) a workgroup each, [wave, n) a wave each; and the largest body
+// count of the last two
 struct GsSegs {
-  int blk = 0, s32 = 0, s16 = 0;
+  int blk = 0, wave = 0;
+  int nb_sub = 0, nb_wave = 0;
 };
-
-// the group's world: list position lo + (block b of the segment) * (64 / G) + group
-template <typename R, int G>
-__device__ __forceinline__ void gs_sub_run(const DevWorld<R>* worlds, const int* list, int lo, int hi, int b,
-                                           float* lds, int keep) {
-  const int sub = ((int)threadIdx.x & 63) / G;
-  const int idx = lo + b * (64 / G) + sub;
-  if (idx >= hi) return;
-  const DevWorld<R>& W = worlds[list[idx]];
-  if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;
-  if (gs_group(W.nb) != G || !gs_sub_fits(W, W.counters[C_LEVELS])) return;
-  float* base = lds + sub * (8 * gs_sub_nb(G) + gs_sub_ls(G));
-  st_gs<R, GSub<G>, true>(W, GSub<G>(), nullptr, nullptr, base, (int*)(base + 8 * gs_sub_nb(G)), keep != 0);
+static size_t lds_gs_sub(const GsSegs& g) {
+  const size_t sub = (size_t)(g.nb_sub + 1) * 8 * sizeof(float) + GS_SS_SUB * sizeof(int);
+  const size_t wave = (size_t)(g.nb_wave + 1) * 8 * sizeof(float) + GS_SS_WAVE * sizeof(int);
+  return std::max(g.nb_sub ? sub : 0, g.nb_wave ? 4 * wave : 0);
 }
-// one wave per workgroup; the workgroups are dealt to the three segments (G = 64 first: their
-// worlds have the longest chains), so that all of them run in one launch
+// bodies of a world over GS_SUB_MAX_NB whose velocities fit in LDS beside the step table and the
+// static arrays (4 KiB kept free), up to the launch's largest world
+static int big_lds_cap(int max_nb, size_t max_lds) {
+  const int most = (int)((max_lds - 4096 - GS_SS_BIG * sizeof(int)) / (8 * sizeof(float))) - 1;
+  return std::min(max_nb, most);
+}
+
+template <typename R, int NW>
+__device__ __forceinline__ void gs_sub_run(const DevWorld<R>& W, float* vw, int nb_cap, double* shd, int* sh, int keep, int self) {
+  constexpr int D = gs_depth<R>();
+  if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;   // k_split_gs solves its islands
+  const int steps = gs_steps(W.counters[C_LEVELS], W.counters[C_ROWS], 16 * NW, D);
+  int* ss = (int*)(vw + 8 * (nb_cap + 1));
+  if (steps < (NW == 1 ? GS_SS_WAVE : GS_SS_SUB)) st_gs<R, NW, D, true>(W, vw, ss, shd, sh, keep != 0, self != 0);
+  else st_gs<R, NW, D, true>(W, vw, (int*)W.last_level, shd, sh, keep != 0, self != 0);
+}
 template <typename R>
-__global__ __launch_bounds__(64) void k_gs_sub(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                               GsSegs g, int n, int keep) {
+__global__ __launch_bounds__(256) void k_gs_sub(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                GsSegs g, int n, int keep, int self) {
+  __shared__ int sh[4];
+  __shared__ double shd[4];
   extern __shared__ float4 lds_f4[];
   float* lds = (float*)lds_f4;
-  const int b = (int)blockIdx.x;
-  const int n64 = g.s32 - g.blk, n32 = (g.s16 - g.s32 + 1) / 2;
-  if (b < n64) gs_sub_run<R, 64>(worlds, list, g.blk, g.s32, b, lds, keep);
-  else if (b < n64 + n32) gs_sub_run<R, 32>(worlds, list, g.s32, g.s16, b - n64, lds, keep);
-  else gs_sub_run<R, 16>(worlds, list, g.s16, n, b - n64 - n32, lds, keep);
-}
-
-// GS iterations of the rest.  GLOBAL = false: the worlds over GS_SUB_MAX_NB bodies whose body
-// velocities and level starts fit in LDS, one per workgroup; GLOBAL = true: every world that
-// neither this nor k_gs_sub runs, from global memory (a separate kernel, so that the common LDS
-// form keeps its own, smaller register count)
-template <typename R, bool GLOBAL>
-__global__ __launch_bounds__(256) void k_gs(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                            int nbig, int n, int big_cap, int keep) {
-  __shared__ int sh[256];
-  __shared__ double shd[256];
-  extern __shared__ float4 lds_f4[];
-  int wave;
-  int id = group_world(worlds, list, nbig, n, sh, wave);
-  if (id < 0) return;
-  const DevWorld<R>& W = worlds[id];
-  if (W.solver_kind == CHP_SOLVER_SPLIT) return;   // k_split_gs solves its islands
-  float* lds = (float*)lds_f4;
-  const int L = W.counters[C_LEVELS];
-  if (wave < 0) {
-    const bool fits = W.nb <= big_cap && L + 1 <= LS_BIG;
-    if constexpr (!GLOBAL) {
-      if (fits) st_gs<R, GBlock, true>(W, GBlock(), shd, sh, lds, (int*)(lds + 8 * big_cap), keep != 0);
-    } else {
-      if (!fits) st_gs<R, GBlock, false>(W, GBlock(), shd, sh, W.vw, nullptr, keep != 0);
-    }
+  const int b = (int)blockIdx.x, nsub = g.wave - g.blk;
+  if (b < nsub) {
+    gs_sub_run<R, 4>(worlds[list[g.blk + b]], lds, g.nb_sub, shd, sh, keep, self);
   } else {
-    if constexpr (GLOBAL) {
-      if (!gs_sub_fits(W, L)) st_gs<R, GWave, false>(W, GWave(), shd, sh, W.vw, nullptr, keep != 0);
-    }
+    const int wave = uni((int)(threadIdx.x >> 6)), idx = g.wave + (b - nsub) * 4 + wave;
+    if (idx >= n) return;
+    gs_sub_run<R, 1>(worlds[list[idx]], lds + wave * (8 * (g.nb_wave + 1) + GS_SS_WAVE), g.nb_wave, shd, sh, keep, self);
   }
 }
+// the worlds over GS_SUB_MAX_NB bodies; big_cap: body velocities that fit in the launch's LDS
+template <typename R, int NW>
+__global__ __launch_bounds__(64 * NW) void k_gs(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                int big_cap, int keep, int self) {
+  __shared__ int sh[1];
+  __shared__ double shd[NW];
+  extern __shared__ float4 lds_f4[];
+  constexpr int D = NW == 16 ? 2 : gs_depth<R>();   // 16 waves: at most 128 registers a lane
+  const DevWorld<R>& W = worlds[list[blockIdx.x]];
+  if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;
+  int* ss = (int*)lds_f4;
+  float* vw = (float*)(ss + GS_SS_BIG);
+  const int steps = gs_steps(W.counters[C_LEVELS], W.counters[C_ROWS], 16 * NW, D);
+  if (steps >= GS_SS_BIG) st_gs<R, NW, D, false>(W, W.vw, (int*)W.last_level, shd, sh, keep != 0, self != 0);
+  else if (W.nb <= big_cap) st_gs<R, NW, D, true>(W, vw, ss, shd, sh, keep != 0, self != 0);
+  else st_gs<R, NW, D, false>(W, W.vw, ss, shd, sh, keep != 0, self != 0);
+}
 
-// the GS stage of a list (the level schedule and the GS records are in place)
+// the GS stage of a list (the level schedule and the GS records are in place).  rows: rows a
+// large world runs at a time (64, 128 or 256: four lanes each).  self: the rows may hold one whose
+// two bodies are one (the Solver slot)
 template <typename R>
-static void launch_gs(const DevWorld<R>* dw, const int* d_list, int n, const GsSegs& g, int bcap, int bd, int keep,
-                      hipStream_t st) {
-  if (g.blk) k_gs<R, false><<<g.blk, bd, lds_gs(bd, bcap), st>>>(dw, d_list, g.blk, g.blk, bcap, keep);
-  const int nsub = (g.s32 - g.blk) + (g.s16 - g.s32 + 1) / 2 + (n - g.s16 + 3) / 4;
-  if (nsub) {
-    size_t bytes = 0;
-    if (g.s32 > g.blk) bytes = std::max(bytes, gs_sub_bytes(64));
-    if (g.s16 > g.s32) bytes = std::max(bytes, gs_sub_bytes(32));
-    if (n > g.s16) bytes = std::max(bytes, gs_sub_bytes(16));
-    k_gs_sub<R><<<nsub, 64, bytes, st>>>(dw, d_list, g, n, keep);
+static void launch_gs(const DevWorld<R>* dw, const int* d_list, int n, const GsSegs& g, int max_nb, size_t max_lds, int rows,
+                      int keep, int self, hipStream_t st) {
+  if (g.blk) {
+    const int cap = big_lds_cap(max_nb, max_lds);
+    const size_t lds = GS_SS_BIG * sizeof(int) + (size_t)(cap + 1) * 8 * sizeof(float);
+    if (rows == 64) k_gs<R, 4><<<g.blk, 256, lds, st>>>(dw, d_list, cap, keep, self);
+    else if (rows == 128) k_gs<R, 8><<<g.blk, 512, lds, st>>>(dw, d_list, cap, keep, self);
+    else k_gs<R, 16><<<g.blk, 1024, lds, st>>>(dw, d_list, cap, keep, self);
   }
-  const int per = bd / 64;
-  k_gs<R, true><<<g.blk + (n - g.blk + per - 1) / per, bd, 0, st>>>(dw, d_list, g.blk, n, bcap, keep);
+  const int nsub = (g.wave - g.blk) + (n - g.wave + 3) / 4;
+  if (nsub) k_gs_sub<R><<<nsub, 256, lds_gs_sub(g), st>>>(dw, d_list, g, n, keep, self);
 }
 
 // World.step(dt, timeSinceLastCalled): the interpolated poses and World.time += the elapsed time

@@ -171,7 +171,6 @@ template <typename R> __device__ void st_split_gs(const DevWorld<R>& W, bool kee
   const int NI = W.counters[C_LEVELS], iters = W.iterations;
   const R tol2 = W.tol2;
   R* lam = W.glam;
-  R* adl = W.absdl;
   for (int i = (int)threadIdx.x; i < NI; i += (int)blockDim.x) {
     const int s0 = W.lvl_start[i], s1 = W.lvl_start[i + 1];
     for (int it = 0; it < iters; it++) {
@@ -179,9 +178,7 @@ template <typename R> __device__ void st_split_gs(const DevWorld<R>& W, bool kee
       for (int k = s0; k < s1; k++) {
         GsRow<R> cr;
         gs_load<R>(gsr, k, cr);
-        double part = 0.0;
-        gs_row<R>(cr, lam[k], true, k, W.vw, lam, adl, part);
-        tot += adl[k];
+        tot += gs_row<R>(cr, W.vw, lam + 2 * (size_t)k);
       }
       if (tot * tot < tol2) break;
     }
@@ -189,7 +186,7 @@ template <typename R> __device__ void st_split_gs(const DevWorld<R>& W, bool kee
   __syncthreads();
   const int E = W.counters[C_ROWS];
   if (keep)
-    for (int k = (int)threadIdx.x; k < E; k += (int)blockDim.x) W.rows[W.sched[k]].lambda = lam[k];
+    for (int k = (int)threadIdx.x; k < E; k += (int)blockDim.x) W.rows[W.sched[k]].lambda = lam[2 * (size_t)k];
   for (int b = (int)threadIdx.x; b < W.nb; b += (int)blockDim.x) {   // vlambda / wlambda to st_post
     const float4 v = ((const float4*)W.vw)[2 * b], w = ((const float4*)W.vw)[2 * b + 1];
     S3<R>(W.vl, b, mk3(v.x, v.y, v.z));

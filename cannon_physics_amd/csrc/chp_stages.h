@@ -950,7 +950,7 @@ __device__ void put_row(const DevWorld<R>& W, int r, int kind, const RowBody<R>&
   if constexpr (MODE == ROWS_GS) {
     const int k = W.rpos[r];
     gs_store<R>((typename GsWord<R>::T*)W.gsr, k, o, (unsigned)fa, (unsigned)fb);
-    W.glam[k] = (R)0;
+    W.glam[2 * k] = (R)0;
     if (keep) W.rows[r] = o;
   } else {
     W.rows[r] = o;
@@ -1296,33 +1296,13 @@ struct GWave {
   }
   __device__ int uni(int v) const { return __builtin_amdgcn_readfirstlane(v); }
 };
-// G lanes of one wave on one world (G = 16, 32 or 64), 64 / G worlds per wave.  A group's lanes
-// always take the same path (every branch of the GS sweep depends on the world only), so the
-// wave's program order orders the group's memory accesses as it does a whole wave's; values
-// uniform over the group are not uniform over the wave unless G = 64.
-template <int G> struct GSub {
-  int tid, n;
-  __device__ GSub() : tid((int)threadIdx.x & (G - 1)), n(G) {}
-  __device__ void sync() const { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup"); }
-  __device__ void lds_sync() const { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local"); }
-  __device__ double sum(double v, double*) const {
-    // fixed butterfly inside the group: every lane of it ends with the same value
-    for (int off = G >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-  }
-  __device__ int bcast0(int v, int*) const { return __shfl(v, ((int)threadIdx.x & 63) & ~(G - 1), 64); }
-  __device__ int uni(int v) const {
-    if constexpr (G == 64) return __builtin_amdgcn_readfirstlane(v);
-    else return v;
-  }
-};
-
-// GS record: 6 groups of 4 words, row position k at words [k * 24, k * 24 + 24) -- a wave reads
-// 64 consecutive records
-//   g0 sa.x sa.y sa.z ra.x | g1 ra.y ra.z rb.x rb.y | g2 rb.z ia.x ia.y ia.z
-//   g3 ib.x ib.y ib.z ima  | g4 imb B invC eps      | g5 minF maxF a' b'
+// GS record: 6 groups of 4 words, row position k at words [k * 24, k * 24 + 24)
+//   g0 sa.x sa.y sa.z ima  | g1 ra.x ra.y ra.z B    | g2 rb.x rb.y rb.z invC
+//   g3 ia.x ia.y ia.z eps  | g4 ib.x ib.y ib.z minF | g5 imb maxF a' b'
 // a' = a | (a dynamic) << 31 | (sb == -sa, else both spatial parts are +0) << 30,
-// b' = b | (b dynamic) << 31.  row_ab holds a and b with the same dynamic bits.
+// b' = b | (b dynamic) << 31.  row_ab holds a and b with the same dynamic bits.  The groups are
+// what the four lanes of a row load (st_gs): each a Jacobian part and the part its impulse moves
+// the velocity along, with one of the row's scalars in the fourth word.
 template <typename R> struct GsWord;
 template <> struct GsWord<float> {
   typedef unsigned int T;
@@ -1358,9 +1338,9 @@ template <typename R> __device__ __forceinline__ void gs_load(const typename GsW
   }
   auto F = [&](int i) { return (float)GsWord<R>::get(w[i]); };
   auto S = [&](int i) { return GsWord<R>::get(w[i]); };
-  o.sa = mk3(F(0), F(1), F(2)); o.ra = mk3(F(3), F(4), F(5)); o.rb = mk3(F(6), F(7), F(8));
-  o.ia = mk3(F(9), F(10), F(11)); o.ib = mk3(F(12), F(13), F(14));
-  o.ima = S(15); o.imb = S(16); o.B = S(17); o.invC = S(18); o.eps = S(19); o.minF = S(20); o.maxF = S(21);
+  o.sa = mk3(F(0), F(1), F(2)); o.ra = mk3(F(4), F(5), F(6)); o.rb = mk3(F(8), F(9), F(10));
+  o.ia = mk3(F(12), F(13), F(14)); o.ib = mk3(F(16), F(17), F(18));
+  o.ima = S(3); o.imb = S(20); o.B = S(7); o.invC = S(11); o.eps = S(15); o.minF = S(19); o.maxF = S(21);
   o.a = (unsigned)w[22]; o.b = (unsigned)w[23];
 }
 
@@ -1369,10 +1349,12 @@ template <typename R> __device__ __forceinline__ void gs_store(typename GsWord<R
   typedef typename GsWord<R>::T T;
   T w[4 * GS_GROUPS];
   auto P = [&](int i, R v) { w[i] = GsWord<R>::put(v); };
-  P(0, r.sa.x); P(1, r.sa.y); P(2, r.sa.z); P(3, r.ra.x); P(4, r.ra.y); P(5, r.ra.z);
-  P(6, r.rb.x); P(7, r.rb.y); P(8, r.rb.z); P(9, r.ia.x); P(10, r.ia.y); P(11, r.ia.z);
-  P(12, r.ib.x); P(13, r.ib.y); P(14, r.ib.z); P(15, r.ima); P(16, r.imb); P(17, r.B);
-  P(18, r.invC); P(19, r.eps); P(20, r.minF); P(21, r.maxF);
+  P(0, r.sa.x); P(1, r.sa.y); P(2, r.sa.z); P(3, r.ima);
+  P(4, r.ra.x); P(5, r.ra.y); P(6, r.ra.z); P(7, r.B);
+  P(8, r.rb.x); P(9, r.rb.y); P(10, r.rb.z); P(11, r.invC);
+  P(12, r.ia.x); P(13, r.ia.y); P(14, r.ia.z); P(15, r.eps);
+  P(16, r.ib.x); P(17, r.ib.y); P(18, r.ib.z); P(19, r.minF);
+  P(20, r.imb); P(21, r.maxF);
   bool neg = !(r.kind == CHP_ROW_ROTATIONAL || r.kind == CHP_ROW_CONE || r.kind == CHP_ROW_MOTOR);
   w[22] = (T)(fa | (neg ? GS_NEG : 0u));
   w[23] = (T)fb;
@@ -1572,7 +1554,7 @@ __device__ __forceinline__ void st_levels(const DevWorld<R>& W, const G& g, int*
       RowRec<R> o = W.rows[r];
       int2 x = ab[r];
       gs_store<R>(gsr, k, o, (unsigned)x.x, (unsigned)x.y);
-      W.glam[k] = (R)0;
+      W.glam[2 * k] = (R)0;
     }
   }
   if (tid == 0) W.counters[C_LEVELS] = L;
@@ -1601,31 +1583,24 @@ template <typename R> __device__ __forceinline__ int gs_decide(double D, int n, 
   return -1;                         // undecided, or NaN: the sequential sum decides
 }
 
-// One row of the sweep: computeGWlambda, the clamped dlambda, addToWlambda.  Returns the new
-// lambda and adds |dlambda| to part.  An idle lane (v false) computes on a valid row but writes
-// no body, stores to the slot ks (a dummy slot) and adds nothing: the memory operations of the
-// step are the same on every lane, which keeps the prefetch counts exact.
-template <typename R>
-__device__ __forceinline__ R gs_row(const GsRow<R>& cr, R clam, bool v, int ks, float* vw, R* lam, R* adl, double& part) {
+// One row of a sweep by one thread (SplitSolver's islands): computeGWlambda, the clamped
+// dlambda, addToWlambda.  lam: the row's lambda and |dlambda|.  Returns |dlambda|.
+template <typename R> __device__ __forceinline__ R gs_row(const GsRow<R>& cr, float* vw, R* lam) {
   const int a = cr.a & GS_IDX, b = cr.b & GS_IDX;
-  const bool da = v && (cr.a & GS_DYN), db = v && (cr.b & GS_DYN);
+  const bool da = cr.a & GS_DYN, db = cr.b & GS_DYN;
   const f3 z = mk3(0.f, 0.f, 0.f);
   const f3 sb = (cr.a & GS_NEG) ? neg3(cr.sa) : z;
+  const R clam = lam[0];
   float4 va4 = ((const float4*)vw)[2 * a], wa4 = ((const float4*)vw)[2 * a + 1];
   float4 vb4 = ((const float4*)vw)[2 * b], wb4 = ((const float4*)vw)[2 * b + 1];
   f3 va = mk3(va4.x, va4.y, va4.z), wa = mk3(wa4.x, wa4.y, wa4.z);
   f3 vb = mk3(vb4.x, vb4.y, vb4.z), wb = mk3(wb4.x, wb4.y, wb4.z);
   R gwl = mulvec<R>(va, wa, cr.sa, cr.ra) + mulvec<R>(vb, wb, sb, cr.rb);
   R dl = cr.invC * (cr.B - gwl - cr.eps * clam);
-  // the clamp of gs_solver.dart:91-96 as selects (a branch per lane costs exec-mask switches on
-  // the sweep's dependent chain); NaN compares false, as in the branches
-  const R t = clam + dl;
+  const R t = clam + dl;   // the clamp of gs_solver.dart:91-96
   dl = t < cr.minF ? cr.minF - clam : (t > cr.maxF ? cr.maxF - clam : dl);
-  R lnew = clam + dl;
   R adlv = dl > (R)0 ? dl : -dl;
-  lam[ks] = lnew;
-  adl[ks] = adlv;
-  part += v ? (double)adlv : 0.0;
+  lam[0] = clam + dl;
   if (da) {
     va = axpy3<R>(va, cr.ima * dl, cr.sa);
     wa = axpy3<R>(wa, dl, cr.ia);
@@ -1639,110 +1614,138 @@ __device__ __forceinline__ R gs_row(const GsRow<R>& cr, R clam, bool v, int ks, 
     ((float4*)vw)[2 * b] = make_float4(vb.x, vb.y, vb.z, 0.f);
     ((float4*)vw)[2 * b + 1] = make_float4(wb.x, wb.y, wb.z, 0.f);
   }
-  return lnew;
+  return adlv;
 }
 
-// vw: 8 floats per body (vlambda xyz, pad, wlambda xyz, pad).  LDS: vw and ls_lds (L + 1 ints)
-// are LDS arrays; else vw is the world's global scratch and the level starts are read from
-// global memory.  The two forms are separate instantiations so that LDS accesses compile to LDS
-// instructions.
-//
-// The sweep is a sequence of steps, one level of one iteration each.  A thread's first row of
-// each level (position ls[l] + tid) is loaded D steps ahead into a ring of registers, so the
-// row stream's memory latency overlaps D levels; further rows of a level wider than the group
-// are loaded when they are reached.  A sweep is padded to a whole number of ring turns, so a row
-// recurs exactly one padded sweep later, in the same slot: when the sweep is a single turn the
-// slot's next row is the row itself, and its new lambda is forwarded in registers.
-// lam / adl have one dummy slot at row_cap for idle lanes.
-#ifndef CHP_GS_DEPTH_F32
-#define CHP_GS_DEPTH_F32 2   // ring depth D of the FP32 sweep (2 measured a few per cent faster than 4)
-#endif
-template <typename R, typename G, bool LDS>
-__device__ __forceinline__ void st_gs(const DevWorld<R>& W, const G& g, double* shd, int* sh, float* vw, int* ls_lds,
-                                      bool keep) {
-  constexpr int D = sizeof(R) == 4 ? CHP_GS_DEPTH_F32 : 2;
-  const int E = g.uni(W.counters[C_ROWS]), L = g.uni(W.counters[C_LEVELS]), iters = g.uni(W.iterations);
-  const int nb = W.nb, tid = g.tid, bd = g.n, dummy = W.row_cap;
-  const R tol2 = W.tol2;
-  const int* ls = W.lvl_start;
-  if constexpr (LDS) {
-    for (int l = tid; l <= L; l += bd) ls_lds[l] = W.lvl_start[l];
-    ls = ls_lds;
-  }
-  for (int i = tid; i < 8 * nb; i += bd) vw[i] = 0.f;
-  g.sync();
-  int it = 0;
-  typedef typename GsWord<R>::T T;
-  const T* gsr = (const T*)W.gsr;
-  R* lam = W.glam;
-  R* adl = W.absdl;
-  if (E != 0 && iters > 0) {
-    GsRow<R> q[D];
-    R ql[D];      // lambda as loaded with the slot's row
-    R qf[D];      // lambda forwarded to the slot (its row ran again after the load)
-    bool qo[D];   // qf, not ql, holds the slot's lambda
-    int qk[D];
-    bool qv[D];
-    // a step is one group-wide slice of a level: a level of c rows takes ceil(c / bd) steps
-    // (its rows are independent, so slicing it keeps the sequential sweep's values)
-    int pl = 0, pj = 0;   // level and slice of the next step to load
-    int ps = 0;           // its step within the sweep
-    // steps per sweep
-    int lp = 0;
-    for (int l = tid; l < L; l += bd) {
-      const int c = ls[l + 1] - ls[l];
-      lp += c > bd ? (c + bd - 1) / bd : 1;
+// values of the other lanes of a row's four (CTRL: a DPP quad permutation)
+template <int CTRL> __device__ __forceinline__ float quad(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ double quad(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+constexpr int QP_SWAP1 = 0xB1, QP_SWAP2 = 0x4E, QP_LANE1 = 0x55, QP_LANE3 = 0xFF;   // [1,0,3,2] [2,3,0,1] [1,..] [3,..]
+// v with its sign flipped where the top bit of m is set
+__device__ __forceinline__ float flip_sign(float v, unsigned m) { return __uint_as_float(__float_as_uint(v) ^ m); }
+__device__ __forceinline__ double flip_sign(double v, unsigned m) {
+  return __longlong_as_double(__double_as_longlong(v) ^ ((long long)m << 32));
+}
+// one group of four words of a GS record
+template <typename R> struct GsQuad {
+  typename GsWord<R>::T w[4];
+  __device__ __forceinline__ void load(const typename GsWord<R>::T* p) {
+    if constexpr (sizeof(R) == 4) {
+      const uint4 v = *(const uint4*)p;
+      w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+    } else {
+      const ulonglong2 v0 = ((const ulonglong2*)p)[0], v1 = ((const ulonglong2*)p)[1];
+      w[0] = v0.x; w[1] = v0.y; w[2] = v1.x; w[3] = v1.y;
     }
-    const int Lp = g.uni((int)g.sum((double)lp, shd));
-    // A sweep is padded with idle steps (no row on any thread) to a multiple of the ring depth,
-    // so that a sweep always ends after the ring's last slot: the loop then has one exit test
-    // per turn, and a loop with one exit keeps the wait counts exact (exits after each slot make
-    // the compiler merge the paths and drain every prefetch at the loop head).
-    const int Lpad = (Lp + D - 1) / D * D;
-    // the step's row of this thread (k, valid), then the cursor moves to the next step
-    auto next = [&](int& k, bool& valid) {
-      if (ps >= Lp) {
-        k = 0;
-        valid = false;
-      } else {
-        const int a0 = ls[pl], a1 = ls[pl + 1];
-        k = a0 + pj * bd + tid;
-        valid = k < a1;
-        if (a0 + (pj + 1) * bd < a1) {
-          pj++;
-        } else {
-          pj = 0;
-          pl++;
-        }
+  }
+  __device__ __forceinline__ R get(int i) const { return GsWord<R>::get(w[i]); }
+};
+
+// GSSolver's sweeps over the level schedule by NW waves on one world (NW = 1: one wave, no
+// barrier).
+//
+// Four lanes run a row: lane p of the four holds one of va, wa, vb, wb, does that part's dot
+// product and impulse, and the four partial products meet in two DPP additions, in the
+// reference's order ((va.sa + wa.ra) + (vb.sb + wb.rb)).  The sweep is a chain of dependent steps
+// whose cost is the instructions one wave issues per step; with a lane doing a whole row a step
+// was about 160 of them (four body loads and stores, 24 record words), with four it is about
+// half that.
+//
+// A step is at most 16 * NW rows of one level.  ss[t] is the first row position of step t (ss[Lp]
+// = E), the sweep is padded to a multiple of the ring depth D with empty steps, and each thread's
+// record and lambda are loaded D steps ahead into a ring of registers.  A sweep is at least D
+// steps, so a row's lambda is stored before it is loaded again, by the same threads.  A thread
+// without a row runs the record at row_cap, all zeros, whose impulse is zero; its writes, and those
+// of bodies that are not dynamic, go to a spare body slot at nb.
+//   vw: 8 floats per body slot (vlambda xyz, pad, wlambda xyz, pad), nb + 1 slots, in LDS when LDS
+//   ss: gs_steps + 1 ints (in LDS or global memory)
+//   self: rows whose two bodies are one are present (the Solver slot may be given them)
+// an upper bound of the entries a sweep's step table takes (see st_gs)
+__host__ __device__ constexpr int gs_steps(int L, int E, int rows_per_step, int D) { return L + E / rows_per_step + D; }
+template <typename R, int NW, int D, bool LDS>
+__device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, double* shd, int* sh, bool keep,
+                                      bool self) {
+  constexpr int T = 64 * NW, RP = 16 * NW;
+  const int tid = NW == 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x, p = tid & 3, row = tid >> 2;
+  const int E = uni(W.counters[C_ROWS]), L = uni(W.counters[C_LEVELS]), iters = uni(W.iterations);
+  const int nb = uni(W.nb), dummy = uni(W.row_cap);
+  const R tol2 = W.tol2;
+  auto sync = [&]() {
+    if constexpr (NW == 1) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    else __syncthreads();
+  };
+  auto step_sync = [&]() {   // the next step reads what this one wrote
+    if constexpr (NW == 1) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local");
+    else if constexpr (LDS) lds_barrier();
+    else __syncthreads();
+  };
+  for (int i = tid; i < 8 * (nb + 1); i += T) vw[i] = 0.f;
+  int Lp = 0;
+  if (E != 0 && iters > 0) {
+    if (tid < 64) {   // the step table: level l is cut into steps of RP rows
+      for (int l0 = 0; l0 < L; l0 += 64) {
+        const int l = l0 + tid;
+        const int a0 = l < L ? W.lvl_start[l] : 0, a1 = l < L ? W.lvl_start[l + 1] : 0;
+        const int n = (a1 - a0 + RP - 1) / RP, inc = wave_incl_scan(n);
+        for (int j = 0; j < n; j++) ss[Lp + inc - n + j] = a0 + j * RP;
+        Lp += __shfl(inc, 63, 64);
       }
-      if (++ps == Lpad) ps = pl = pj = 0;
+      if (NW > 1 && tid == 0) sh[0] = Lp;
+    }
+    if constexpr (NW > 1) {
+      __syncthreads();
+      Lp = sh[0];
+    }
+    Lp = uni(Lp);
+  }
+  const int Lpad = max(1, (Lp + D - 1) / D) * D;
+  for (int t = Lp + tid; t <= Lpad; t += T) ss[t] = E;
+  typedef typename GsWord<R>::T WT;
+  const WT* gsr = (const WT*)W.gsr;
+  R* lam = W.glam;
+  if (tid == 0) {
+    lam[2 * (size_t)dummy] = (R)0;
+    lam[2 * (size_t)dummy + 1] = (R)0;
+  }
+  sync();
+  int it = 0;
+  if (E != 0 && iters > 0) {
+    const unsigned oa = p == 1 ? 4u : p == 3 ? 8u : 0u, ok = p == 1 ? 12u : p == 3 ? 16u : 0u;   // words
+    const unsigned negm = p == 2 ? GS_NEG : 0u;
+    const bool first = p < 2;
+    const int half = p & 1;
+    GsQuad<R> qa[D], qk[D], qc[D];
+    R ql[D];
+    int qr[D];
+    int pt = 0;   // the next step to load
+    auto load = [&](int s, int s0, int s1) {
+      const int k = s0 + row < s1 ? s0 + row : dummy;
+      const unsigned w = (unsigned)k * (4u * GS_GROUPS);
+      qa[s].load(gsr + (size_t)(w + oa));
+      qk[s].load(gsr + (size_t)(w + ok));
+      qc[s].load(gsr + (size_t)(w + 20u));
+      ql[s] = lam[2 * (size_t)(unsigned)k];
+      qr[s] = k;
+      if (++pt == Lpad) pt = 0;
     };
-    const int* rpos = W.rpos;
     // The sweeps run in an inner loop whose only memory traffic is the ring's loads and the
     // lambda stores.  The rare undecided early-exit test reads the stored |dlambda| outside
     // it, and the ring then starts again at the first step of the next sweep.
     for (;;) {
-      ps = pl = pj = 0;
+      pt = 0;
 #pragma unroll
       for (int s = 0; s < D; s++) {
-        int k;
-        next(k, qv[s]);
-        qk[s] = qv[s] ? k : 0;
-        // the two stores a step issues before its slot's loads (to the dummy slot here), so that
-        // the loop entered from here holds the memory operations in flight that it holds after
-        // a turn: the waits at its head then cover only the slot the step uses
-        lam[dummy] = (R)0;
-        adl[dummy] = (R)0;
-        gs_load<R>(gsr, qk[s], q[s]);
-        ql[s] = lam[qk[s]];
-        qf[s] = (R)0;
-        qo[s] = false;
-        // keep the slots' loads in slot order, as the steady state issues them: the wait before
-        // the first step of the loop then allows the later slots to stay in flight
-        __builtin_amdgcn_sched_barrier(0);
+        load(s, ss[pt], ss[pt + 1]);
+        __builtin_amdgcn_sched_barrier(0);   // the slots' loads stay in slot order
       }
-      int step = 0;   // of the sweep
-      int dec = 0;    // the sweep-end decision: 1 stop, -1 undecided
+      int step = 0, dec = 0;   // dec, the sweep-end decision: 1 stop, -1 undecided
       double part = 0.0;
       for (;;) {
 #pragma unroll
@@ -1751,30 +1754,62 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, const G& g, double* 
           // slot's row before its own step makes the wave wait for that row's loads, and the
           // ring then hides no latency
           __builtin_amdgcn_sched_barrier(0);
-          const int k = qk[s];
-          const bool v = qv[s];
-          const R lnew = gs_row<R>(q[s], qo[s] ? qf[s] : ql[s], v, v ? k : dummy, vw, lam, adl, part);
-          {  // the slot's next row (D steps on)
-            int kn;
-            bool vn;
-            next(kn, vn);
-            int kc = vn ? kn : 0;
-            gs_load<R>(gsr, kc, q[s]);
-            ql[s] = lam[kc];
-            qf[s] = lnew;
-            qo[s] = v && vn && kc == k;
-            qk[s] = kc;
-            qv[s] = vn;
+          const unsigned wa = (unsigned)qc[s].w[2], wb = (unsigned)qc[s].w[3];
+          const unsigned w = first ? wa : wb;
+          const int slot = 2 * (int)(w & GS_IDX) + half;
+          const float4 v4 = ((const float4*)vw)[slot];
+          const int s0 = ss[pt], s1 = ss[pt + 1];
+          const unsigned neg = (wa & negm) << 1;
+          const R jx = flip_sign(qa[s].get(0), neg), jy = flip_sign(qa[s].get(1), neg), jz = flip_sign(qa[s].get(2), neg);
+          R d = (R)v4.x * jx;
+          d += (R)v4.y * jy;
+          d += (R)v4.z * jz;
+          d += quad<QP_SWAP1>(d);
+          const R gwl = d + quad<QP_SWAP2>(d);
+          const R own = qa[s].get(3);
+          const R B = quad<QP_LANE1>(own), invC = quad<QP_LANE3>(own);
+          const R eps = quad<QP_LANE1>(qk[s].get(3)), minF = quad<QP_LANE3>(qk[s].get(3)), maxF = qc[s].get(1);
+          const R clam = ql[s];
+          R dl = invC * (B - gwl - eps * clam);
+          // the clamp of gs_solver.dart:91-96 as selects; NaN compares false, as in the branches
+          const R t = clam + dl;
+          dl = t < minF ? minF - clam : (t > maxF ? maxF - clam : dl);
+          const R adlv = dl > (R)0 ? dl : -dl;
+          part += (double)adlv;
+          R* lp = lam + 2 * (size_t)(unsigned)qr[s];
+          if constexpr (sizeof(R) == 4) *(float2*)lp = make_float2((float)(clam + dl), (float)adlv);
+          else *(double2*)lp = make_double2((double)(clam + dl), (double)adlv);
+          // va += (ima dl) sa, wa += dl ia, vb += (imb dl) sb, wb += dl ib
+          const R c = half ? (R)1 : (first ? own : qc[s].get(0));
+          const R sc = flip_sign(c * dl, neg);
+          const R kx = qk[s].get(0), ky = qk[s].get(1), kz = qk[s].get(2);
+          float4 o = make_float4((float)((R)v4.x + sc * kx), (float)((R)v4.y + sc * ky), (float)((R)v4.z + sc * kz), 0.f);
+          int wslot = (w & GS_DYN) ? slot : 2 * nb + half;
+          if (self) {   // one body on both sides: its second impulse follows the first
+            const bool same = ((wa ^ wb) & GS_IDX) == 0;
+            const float ax = quad<0x44>(o.x), ay = quad<0x44>(o.y), az = quad<0x44>(o.z);   // lanes 0, 1, 0, 1
+            if (same && !first && (wa & GS_DYN))
+              o = make_float4((float)((R)ax + sc * kx), (float)((R)ay + sc * ky), (float)((R)az + sc * kz), 0.f);
+            if (same && first) wslot = 2 * nb + half;
           }
-          if constexpr (LDS) g.lds_sync();   // the next step reads what this one wrote
-          else g.sync();
+          ((float4*)vw)[wslot] = o;
+          load(s, s0, s1);   // the slot's next row (D steps on)
+          step_sync();
         }
         step += D;
         if (step == Lpad) {   // end of a sweep: GSSolver's early-exit test
           step = 0;
-          const double Dsum = g.sum(part, shd);
+          double S = part;
+          for (int off = 32; off > 0; off >>= 1) S += __shfl_xor(S, off, 64);
+          if constexpr (NW > 1) {
+            if ((tid & 63) == 0) shd[tid >> 6] = S;
+            lds_barrier();
+            S = 0.0;
+            for (int u = 0; u < NW; u++) S += shd[u];
+            lds_barrier();
+          }
           part = 0.0;
-          dec = g.uni(gs_decide<R>(Dsum, E, tol2));
+          dec = uni(gs_decide<R>(0.25 * S, E, tol2));   // the four lanes of a row add the same |dlambda|
           if (dec != 0) break;
           if (++it == iters) {
             dec = 1;
@@ -1785,30 +1820,37 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, const G& g, double* 
       if (dec > 0) break;
       // undecided: the sequential sum in solver order decides (every |dlambda| of the sweep is
       // stored)
-      g.sync();
+      sync();
       int vv = 0;
       if (tid == 0) {
+        const int* rpos = W.rpos;
         R tot = 0;
-        for (int r = 0; r < E; r++) tot += adl[rpos[r]];
+        for (int r = 0; r < E; r++) tot += lam[2 * (size_t)(unsigned)rpos[r] + 1];
         vv = tot * tot < tol2 ? 1 : 0;
+        if (NW > 1) sh[0] = vv;
       }
-      if (g.uni(g.bcast0(vv, sh)) || ++it == iters) break;
+      if constexpr (NW > 1) {
+        __syncthreads();
+        vv = sh[0];
+        __syncthreads();
+      } else {
+        vv = __shfl(vv, 0, 64);
+      }
+      if (uni(vv) || ++it == iters) break;
       // next sweep: the ring starts again at its first step
     }
-    g.sync();
+    sync();
     // Equation.multiplier and the capture read lambda from the row records (keep)
     if (keep)
-      for (int k = tid; k < E; k += bd) W.rows[W.sched[k]].lambda = lam[k];
+      for (int k = tid; k < E; k += T) W.rows[W.sched[k]].lambda = lam[2 * (size_t)k];
   }
-  g.sync();
   // hand the lambda velocities to st_post
-  for (int i = tid; i < nb; i += bd) {
-    float4 v = ((const float4*)vw)[2 * i], w = ((const float4*)vw)[2 * i + 1];
+  for (int i = tid; i < nb; i += T) {
+    const float4 v = ((const float4*)vw)[2 * i], w = ((const float4*)vw)[2 * i + 1];
     S3<R>(W.vl, i, mk3(v.x, v.y, v.z));
     S3<R>(W.wl, i, mk3(w.x, w.y, w.z));
   }
   if (tid == 0) W.counters[C_ITERS] = it;
-  g.sync();
 }
 
 // ---- interpolation (World.step with timeSinceLastCalled, world_class.dart:421-428) ----------------
