@@ -1006,7 +1006,7 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
       k_levels<R><<<groups(b), b, lds_levels(b, lcap), st>>>(dw, d_list, nbig, n, lcap, 0);
       build_rows();   // at the positions this schedule gave (the order inside a level may differ)
       HIPCHK(ctx, hipEventRecord(ctx->tev[3 * c + 1], st));
-      launch_gs<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, b, keep, 0, st);
+      launch_gs<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, b, keep, st);
       HIPCHK(ctx, hipEventRecord(ctx->tev[3 * c + 2], st));
     }
     if (ev) {
@@ -1020,7 +1020,7 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
     if (ev) HIPCHK(ctx, hipEventRecord(ev[4], st));
     build_rows();
     if (ev) HIPCHK(ctx, hipEventRecord(ev[5], st));
-    launch_gs<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, bg, keep, 0, st);
+    launch_gs<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, bg, keep, st);
     if (ev) HIPCHK(ctx, hipEventRecord(ev[6], st));
   }
   if (V.n_split) k_split_gs<R><<<n, 256, 0, st>>>(dw, d_list, keep);
@@ -1706,10 +1706,10 @@ static int solve_t(chp_ctx* ctx, uint32_t id, const chp_equation* eqs, uint32_t 
   if (n > (uint32_t)S.row_cap)
     return fail(ctx, CHP_E_CAPACITY, "more equations than the world's row slab (" + std::to_string(S.row_cap) +
                                          "); raise it with chp_world_set_capacity");
-  int self = 0;   // an equation of one body with itself
+  bool self = false;   // an equation of one body with itself
   for (uint32_t k = 0; k < n; k++) {
     const chp_equation& e = eqs[k];
-    if (e.body_i == e.body_j) self = 1;
+    if (e.body_i == e.body_j) self = true;
     if (e.body_i < 0 || e.body_j < 0 || e.body_i >= S.nb || e.body_j >= S.nb || e.kind < CHP_ROW_FRICTION ||
         e.kind > CHP_ROW_MOTOR)
       return fail(ctx, CHP_E_INVALID, "equation " + std::to_string(k) + " is malformed");
@@ -1728,7 +1728,8 @@ static int solve_t(chp_ctx* ctx, uint32_t id, const chp_equation* eqs, uint32_t 
   k_solve_rows<R><<<1, 256, 0, st>>>(dw, (int)id, ctx->d_eq, (int)n, dt);
   const int lcap = levels_lds_cap(nbig, S.nb, ctx->max_lds);
   k_levels<R><<<1, bl, lds_levels(bl, lcap), st>>>(dw, ctx->d_list, nbig, 1, lcap, 1);
-  launch_gs<R>(dw, ctx->d_list, 1, ctx->gsg, S.nb, ctx->max_lds, bg, 1, self, st);
+  if (self) launch_gs<R, true>(dw, ctx->d_list, 1, ctx->gsg, S.nb, ctx->max_lds, bg, 1, st);
+  else launch_gs<R>(dw, ctx->d_list, 1, ctx->gsg, S.nb, ctx->max_lds, bg, 1, st);
   k_solve_finish<R><<<1, 256, 0, st>>>(dw, (int)id);
   HIPCHK(ctx, hipGetLastError());
   HIPCHK(ctx, hipStreamSynchronize(st));

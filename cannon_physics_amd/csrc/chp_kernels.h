@@ -339,10 +339,9 @@ __global__ __launch_bounds__(256) void k_levels(const DevWorld<R>* __restrict__ 
 // they fit.
 constexpr int GS_SUB_MAX_NB = 512, GS_WAVE_NB = 128;
 constexpr int GS_SS_WAVE = 1024, GS_SS_SUB = 2048, GS_SS_BIG = 4096;   // step table entries in LDS
-#ifndef CHP_GS_DEPTH
-#define CHP_GS_DEPTH 4
-#endif
-template <typename R> constexpr int gs_depth() { return sizeof(R) == 4 ? CHP_GS_DEPTH : 2; }
+// ring depth: FP32 4, 6 and 8 measured 1188, 1165 and 1186 us on 1024 chains, 338, 329 and 324 us
+// on half a batch of 2048 piles, 60, 62 and 66 us on one 217-body world
+template <typename R> constexpr int gs_depth() { return sizeof(R) == 4 ? 6 : 2; }
 
 // the list positions of a list sorted by body count (largest first): [0, blk) over
 // GS_SUB_MAX_NB bodies, [blk, wave) a workgroup each, [wave, n) a wave each; and the largest body
@@ -363,35 +362,37 @@ static int big_lds_cap(int max_nb, size_t max_lds) {
   return std::min(max_nb, most);
 }
 
-template <typename R, int NW>
-__device__ __forceinline__ void gs_sub_run(const DevWorld<R>& W, float* vw, int nb_cap, double* shd, int* sh, int keep, int self) {
+template <typename R, int NW, bool SELF>
+__device__ __forceinline__ void gs_sub_run(const DevWorld<R>& W, float* vw, int nb_cap, double* shd, int* sh, int keep) {
   constexpr int D = gs_depth<R>();
   if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;   // k_split_gs solves its islands
-  const int steps = gs_steps(W.counters[C_LEVELS], W.counters[C_ROWS], 16 * NW, D);
+  const int E = uni(W.counters[C_ROWS]), steps = gs_steps(uni(W.counters[C_LEVELS]), E, 16 * NW, D);
   int* ss = (int*)(vw + 8 * (nb_cap + 1));
-  if (steps < (NW == 1 ? GS_SS_WAVE : GS_SS_SUB)) st_gs<R, NW, D, true>(W, vw, ss, shd, sh, keep != 0, self != 0);
-  else st_gs<R, NW, D, true>(W, vw, (int*)W.last_level, shd, sh, keep != 0, self != 0);
+  if (steps < (NW == 1 ? GS_SS_WAVE : GS_SS_SUB) && E <= gs_narrow_rows<R>())
+    st_gs<R, NW, D, true, SELF, false>(W, vw, ss, shd, sh, keep != 0);
+  else
+    st_gs<R, NW, 2, true, SELF, true>(W, vw, (int*)W.last_level, shd, sh, keep != 0);
 }
-template <typename R>
+template <typename R, bool SELF>
 __global__ __launch_bounds__(256) void k_gs_sub(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                GsSegs g, int n, int keep, int self) {
+                                                GsSegs g, int n, int keep) {
   __shared__ int sh[4];
   __shared__ double shd[4];
   extern __shared__ float4 lds_f4[];
   float* lds = (float*)lds_f4;
   const int b = (int)blockIdx.x, nsub = g.wave - g.blk;
   if (b < nsub) {
-    gs_sub_run<R, 4>(worlds[list[g.blk + b]], lds, g.nb_sub, shd, sh, keep, self);
+    gs_sub_run<R, 4, SELF>(worlds[list[g.blk + b]], lds, g.nb_sub, shd, sh, keep);
   } else {
     const int wave = uni((int)(threadIdx.x >> 6)), idx = g.wave + (b - nsub) * 4 + wave;
     if (idx >= n) return;
-    gs_sub_run<R, 1>(worlds[list[idx]], lds + wave * (8 * (g.nb_wave + 1) + GS_SS_WAVE), g.nb_wave, shd, sh, keep, self);
+    gs_sub_run<R, 1, SELF>(worlds[list[idx]], lds + wave * (8 * (g.nb_wave + 1) + GS_SS_WAVE), g.nb_wave, shd, sh, keep);
   }
 }
 // the worlds over GS_SUB_MAX_NB bodies; big_cap: body velocities that fit in the launch's LDS
-template <typename R, int NW>
+template <typename R, int NW, bool SELF>
 __global__ __launch_bounds__(64 * NW) void k_gs(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                int big_cap, int keep, int self) {
+                                                int big_cap, int keep) {
   __shared__ int sh[1];
   __shared__ double shd[NW];
   extern __shared__ float4 lds_f4[];
@@ -400,27 +401,30 @@ __global__ __launch_bounds__(64 * NW) void k_gs(const DevWorld<R>* __restrict__ 
   if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;
   int* ss = (int*)lds_f4;
   float* vw = (float*)(ss + GS_SS_BIG);
-  const int steps = gs_steps(W.counters[C_LEVELS], W.counters[C_ROWS], 16 * NW, D);
-  if (steps >= GS_SS_BIG) st_gs<R, NW, D, false>(W, W.vw, (int*)W.last_level, shd, sh, keep != 0, self != 0);
-  else if (W.nb <= big_cap) st_gs<R, NW, D, true>(W, vw, ss, shd, sh, keep != 0, self != 0);
-  else st_gs<R, NW, D, false>(W, W.vw, ss, shd, sh, keep != 0, self != 0);
+  const int E = uni(W.counters[C_ROWS]), steps = gs_steps(uni(W.counters[C_LEVELS]), E, 16 * NW, D);
+  if (steps >= GS_SS_BIG || E > gs_narrow_rows<R>())
+    st_gs<R, NW, 2, false, SELF, true>(W, W.vw, (int*)W.last_level, shd, sh, keep != 0);
+  else if (W.nb <= big_cap)
+    st_gs<R, NW, D, true, SELF, false>(W, vw, ss, shd, sh, keep != 0);
+  else
+    st_gs<R, NW, D, false, SELF, false>(W, W.vw, ss, shd, sh, keep != 0);
 }
 
 // the GS stage of a list (the level schedule and the GS records are in place).  rows: rows a
-// large world runs at a time (64, 128 or 256: four lanes each).  self: the rows may hold one whose
+// large world runs at a time (64, 128 or 256: four lanes each).  SELF: the rows may hold one whose
 // two bodies are one (the Solver slot)
-template <typename R>
+template <typename R, bool SELF = false>
 static void launch_gs(const DevWorld<R>* dw, const int* d_list, int n, const GsSegs& g, int max_nb, size_t max_lds, int rows,
-                      int keep, int self, hipStream_t st) {
+                      int keep, hipStream_t st) {
   if (g.blk) {
     const int cap = big_lds_cap(max_nb, max_lds);
     const size_t lds = GS_SS_BIG * sizeof(int) + (size_t)(cap + 1) * 8 * sizeof(float);
-    if (rows == 64) k_gs<R, 4><<<g.blk, 256, lds, st>>>(dw, d_list, cap, keep, self);
-    else if (rows == 128) k_gs<R, 8><<<g.blk, 512, lds, st>>>(dw, d_list, cap, keep, self);
-    else k_gs<R, 16><<<g.blk, 1024, lds, st>>>(dw, d_list, cap, keep, self);
+    if (rows == 64) k_gs<R, 4, SELF><<<g.blk, 256, lds, st>>>(dw, d_list, cap, keep);
+    else if (rows == 128) k_gs<R, 8, SELF><<<g.blk, 512, lds, st>>>(dw, d_list, cap, keep);
+    else k_gs<R, 16, SELF><<<g.blk, 1024, lds, st>>>(dw, d_list, cap, keep);
   }
   const int nsub = (g.wave - g.blk) + (n - g.wave + 3) / 4;
-  if (nsub) k_gs_sub<R><<<nsub, 256, lds_gs_sub(g), st>>>(dw, d_list, g, n, keep, self);
+  if (nsub) k_gs_sub<R, SELF><<<nsub, 256, lds_gs_sub(g), st>>>(dw, d_list, g, n, keep);
 }
 
 // World.step(dt, timeSinceLastCalled): the interpolated poses and World.time += the elapsed time

@@ -85,7 +85,7 @@ template <typename R> __device__ __forceinline__ R block_sum(R v, R* sh) {
   return r;
 }
 // flag bits of the body indices in the solver's row records
-enum : unsigned { GS_DYN = 0x80000000u, GS_NEG = 0x40000000u, GS_IDX = 0x3fffffffu };
+enum : unsigned { GS_DYN = 0x80000000u, GS_IDX = 0x3fffffffu };
 
 // barrier that orders LDS only: outstanding global loads (prefetches) stay in flight
 __device__ __forceinline__ void lds_barrier() {
@@ -1299,8 +1299,8 @@ struct GWave {
 // GS record: 6 groups of 4 words, row position k at words [k * 24, k * 24 + 24)
 //   g0 sa.x sa.y sa.z ima  | g1 ra.x ra.y ra.z B    | g2 rb.x rb.y rb.z invC
 //   g3 ia.x ia.y ia.z eps  | g4 ib.x ib.y ib.z minF | g5 imb maxF a' b'
-// a' = a | (a dynamic) << 31 | (sb == -sa, else both spatial parts are +0) << 30,
-// b' = b | (b dynamic) << 31.  row_ab holds a and b with the same dynamic bits.  The groups are
+// a' = a | (a dynamic) << 31, b' = b | (b dynamic) << 31, as in row_ab; imb (never negative) has its
+// sign set when sb == -sa (else both spatial parts are +0).  The groups are
 // what the four lanes of a row load (st_gs): each a Jacobian part and the part its impulse moves
 // the velocity along, with one of the row's scalars in the fourth word.
 template <typename R> struct GsWord;
@@ -1320,7 +1320,10 @@ template <typename R> struct GsRow {
   f3 sa, ra, rb, ia, ib;
   R ima, imb, B, invC, eps, minF, maxF;
   unsigned a, b;
+  bool neg;   // sb == -sa
 };
+// the sign bit of a word that holds an R
+template <typename R> __device__ __forceinline__ bool flip_top(typename GsWord<R>::T w) { return (w >> (8 * sizeof(R) - 1)) != 0; }
 
 template <typename R> __device__ __forceinline__ void gs_load(const typename GsWord<R>::T* base, int k, GsRow<R>& o) {
   typedef typename GsWord<R>::T T;
@@ -1340,7 +1343,8 @@ template <typename R> __device__ __forceinline__ void gs_load(const typename GsW
   auto S = [&](int i) { return GsWord<R>::get(w[i]); };
   o.sa = mk3(F(0), F(1), F(2)); o.ra = mk3(F(4), F(5), F(6)); o.rb = mk3(F(8), F(9), F(10));
   o.ia = mk3(F(12), F(13), F(14)); o.ib = mk3(F(16), F(17), F(18));
-  o.ima = S(3); o.imb = S(20); o.B = S(7); o.invC = S(11); o.eps = S(15); o.minF = S(19); o.maxF = S(21);
+  o.neg = flip_top<R>(w[20]);
+  o.ima = S(3); o.imb = o.neg ? -S(20) : S(20); o.B = S(7); o.invC = S(11); o.eps = S(15); o.minF = S(19); o.maxF = S(21);
   o.a = (unsigned)w[22]; o.b = (unsigned)w[23];
 }
 
@@ -1354,9 +1358,10 @@ template <typename R> __device__ __forceinline__ void gs_store(typename GsWord<R
   P(8, r.rb.x); P(9, r.rb.y); P(10, r.rb.z); P(11, r.invC);
   P(12, r.ia.x); P(13, r.ia.y); P(14, r.ia.z); P(15, r.eps);
   P(16, r.ib.x); P(17, r.ib.y); P(18, r.ib.z); P(19, r.minF);
-  P(20, r.imb); P(21, r.maxF);
+  P(21, r.maxF);
   bool neg = !(r.kind == CHP_ROW_ROTATIONAL || r.kind == CHP_ROW_CONE || r.kind == CHP_ROW_MOTOR);
-  w[22] = (T)(fa | (neg ? GS_NEG : 0u));
+  P(20, neg ? -r.imb : r.imb);
+  w[22] = (T)fa;
   w[23] = (T)fb;
 #pragma unroll
   for (int g = 0; g < GS_GROUPS; g++) {
@@ -1589,7 +1594,7 @@ template <typename R> __device__ __forceinline__ R gs_row(const GsRow<R>& cr, fl
   const int a = cr.a & GS_IDX, b = cr.b & GS_IDX;
   const bool da = cr.a & GS_DYN, db = cr.b & GS_DYN;
   const f3 z = mk3(0.f, 0.f, 0.f);
-  const f3 sb = (cr.a & GS_NEG) ? neg3(cr.sa) : z;
+  const f3 sb = cr.neg ? neg3(cr.sa) : z;
   const R clam = lam[0];
   float4 va4 = ((const float4*)vw)[2 * a], wa4 = ((const float4*)vw)[2 * a + 1];
   float4 vb4 = ((const float4*)vw)[2 * b], wb4 = ((const float4*)vw)[2 * b + 1];
@@ -1662,21 +1667,29 @@ template <typename R> struct GsQuad {
 // = E), the sweep is padded to a multiple of the ring depth D with empty steps, and each thread's
 // record and lambda are loaded D steps ahead into a ring of registers.  A sweep is at least D
 // steps, so a row's lambda is stored before it is loaded again, by the same threads.  A thread
-// without a row runs the record at row_cap, all zeros, whose impulse is zero; its writes, and those
-// of bodies that are not dynamic, go to a spare body slot at nb.
+// without a row runs the record at position E, all zeros, whose impulse is zero; its writes, and
+// those of bodies that are not dynamic, go to a spare body slot at nb.
+//
+// Within a step the next step's body velocities are read straight after this step's are written
+// (the barrier between them when NW > 1), and the ring's loads are issued while they arrive.
 //   vw: 8 floats per body slot (vlambda xyz, pad, wlambda xyz, pad), nb + 1 slots, in LDS when LDS
 //   ss: gs_steps + 1 ints (in LDS or global memory)
-//   self: rows whose two bodies are one are present (the Solver slot may be given them)
-// an upper bound of the entries a sweep's step table takes (see st_gs)
+//   SELF: rows whose two bodies are one may be present (the Solver slot may be given them)
+//   WIDE: record offsets may pass 32 bits
+// an upper bound of the entries a sweep's step table takes
 __host__ __device__ constexpr int gs_steps(int L, int E, int rows_per_step, int D) { return L + E / rows_per_step + D; }
-template <typename R, int NW, int D, bool LDS>
-__device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, double* shd, int* sh, bool keep,
-                                      bool self) {
+// rows whose record offsets fit 24 x 24 bit multiplications (full rate) and 32 bits
+template <typename R> constexpr int gs_narrow_rows() {
+  const unsigned k = 0xffffffffu / (4 * GS_GROUPS * sizeof(R)) - 1;
+  return (int)(k < 0xffffffu ? k : 0xffffffu);
+}
+template <typename R, int NW, int D, bool LDS, bool SELF, bool WIDE>
+__device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, double* shd, int* sh, bool keep) {
   constexpr int T = 64 * NW, RP = 16 * NW;
   const int tid = NW == 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x, p = tid & 3, row = tid >> 2;
-  const int E = uni(W.counters[C_ROWS]), L = uni(W.counters[C_LEVELS]), iters = uni(W.iterations);
-  const int nb = uni(W.nb), dummy = uni(W.row_cap);
+  const int E = uni(W.counters[C_ROWS]), L = uni(W.counters[C_LEVELS]), iters = uni(W.iterations), nb = uni(W.nb);
   const R tol2 = W.tol2;
+  typedef typename GsWord<R>::T WT;
   auto sync = [&]() {
     if constexpr (NW == 1) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     else __syncthreads();
@@ -1707,33 +1720,45 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
   }
   const int Lpad = max(1, (Lp + D - 1) / D) * D;
   for (int t = Lp + tid; t <= Lpad; t += T) ss[t] = E;
-  typedef typename GsWord<R>::T WT;
-  const WT* gsr = (const WT*)W.gsr;
-  R* lam = W.glam;
-  if (tid == 0) {
-    lam[2 * (size_t)dummy] = (R)0;
-    lam[2 * (size_t)dummy + 1] = (R)0;
-  }
+  const char* gsr = (const char*)(const WT*)W.gsr;
+  char* lam = (char*)(R*)W.glam;
+  constexpr unsigned REC = 4 * GS_GROUPS * sizeof(R), LAM = 2 * sizeof(R);   // bytes per row
+  if (tid < 4 * GS_GROUPS) ((WT*)(gsr + (size_t)E * REC))[tid] = (WT)0;      // the idle threads' record
+  if (tid < 2) ((R*)(lam + (size_t)E * LAM))[tid] = (R)0;
   sync();
   int it = 0;
   if (E != 0 && iters > 0) {
-    const unsigned oa = p == 1 ? 4u : p == 3 ? 8u : 0u, ok = p == 1 ? 12u : p == 3 ? 16u : 0u;   // words
-    const unsigned negm = p == 2 ? GS_NEG : 0u;
-    const bool first = p < 2;
-    const int half = p & 1;
+    // this lane's groups of a record, its half of a body slot, the sign of its spatial part
+    const unsigned oa = (p == 1 ? 4u : p == 3 ? 8u : 0u) * sizeof(R), ok = (p == 1 ? 12u : p == 3 ? 16u : 0u) * sizeof(R);
+    const unsigned negm = p == 2 ? 0x80000000u : 0u, half = (p & 1) * 16u, spare = 32u * nb + half;
+    const bool first = p < 2, odd = p & 1;
+    char* vb = (char*)vw;
     GsQuad<R> qa[D], qk[D], qc[D];
     R ql[D];
-    int qr[D];
-    int pt = 0;   // the next step to load
-    auto load = [&](int s, int s0, int s1) {
-      const int k = s0 + row < s1 ? s0 + row : dummy;
-      const unsigned w = (unsigned)k * (4u * GS_GROUPS);
-      qa[s].load(gsr + (size_t)(w + oa));
-      qk[s].load(gsr + (size_t)(w + ok));
-      qc[s].load(gsr + (size_t)(w + 20u));
-      ql[s] = lam[2 * (size_t)(unsigned)k];
+    unsigned qr[D];   // the row's position
+    int pt = 0, s0, s1;   // the next step to load and its rows
+    auto fetch = [&]() { s0 = ss[pt]; s1 = ss[pt + 1]; };
+    auto load = [&](int s) {
+      const unsigned k = (unsigned)(s0 + row < s1 ? s0 + row : E);
+      if constexpr (WIDE) {
+        const size_t o = (size_t)k * REC;
+        qa[s].load((const WT*)(gsr + (o + oa)));
+        qk[s].load((const WT*)(gsr + (o + ok)));
+        qc[s].load((const WT*)(gsr + (o + 20 * sizeof(R))));
+        ql[s] = *(const R*)(lam + (size_t)k * LAM);
+      } else {
+        qa[s].load((const WT*)(gsr + (__umul24(k, REC) + oa)));
+        qk[s].load((const WT*)(gsr + (__umul24(k, REC) + ok)));
+        qc[s].load((const WT*)(gsr + (__umul24(k, REC) + 20u * (unsigned)sizeof(R))));
+        ql[s] = *(const R*)(lam + k * LAM);
+      }
       qr[s] = k;
-      if (++pt == Lpad) pt = 0;
+      pt = pt + 1 == Lpad ? 0 : pt + 1;
+    };
+    // the body slot half this lane reads for slot s's row
+    auto body = [&](int s) {
+      const unsigned w = first ? (unsigned)qc[s].w[2] : (unsigned)qc[s].w[3];
+      return (w << 5) + half;
     };
     // The sweeps run in an inner loop whose only memory traffic is the ring's loads and the
     // lambda stores.  The rare undecided early-exit test reads the stored |dlambda| outside
@@ -1742,11 +1767,15 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
       pt = 0;
 #pragma unroll
       for (int s = 0; s < D; s++) {
-        load(s, ss[pt], ss[pt + 1]);
+        fetch();
+        load(s);
         __builtin_amdgcn_sched_barrier(0);   // the slots' loads stay in slot order
       }
+      fetch();
       int step = 0, dec = 0;   // dec, the sweep-end decision: 1 stop, -1 undecided
       double part = 0.0;
+      unsigned at = body(0);
+      float4 v4 = *(const float4*)(vb + at);
       for (;;) {
 #pragma unroll
         for (int s = 0; s < D; s++) {
@@ -1754,12 +1783,8 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
           // slot's row before its own step makes the wave wait for that row's loads, and the
           // ring then hides no latency
           __builtin_amdgcn_sched_barrier(0);
-          const unsigned wa = (unsigned)qc[s].w[2], wb = (unsigned)qc[s].w[3];
-          const unsigned w = first ? wa : wb;
-          const int slot = 2 * (int)(w & GS_IDX) + half;
-          const float4 v4 = ((const float4*)vw)[slot];
-          const int s0 = ss[pt], s1 = ss[pt + 1];
-          const unsigned neg = (wa & negm) << 1;
+          const unsigned wa = (unsigned)qc[s].w[2], wb = (unsigned)qc[s].w[3], w = first ? wa : wb;
+          const unsigned neg = (unsigned)(qc[s].w[0] >> (8 * sizeof(R) - 32)) & negm;
           const R jx = flip_sign(qa[s].get(0), neg), jy = flip_sign(qa[s].get(1), neg), jz = flip_sign(qa[s].get(2), neg);
           R d = (R)v4.x * jx;
           d += (R)v4.y * jy;
@@ -1774,27 +1799,31 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
           // the clamp of gs_solver.dart:91-96 as selects; NaN compares false, as in the branches
           const R t = clam + dl;
           dl = t < minF ? minF - clam : (t > maxF ? maxF - clam : dl);
-          const R adlv = dl > (R)0 ? dl : -dl;
-          part += (double)adlv;
-          R* lp = lam + 2 * (size_t)(unsigned)qr[s];
-          if constexpr (sizeof(R) == 4) *(float2*)lp = make_float2((float)(clam + dl), (float)adlv);
-          else *(double2*)lp = make_double2((double)(clam + dl), (double)adlv);
           // va += (ima dl) sa, wa += dl ia, vb += (imb dl) sb, wb += dl ib
-          const R c = half ? (R)1 : (first ? own : qc[s].get(0));
+          const R c = odd ? (R)1 : (first ? own : (R)fabs(qc[s].get(0)));
           const R sc = flip_sign(c * dl, neg);
           const R kx = qk[s].get(0), ky = qk[s].get(1), kz = qk[s].get(2);
           float4 o = make_float4((float)((R)v4.x + sc * kx), (float)((R)v4.y + sc * ky), (float)((R)v4.z + sc * kz), 0.f);
-          int wslot = (w & GS_DYN) ? slot : 2 * nb + half;
-          if (self) {   // one body on both sides: its second impulse follows the first
+          unsigned to = (w & GS_DYN) ? at : spare;
+          if constexpr (SELF) {   // one body on both sides: its second impulse follows the first
             const bool same = ((wa ^ wb) & GS_IDX) == 0;
             const float ax = quad<0x44>(o.x), ay = quad<0x44>(o.y), az = quad<0x44>(o.z);   // lanes 0, 1, 0, 1
             if (same && !first && (wa & GS_DYN))
               o = make_float4((float)((R)ax + sc * kx), (float)((R)ay + sc * ky), (float)((R)az + sc * kz), 0.f);
-            if (same && first) wslot = 2 * nb + half;
+            if (same && first) to = spare;
           }
-          ((float4*)vw)[wslot] = o;
-          load(s, s0, s1);   // the slot's next row (D steps on)
+          *(float4*)(vb + to) = o;
           step_sync();
+          at = body((s + 1) % D);
+          v4 = *(const float4*)(vb + at);
+          __builtin_amdgcn_sched_barrier(0);
+          const R adlv = (R)fabs(dl);
+          part += (double)adlv;
+          R* lp = (R*)(WIDE ? lam + (size_t)qr[s] * LAM : lam + qr[s] * LAM);
+          if constexpr (sizeof(R) == 4) *(float2*)lp = make_float2((float)(clam + dl), (float)adlv);
+          else *(double2*)lp = make_double2((double)(clam + dl), (double)adlv);
+          load(s);   // the slot's next row (D steps on)
+          fetch();
         }
         step += D;
         if (step == Lpad) {   // end of a sweep: GSSolver's early-exit test
@@ -1825,7 +1854,7 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
       if (tid == 0) {
         const int* rpos = W.rpos;
         R tot = 0;
-        for (int r = 0; r < E; r++) tot += lam[2 * (size_t)(unsigned)rpos[r] + 1];
+        for (int r = 0; r < E; r++) tot += ((const R*)(lam + (size_t)(unsigned)rpos[r] * LAM))[1];
         vv = tot * tot < tol2 ? 1 : 0;
         if (NW > 1) sh[0] = vv;
       }
@@ -1842,7 +1871,7 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
     sync();
     // Equation.multiplier and the capture read lambda from the row records (keep)
     if (keep)
-      for (int k = tid; k < E; k += T) W.rows[W.sched[k]].lambda = lam[2 * (size_t)k];
+      for (int k = tid; k < E; k += T) W.rows[W.sched[k]].lambda = *(const R*)(lam + (size_t)k * LAM);
   }
   // hand the lambda velocities to st_post
   for (int i = tid; i < nb; i += T) {

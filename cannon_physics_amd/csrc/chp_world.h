@@ -130,7 +130,7 @@ template <typename R> struct DevWorld {
   CHP_G(RowRec<R>) rows;
   CHP_G(int) level, sched, lvl_start, last_level, row_ab, rpos;
   CHP_G(R) glam;   // per row position in level order: lambda, |dlambda| of the last sweep (row_cap + 1)
-  CHP_G(void) gsr;   // GS records in level order (24 R-sized words per row; all zeros at row_cap)
+  CHP_G(void) gsr;   // GS records in level order (24 R-sized words per row, row_cap + 1 of them)
   CHP_G(float) vw;   // vlambda / wlambda, 8 floats per body and a spare slot, when the world is too big for LDS
   CHP_G(unsigned long long) sort_keys;
   // large SAP worlds (see BP_BIG): the sweep's body data in axis-list order (position and
