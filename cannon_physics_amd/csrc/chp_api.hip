@@ -25,11 +25,9 @@ CHP_NARROW_KERNELS(extern template __global__, float)
 CHP_NARROW_KERNELS(extern template __global__, double)
 }  // namespace chp
 
-__global__ __launch_bounds__(1024) void k_narrow_scan(int* __restrict__ qcls, int n, int* __restrict__ bounds) {
-  __shared__ int sh[1024];
-  st_narrow_scan(qcls, n, bounds, sh);
+__global__ __launch_bounds__(64) void k_queue_clear(int* qw) {
+  if (threadIdx.x < 2 * NP_NCLS) qw[QW_TOT + threadIdx.x] = 0;
 }
-
 // counter words of the listed worlds; the pointers and the words are in pinned host memory
 __global__ __launch_bounds__(256) void k_gather_status(const int* const* __restrict__ counters, int n, int* __restrict__ out) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
@@ -190,6 +188,9 @@ struct WorldSlot {
   double last_dt = -1;
   bool may_sleep = false;  // World.allowSleep, or a body asleep: the step runs the wake-up pass
   bool split = false;      // World.solver is a SplitSolver
+  unsigned classes = 0;    // narrowphase classes its pairs can have (bit NP_*), without justTest pairs
+  bool kinematic = false;  // has kinematic bodies (their justTest pairs are on the wave path)
+  bool joints = false;     // has constraints
   double accumulator = 0;  // World.accumulator of World.step(dt, timeSinceLastCalled)
   // contact events: one device allocation (keys, sort buffers, scan, justTest list, control
   // words, events) while a kind mask is set
@@ -225,7 +226,8 @@ struct ListState {
   size_t d_big_cap = 0;
   std::vector<int> h_big;
   int big_nspans = 0, big_ntiles = 0, big_nw = 0, big_rounds = 0;
-  int n_sap = 0, n_sleep = 0, n_events = 0, n_split = 0;
+  int n_sap = 0, n_sleep = 0, n_events = 0, n_split = 0, n_joints = 0;
+  unsigned classes = 0;
   GsSegs gsg;
   int2* d_q = nullptr;
   size_t d_q_cap = 0;
@@ -262,6 +264,8 @@ struct chp_ctx {
   int n_sleep = 0; // worlds in the current list that may hold sleeping bodies
   int n_events = 0; // worlds in the current list with contact events on
   int n_split = 0;  // worlds in the current list with a SplitSolver
+  int n_joints = 0; // worlds in the current list with constraints
+  unsigned classes = 0;   // narrowphase classes the current list's pairs can have
   GsSegs gsg;       // the GS kernels' segments of the current list
   ListState second;          // the second stream's list state (see ListState)
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -288,7 +292,7 @@ struct chp_ctx {
     bool keep = false;
     double dt = 0;
     const void *dq = nullptr, *dqcls = nullptr, *dlist = nullptr, *dworlds = nullptr, *dbig = nullptr;
-    std::array<int, 8> big{};
+    std::array<int, 10> big{};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
   } sg;
@@ -340,6 +344,8 @@ static void swap_lists(chp_ctx* ctx) {
   std::swap(ctx->n_sleep, o.n_sleep);
   std::swap(ctx->n_events, o.n_events);
   std::swap(ctx->n_split, o.n_split);
+  std::swap(ctx->n_joints, o.n_joints);
+  std::swap(ctx->classes, o.classes);
   std::swap(ctx->gsg, o.gsg);
   std::swap(ctx->d_q, o.d_q);
   std::swap(ctx->d_q_cap, o.d_q_cap);
@@ -375,6 +381,38 @@ static void default_caps(int nb, int nhf, int& pairs, int& contacts, int& rows) 
 
 template <typename R> static int events_alloc(chp_ctx* ctx, WorldSlot& S, uint32_t mask, int cap);
 static void events_free(chp_ctx* ctx, WorldSlot& S);
+
+// the narrowphase classes (bits NP_*) pairs of the world's bodies can have, by the shapes present
+// (pair_class without its justTest rule): a step launches only the classes its worlds can fill.
+// An empty class kernel costs a launch, 5 us, and 27 us where a workgroup holds the wave path's
+// LDS.
+template <typename R> static unsigned world_classes(const HostWorld<R>& H) {
+  int ns = 0, np = 0, nbx = 0, nc = 0, nf = 0, other = 0;
+  for (int i = 0; i < H.nb; i++) {
+    if (H.shape_count[i] != 1) { other++; continue; }
+    switch (H.si_type[H.shape_first[i]]) {
+      case CHP_SHAPE_SPHERE: ns++; break;
+      case CHP_SHAPE_PLANE: np++; break;
+      case CHP_SHAPE_BOX: nbx++; break;
+      case CHP_SHAPE_CONVEX: nc++; break;
+      case CHP_SHAPE_HEIGHTFIELD: nf++; break;
+      default: other++;
+    }
+  }
+  unsigned m = 0;
+  auto on = [&](bool c, int cls) { if (c) m |= 1u << cls; };
+  on(ns > 1, NP_SS);
+  on(ns && np, NP_SP);
+  on(ns && nbx, NP_SB);
+  on(ns && nc, NP_SC);
+  on(np && nbx + nc, NP_PC);
+  on(nbx + nc > 1, NP_CC);
+  on(nf && ns + nbx + nc, NP_WHC);
+  on(nc > 0, NP_WHC);              // large hulls take the wave path
+  on(np + nf > 1 || other, NP_OTHER);   // plane / heightfield pairs have no resolver
+  on(other > 0, NP_WAVE);
+  return m;
+}
 
 template <typename R>
 static int build_slot(chp_ctx* ctx, WorldSlot& S, const HostWorld<R>& H, int pair_cap, int contact_cap, int row_cap) {
@@ -512,6 +550,9 @@ static int build_slot(chp_ctx* ctx, WorldSlot& S, const HostWorld<R>& H, int pai
   S.may_sleep = H.wd.allow_sleep != 0;
   for (int v : H.sleep_state) S.may_sleep = S.may_sleep || v == CHP_SLEEP_SLEEPING;
   S.split = H.wd.solver == CHP_SOLVER_SPLIT;
+  S.classes = world_classes(H);
+  S.kinematic = std::count(H.type.begin(), H.type.end(), (int)CHP_BODY_KINEMATIC) > 0;
+  S.joints = !H.c_type.empty();
   S.shape_body = H.shape_body;
   S.devworld.assign((char*)&D, (char*)&D + sizeof(D));
   if (S.ev.mask) {   // a rebuilt slab keeps the event bookkeeping (sized for the new capacities)
@@ -780,18 +821,20 @@ static int check_status(chp_ctx* ctx, const uint32_t* ids, uint32_t n) {
 }
 
 // the narrowphase queue holds one entry per pair of the listed worlds (at most their pair
-// capacities); qcls holds the per-world class counts and the class bounds
+// capacities); qcls holds the queue's words
 static int ensure_queue(chp_ctx* ctx, const uint32_t* ids, uint32_t n) {
   size_t need = 1;
   for (uint32_t k = 0; k < n; k++) need += (size_t)ctx->worlds[ids[k]].pair_cap;
   if (need > ((size_t)1 << 31) - 1) return fail(ctx, CHP_E_CAPACITY, "more than 2^31 pairs in one batch");
-  size_t ncls = (size_t)n * NP_NCLS + NP_NCLS + 1 + NP_NTICKET;
+  const size_t ncls = queue_words(n);
   if (ctx->d_qcls_cap < ncls) {
     if (ctx->d_qcls) (void)hipFree(ctx->d_qcls);
     ctx->d_qcls = nullptr;
     ctx->d_qcls_cap = 0;
     HIPCHK(ctx, hipMalloc(&ctx->d_qcls, ncls * sizeof(int)));
     ctx->d_qcls_cap = ncls;
+    k_queue_clear<<<1, 64, 0, ctx->stream>>>(ctx->d_qcls);
+    HIPCHK(ctx, hipGetLastError());
   }
   if (ctx->d_q_cap >= need) return CHP_OK;
   if (ctx->d_q) (void)hipFree(ctx->d_q);
@@ -801,6 +844,9 @@ static int ensure_queue(chp_ctx* ctx, const uint32_t* ids, uint32_t n) {
   ctx->d_q_cap = need;
   return CHP_OK;
 }
+
+// the narrowphase classes of a step of the world
+static unsigned step_classes(const WorldSlot& S) { return S.classes | (S.ev.mask && S.kinematic ? 1u << NP_WAVE : 0u); }
 
 // uploads the world list of the next launches and the large-world tables that go with it (the
 // host copies stay alive in the context until the next upload)
@@ -838,12 +884,16 @@ static int upload_list(chp_ctx* ctx, const std::vector<int>& list) {
   ctx->n_sleep = 0;
   ctx->n_events = 0;
   ctx->n_split = 0;
+  ctx->n_joints = 0;
+  ctx->classes = 0;
   for (size_t li = 0; li < n; li++) {
     const WorldSlot& S = ctx->worlds[list[li]];
     if (S.broadphase == CHP_BROADPHASE_SAP) ctx->n_sap++;
     if (S.may_sleep) ctx->n_sleep++;
     if (S.ev.mask) ctx->n_events++;
     if (S.split) ctx->n_split++;
+    if (S.joints) ctx->n_joints++;
+    ctx->classes |= step_classes(S);
     if (S.nb < BP_BIG) continue;
     bigw.push_back((int)li);
     for (int s0 = 0; s0 < S.nb; s0 += BP_SPAN) { spans.push_back((int)li); spans.push_back(s0); }
@@ -885,7 +935,8 @@ struct StepView {
   const void* worlds = nullptr;
   const int* list = nullptr;
   const int* big = nullptr;
-  int nspans = 0, ntiles = 0, nw = 0, rounds = 0, n_sap = 0, n_sleep = 0, n_events = 0, n_split = 0;
+  int nspans = 0, ntiles = 0, nw = 0, rounds = 0, n_sap = 0, n_sleep = 0, n_events = 0, n_split = 0, n_joints = 0;
+  unsigned classes = 0;
   GsSegs gsg;
   int2* q = nullptr;
   size_t qcap = 0;
@@ -904,11 +955,23 @@ static StepView ctx_view(const chp_ctx* ctx) {
   v.n_sleep = ctx->n_sleep;
   v.n_events = ctx->n_events;
   v.n_split = ctx->n_split;
+  v.n_joints = ctx->n_joints;
+  v.classes = ctx->classes;
   v.gsg = ctx->gsg;
   v.q = ctx->d_q;
   v.qcap = ctx->d_q_cap;
   v.qcls = ctx->d_qcls;
   return v;
+}
+
+// the broadphase of the listed worlds of fewer than BP_BIG bodies (n_sap of them SAP worlds).  A
+// world has a workgroup: of 1024 threads while the worlds leave CUs idle, else of 256, four to a
+// CU (one 300-body world 108 us with the 256 threads and FP64 tests it had before)
+template <typename R>
+static void launch_bp(const DevWorld<R>* dw, const int* list, int n, int max_nb, int n_sap, int* qw, hipStream_t st) {
+  const int lds_nb = std::min(max_nb, BP_BIG - 1), bd = n <= 256 ? 1024 : 256;
+  if (n_sap < n) k_bp<R, false><<<n, bd, BpLds<R>::bytes(lds_nb, false), st>>>(dw, list, lds_nb, qw);
+  if (n_sap) k_bp<R, true><<<n, bd, BpLds<R>::bytes(lds_nb, true), st>>>(dw, list, lds_nb, qw);
 }
 
 // the broadphase of the large worlds of the list (after k_bp, which leaves them alone)
@@ -946,37 +1009,31 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
   hipStream_t st = ctx->stream;
   if (ev) HIPCHK(ctx, hipEventRecord(ev[0], st));
   {
-    // naive broadphase body data in LDS when it fits beside the static LDS (4 KiB kept free)
-    int lds_nb = max_nb;
-    while (lds_nb > 0 && BpLds<R>::bytes(lds_nb) > ctx->max_lds - 4096) lds_nb--;
-    k_bp<R, false><<<n, 256, BpLds<R>::bytes(lds_nb), st>>>(dw, d_list, lds_nb);
-    if (V.n_sap) k_bp<R, true><<<n, 256, 0, st>>>(dw, d_list, 0);
+    launch_bp<R>(dw, d_list, n, max_nb, V.n_sap, V.qcls, st);
     launch_big_bp<R>(V, st);
   }
   if (ev) HIPCHK(ctx, hipEventRecord(ev[1], st));
   {
     const int qcap = (int)V.qcap;
-    int* bounds = V.qcls + (size_t)n * NP_NCLS;
-    // the per-world classification passes: 256 threads a world (a world's pairs are a few
-    // dependent loads each, so the largest worlds' loops set the time)
-    k_narrow_count<R><<<n, 256, 0, st>>>(dw, d_list, V.qcls, n);
-    if (V.nw) k_big_ncount<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls, n);
-    k_narrow_scan<<<1, 1024, 0, st>>>(V.qcls, n, bounds);
-    k_narrow<R><<<n, 256, 0, st>>>(dw, d_list, V.qcls, V.q, n);
-    if (V.nw) k_big_nplace<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls, V.q, n);
-    // one kernel per thread class (each compiles only its resolver), up to 4 waves per SIMD
+    int* bounds = V.qcls + QW_BOUNDS;
+    if (V.nw) k_big_ncount<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls);
+    k_narrow<R><<<n, 256, 0, st>>>(dw, d_list, V.qcls, V.q);
+    if (V.nw) k_big_nplace<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls, V.q);
+    // one kernel per thread class that the listed worlds can fill (each compiles only its
+    // resolver), up to 4 waves per SIMD
     const int blocks = (std::max(64, std::min(qcap, 256 * 4 * 4 * 64)) + 63) / 64;
-    k_narrow_cls<R, NP_SS><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    k_narrow_cls<R, NP_SP><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    k_narrow_cls<R, NP_SB><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    k_narrow_cls<R, NP_SC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    k_narrow_cls<R, NP_PC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    k_narrow_cls<R, NP_CC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    k_narrow_cls<R, NP_OTHER><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    auto has = [&](int c) { return (V.classes >> c) & 1u; };
+    if (has(NP_SS)) k_narrow_cls<R, NP_SS><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_SP)) k_narrow_cls<R, NP_SP><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_SB)) k_narrow_cls<R, NP_SB><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_SC)) k_narrow_cls<R, NP_SC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_PC)) k_narrow_cls<R, NP_PC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_CC)) k_narrow_cls<R, NP_CC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_OTHER)) k_narrow_cls<R, NP_OTHER><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
     const int waves = std::max(1, std::min(qcap, 4096));
-    k_narrow_wave<R, NP_WHC><<<(waves + 3) / 4, 256, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_WHC)) k_narrow_wave<R, NP_WHC><<<(waves + 3) / 4, 256, 0, st>>>(dw, V.q, bounds, dt);
     // compound-body pairs are rare: a small grid, strided over however many there are
-    k_narrow_wave<R, NP_WAVE><<<32, 256, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_WAVE)) k_narrow_wave<R, NP_WAVE><<<32, 256, 0, st>>>(dw, V.q, bounds, dt);
     if (V.n_sleep) k_wake<R><<<n, 256, 0, st>>>(dw, d_list);
     if (V.n_events) k_events<R><<<n, 1024, 0, st>>>(dw, d_list, 0);
   }
@@ -984,19 +1041,19 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
   // rows: offsets, then the rows' body pairs; the level schedule; then the rows, written as GS
   // records in level order (keep: also as row records, for the capture)
   const int keep = ctx->keep_rows ? 1 : 0;
-  const int* qbounds = V.qcls + (size_t)n * NP_NCLS;
+  const int* qbounds = V.qcls + QW_BOUNDS;
   // one queued pair per thread: a grid of up to 1M threads (a pair's rows are a chain of
   // dependent loads, so the more pairs in flight the better; the resident waves are what the
   // registers allow, the rest wait for a slot)
   const int qblocks = (std::max(64, std::min((int)V.qcap, 256 * 4 * 16 * 64)) + 63) / 64;
   auto build_rows = [&]() {
     k_pair_rows<R, ROWS_GS><<<qblocks, 64, 0, st>>>(dw, V.q, qbounds, dt, keep);
-    k_joint_rows<R, ROWS_GS><<<n, 64, 0, st>>>(dw, d_list, dt, keep);
+    if (V.n_joints) k_joint_rows<R, ROWS_GS><<<n, 64, 0, st>>>(dw, d_list, dt, keep);
   };
-  k_rows<R><<<n, 128, 0, st>>>(dw, d_list);
+  k_rows<R><<<n, 128, 0, st>>>(dw, d_list, V.qcls);
   if (V.nw) k_big_rowscan<R><<<V.nw, 1024, 0, st>>>(dw, d_list, V.bigw());
   k_pair_rows<R, ROWS_AB><<<qblocks, 64, 0, st>>>(dw, V.q, qbounds, dt, 0);
-  k_joint_rows<R, ROWS_AB><<<n, 64, 0, st>>>(dw, d_list, dt, 0);
+  if (V.n_joints) k_joint_rows<R, ROWS_AB><<<n, 64, 0, st>>>(dw, d_list, dt, 0);
   if (V.n_split) k_split_prep<R><<<n, 1024, 0, st>>>(dw, d_list);
   if (ev) HIPCHK(ctx, hipEventRecord(ev[3], st));
   if (tune) {
@@ -1037,6 +1094,12 @@ static void drop_graph(chp_ctx* ctx) {
   ctx->sg = chp_ctx::StepGraph();
 }
 
+// what of the list decides which kernels a step launches, and their grids
+static std::array<int, 10> step_shape(const chp_ctx* ctx) {
+  return {ctx->big_nspans, ctx->big_ntiles, ctx->big_nw, ctx->big_rounds, ctx->n_sap, ctx->n_sleep, ctx->n_events, ctx->n_split,
+          ctx->n_joints, (int)ctx->classes};
+}
+
 // the captured step for this configuration (captured anew when anything baked into its kernel
 // arguments changed)
 template <typename R>
@@ -1046,8 +1109,7 @@ static int step_graph(chp_ctx* ctx, const std::vector<int>& list, int nbig, int 
   *out = nullptr;
   if (!(g.valid && g.list == list && g.nbig == nbig && g.max_nb == max_nb && g.dt == dt && g.bl == ctx->levels_block && g.keep == ctx->keep_rows &&
         g.bg == ctx->solve_block && g.dq == ctx->d_q && g.dqcls == ctx->d_qcls && g.dlist == ctx->d_list &&
-        g.dbig == ctx->d_big && g.big == std::array<int, 8>{ctx->big_nspans, ctx->big_ntiles, ctx->big_nw, ctx->big_rounds, ctx->n_sap, ctx->n_sleep,
-                                       ctx->n_events, ctx->n_split} &&
+        g.dbig == ctx->d_big && g.big == step_shape(ctx) &&
         g.dworlds == ctx->d_worlds)) {
     if (!may_capture) return CHP_OK;
     drop_graph(ctx);
@@ -1066,8 +1128,7 @@ static int step_graph(chp_ctx* ctx, const std::vector<int>& list, int nbig, int 
     g.valid = true; g.list = list; g.nbig = nbig; g.max_nb = max_nb; g.dt = dt;
     g.bl = ctx->levels_block; g.bg = ctx->solve_block; g.keep = ctx->keep_rows;
     g.dq = ctx->d_q; g.dqcls = ctx->d_qcls; g.dlist = ctx->d_list; g.dworlds = ctx->d_worlds;
-    g.dbig = ctx->d_big; g.big = {ctx->big_nspans, ctx->big_ntiles, ctx->big_nw, ctx->big_rounds, ctx->n_sap, ctx->n_sleep, ctx->n_events,
-             ctx->n_split};
+    g.dbig = ctx->d_big; g.big = step_shape(ctx);
     g.graph = graph;
     g.exec = exec;
   }
@@ -1279,7 +1340,7 @@ template <typename R> static int step_noalloc_t(chp_ctx* ctx, uint32_t id, doubl
   };
   const size_t nbig_ints = 2 * (size_t)nspans + 2 * (size_t)ntiles + (big ? 1 : 0);
   const size_t o_tab = take(sizeof(DevWorld<R>)), o_list = take(sizeof(int)), o_big = take(nbig_ints * sizeof(int)),
-               o_qcls = take((2 * NP_NCLS + 1 + NP_NTICKET) * sizeof(int)), o_q = take((size_t)S.pair_cap * sizeof(int2));
+               o_qcls = take(queue_words(1) * sizeof(int)), o_q = take((size_t)S.pair_cap * sizeof(int2));
   if (off > NOALLOC_SCRATCH_BYTES)
     return fail(ctx, CHP_E_CAPACITY, "world " + std::to_string(id) + " needs " + std::to_string(off) +
                                          " bytes of step buffers; the no-allocation path holds " +
@@ -1307,6 +1368,8 @@ template <typename R> static int step_noalloc_t(chp_ctx* ctx, uint32_t id, doubl
   V.n_sleep = S.may_sleep ? 1 : 0;
   V.n_events = S.ev.mask ? 1 : 0;
   V.n_split = S.split ? 1 : 0;
+  V.n_joints = S.joints ? 1 : 0;
+  V.classes = step_classes(S);
   V.gsg.blk = S.nb > GS_SUB_MAX_NB ? 1 : 0;
   V.gsg.wave = S.nb > GS_WAVE_NB ? 1 : 0;
   V.gsg.nb_sub = V.gsg.wave > V.gsg.blk ? S.nb : 0;
@@ -1314,6 +1377,7 @@ template <typename R> static int step_noalloc_t(chp_ctx* ctx, uint32_t id, doubl
   V.qcls = (int*)(base + o_qcls);
   V.q = (int2*)(base + o_q);
   V.qcap = (size_t)S.pair_cap;
+  k_queue_clear<<<1, 64, 0, ctx->stream>>>(V.qcls);
   HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
   for (int s = 0; s < nsteps; s++) {
     r = launch_step<R>(ctx, V, 1, S.nb > SMALL_NB ? 1 : 0, S.nb, dt, nullptr);
@@ -1459,13 +1523,10 @@ static int step_interp_t(chp_ctx* ctx, uint32_t id, double dt, double elapsed, i
 template <typename R> static int broadphase_t(chp_ctx* ctx, uint32_t id, int32_t* pi, int32_t* pj, uint32_t cap, uint32_t* np) {
   int r = prepare<R>(ctx, &id, 1, ctx->worlds[id].last_dt > 0 ? ctx->worlds[id].last_dt : 1.0 / 60);
   if (r != CHP_OK) return r;
-  if (ctx->worlds[id].nb >= BP_BIG) {
-    r = upload_list(ctx, {(int)id});
-    if (r != CHP_OK) return r;
-    launch_big_bp<R>(ctx_view(ctx), ctx->stream);
-  } else {
-    k_broadphase<R><<<1, CHP_BLOCK, 0, ctx->stream>>>((const DevWorld<R>*)ctx->d_worlds, (int)id);
-  }
+  r = upload_list(ctx, {(int)id});
+  if (r != CHP_OK) return r;
+  if (ctx->worlds[id].nb >= BP_BIG) launch_big_bp<R>(ctx_view(ctx), ctx->stream);
+  else launch_bp<R>((const DevWorld<R>*)ctx->d_worlds, ctx->d_list, 1, ctx->worlds[id].nb, ctx->n_sap, nullptr, ctx->stream);
   HIPCHK(ctx, hipGetLastError());
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   DevWorld<R>& D = dev_of<R>(ctx->worlds[id]);

@@ -19,24 +19,6 @@ __device__ __forceinline__ u64 ev_key(int a, int b) {
 // bits that hold every index below n
 __device__ __forceinline__ int ev_bits(int n) { return n <= 2 ? 1 : 32 - __clz(n - 1); }
 
-// exclusive scan of one value per thread over the workgroup (blockDim.x a multiple of 64); sh
-// needs blockDim.x / 64 ints
-__device__ __forceinline__ int tile_exscan(int v, int* sh, int* total) {
-  const int lane = (int)(threadIdx.x & 63), wv = (int)(threadIdx.x >> 6), nw = (int)(blockDim.x >> 6);
-  const int inc = wave_incl_scan(v);
-  if (lane == 63) sh[wv] = inc;
-  __syncthreads();
-  int before = 0, tot = 0;
-  for (int w = 0; w < nw; w++) {
-    const int x = sh[w];
-    before += w < wv ? x : 0;
-    tot += x;
-  }
-  __syncthreads();
-  *total = tot;
-  return before + inc - v;
-}
-
 // stable LSD sort of a[0..n) on bits [0, kb) of the low word, then [32, 32 + kb) of the high
 // word, one bit per pass: keys with the bit clear keep their order ahead of the keys with it
 // set; a pass whose bit is the same in every key moves nothing.  Returns the buffer holding

@@ -23,35 +23,37 @@ namespace chp {
 
 // gravity / solve mass / AABBs, broadphase and the collideConnected filter.  One kernel per
 // broadphase kind (each holds only its code and registers), each skipping the other kind's
-// worlds.  Dynamic LDS holds the naive broadphase's body data of worlds with at most lds_nb
-// bodies.
+// worlds.  Dynamic LDS holds the broadphase data of worlds of at most lds_nb bodies.  The pairs
+// are then counted by narrowphase class (qw: the queue's words; null: the Broadphase slot, the
+// pairs alone).
 template <typename R, bool SAP>
-__global__ __launch_bounds__(256) void k_bp(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                            int lds_nb) {
-  __shared__ int sh[256];
-  extern __shared__ double lds_d[];
-  CHP_WORLD_PROLOGUE
+__global__ __launch_bounds__(1024) void k_bp(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                             int lds_nb, int* __restrict__ qw) {
+  __shared__ int sh[32];
+  extern __shared__ float4 lds_bp[];
+  const DevWorld<R>& W = worlds[list[blockIdx.x]];
+  if (qw && block_bcast(W.counters[C_STATUS], sh) != 0) return;
   if ((W.broadphase == CHP_BROADPHASE_SAP) != SAP) return;
-  if (threadIdx.x == 0) {
+  if (qw && threadIdx.x == 0) {
     W.counters[C_STAGING] = 0;
     if (W.ev_mask) W.ev_ctl[EV_JT] = 0;
   }
-  if (W.nb >= BP_BIG) return;  // the grid-wide kernels below take large worlds
-  st_prestep<R, SAP>(W);
-  __syncthreads();
-  bool ok;
-  if constexpr (SAP) {
-    ok = st_bp_sap(W, sh);
-  } else {
-    BpLds<R> L;
-    if (W.nb <= lds_nb) {
-      L.carve(lds_d, lds_nb);
-      ok = st_bp_naive<R, true>(W, sh, L);
-    } else {
-      ok = st_bp_naive<R, false>(W, sh, L);
-    }
+  if (W.nb > lds_nb) return;  // the grid-wide kernels below take large worlds
+  if (qw) {
+    st_prestep<R, SAP>(W);
+  } else if (SAP) {
+    for (int i = threadIdx.x; i < W.nb; i += blockDim.x)
+      if (W.flags[i] & BF_AABB_DIRTY) { body_aabb(W, i); W.flags[i] &= ~BF_AABB_DIRTY; }
   }
-  if (ok) st_filter(W);
+  __syncthreads();
+  BpLds<R> L;
+  L.carve(lds_bp, lds_nb, SAP);
+  bool ok;
+  if constexpr (SAP) ok = st_bp_sap(W, sh, L);
+  else ok = st_bp_naive(W, sh, L);
+  if (!ok || !qw) return;
+  st_filter(W);
+  st_narrow_count(W, qw, (int)blockIdx.x, sh);
 }
 
 // large worlds (at least BP_BIG bodies): prestep, SAP sort and pair passes over the grid.
@@ -117,8 +119,8 @@ __global__ __launch_bounds__(1024) void k_big_scan(const DevWorld<R>* __restrict
 }
 
 // narrowphase class counts and queue placement of a large world's pairs: the world's spans are
-// its K workers, worker k takes pairs k * 256 + t, stride K * 256.  Counts add into the world's
-// qcls entries (zeroed by k_narrow_count); placement reserves each class range per workgroup.
+// its K workers, worker k takes pairs k * 256 + t, stride K * 256.  Counts add into the class
+// totals; placement reserves each class range per workgroup.
 template <typename R>
 __device__ __forceinline__ void big_pair_classes(const DevWorld<R>& W, int2 sp, int* sh, bool mark_filtered) {
   const int K = (W.nb + BP_SPAN - 1) / BP_SPAN, k = sp.y / BP_SPAN, P = W.counters[C_PAIRS];
@@ -133,19 +135,19 @@ __device__ __forceinline__ void big_pair_classes(const DevWorld<R>& W, int2 sp, 
 }
 template <typename R>
 __global__ __launch_bounds__(256) void k_big_ncount(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                    const int2* __restrict__ spans, int* __restrict__ qcls, int n) {
+                                                    const int2* __restrict__ spans, int* __restrict__ qw) {
   __shared__ int sh[NP_NCLS];
   CHP_SPAN_PROLOGUE(spans)
   if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = 0;
   __syncthreads();
   big_pair_classes(W, sp, sh, true);
   __syncthreads();
-  if (threadIdx.x < NP_NCLS && sh[threadIdx.x]) atomicAdd(&qcls[threadIdx.x * n + sp.x], sh[threadIdx.x]);
+  if (threadIdx.x < NP_NCLS && sh[threadIdx.x]) atomicAdd(&qw[QW_TOT + threadIdx.x], sh[threadIdx.x]);
 }
 template <typename R>
 __global__ __launch_bounds__(256) void k_big_nplace(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                    const int2* __restrict__ spans, int* __restrict__ qcls,
-                                                    int2* __restrict__ q, int n) {
+                                                    const int2* __restrict__ spans, int* __restrict__ qw,
+                                                    int2* __restrict__ q) {
   __shared__ int sh[NP_NCLS];
   CHP_SPAN_PROLOGUE(spans)
   if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = 0;
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(256) void k_big_nplace(const DevWorld<R>* __restric
   big_pair_classes(W, sp, sh, false);
   __syncthreads();
   if (threadIdx.x < NP_NCLS)
-    sh[threadIdx.x] = sh[threadIdx.x] ? atomicAdd(&qcls[threadIdx.x * n + sp.x], sh[threadIdx.x]) : 0;
+    sh[threadIdx.x] = sh[threadIdx.x] ? queue_base(qw) + atomicAdd(&qw[QW_CUR + threadIdx.x], sh[threadIdx.x]) : 0;
   __syncthreads();
   const int K = (W.nb + BP_SPAN - 1) / BP_SPAN, k = sp.y / BP_SPAN, P = W.counters[C_PAIRS], wid = list[sp.x];
   for (int p = k * 256 + (int)threadIdx.x; p < P; p += K * 256) {
@@ -196,29 +198,17 @@ __global__ __launch_bounds__(64) void k_big_post(const DevWorld<R>* __restrict__
   if (i < W.nb && !post_body(W, i, (R)dt, W.counters[C_ROWS], post_qn(W))) W.counters[C_POSTFAIL] = 1;
 }
 
-// narrowphase: per-class pair counts per world, class-major offsets, placement in the queue,
-// then one pair per thread over the thread classes and one pair per wave over the wave class,
-// each grid-wide over the whole batch.  qcls: class-major, qcls[c * n + list index]; bounds:
-// NP_NCLS + 1 ints, then the wave classes' NP_NTICKET pair tickets.
-template <typename R>
-__global__ __launch_bounds__(256) void k_narrow_count(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                      int* __restrict__ qcls, int n) {
-  __shared__ int sh[64];
-  int* cnt = qcls + blockIdx.x;
-  const DevWorld<R>& W = worlds[list[blockIdx.x]];
-  if (block_bcast(W.counters[C_STATUS], sh) != 0 || W.nb >= BP_BIG) {  // large worlds: k_big_ncount
-    if (threadIdx.x < NP_NCLS) cnt[threadIdx.x * n] = 0;
-    return;
-  }
-  st_narrow_count(W, cnt, n, sh);
-}
+// narrowphase: the pairs placed in the queue by class (the counts are the broadphase's), then one
+// pair per thread over the thread classes and one pair per wave over the wave class, each
+// grid-wide over the whole batch.
 template <typename R>
 __global__ __launch_bounds__(256) void k_narrow(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                const int* __restrict__ qcls, int2* __restrict__ q, int n) {
+                                                int* __restrict__ qw, int2* __restrict__ q) {
   __shared__ int sh[64];
+  if (blockIdx.x == 0) queue_bounds(qw);
   CHP_WORLD_PROLOGUE
   if (W.nb >= BP_BIG) return;  // k_big_nplace
-  st_narrow_place(W, list[blockIdx.x], qcls + blockIdx.x, n, q, sh);
+  st_narrow_place(W, list[blockIdx.x], qw, (int)blockIdx.x, q, sh);
 }
 // classes whose resolvers clip polygons (convex-convex, and the mixed class) hold the clip
 // polygons of the block's 64 lanes in LDS
@@ -245,8 +235,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // contact rows of every queued pair (one pair per thread over the whole batch), then the joint
 // rows (one workgroup per world)
 template <typename R>
-__global__ __launch_bounds__(128) void k_rows(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list) {
+__global__ __launch_bounds__(128) void k_rows(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                              int* __restrict__ qw) {
   __shared__ int sh[128];
+  if (blockIdx.x == 0 && threadIdx.x < 2 * NP_NCLS) qw[QW_TOT + threadIdx.x] = 0;   // totals and cursors of the next step
   CHP_WORLD_PROLOGUE
   if (W.nb >= BP_BIG) return;
   st_rowscan(W, sh);
@@ -519,22 +511,6 @@ __global__ __launch_bounds__(256) void k_post(const DevWorld<R>* __restrict__ wo
     return;
   }
   st_post(W, dt);
-}
-
-// broadphase only (Broadphase.collisionPairs on the current state)
-template <typename R>
-__global__ __launch_bounds__(CHP_BLOCK) void k_broadphase(const DevWorld<R>* __restrict__ worlds, int wid) {
-  __shared__ int sh[CHP_BLOCK];
-  const DevWorld<R>& W = worlds[wid];
-  if (W.broadphase == CHP_BROADPHASE_SAP) {
-    for (int i = threadIdx.x; i < W.nb; i += blockDim.x)
-      if (W.flags[i] & BF_AABB_DIRTY) { body_aabb(W, i); W.flags[i] &= ~BF_AABB_DIRTY; }
-    __syncthreads();
-    st_bp_sap(W, sh);
-  } else {
-    BpLds<R> L;
-    st_bp_naive<R, false>(W, sh, L);
-  }
 }
 
 // Narrowphase slot: contacts for the pairs in the world's pair slab, then the equations

@@ -17,6 +17,8 @@ enum { C_STATUS = 0, C_PAIRS = 1, C_CONTACTS = 2, C_ROWS = 3, C_ITERS = 4, C_LEV
 
 __device__ __forceinline__ void ws_fail(int* counters, int bit) { atomicOr(&counters[C_STATUS], bit); }
 
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // exclusive scan of one value per thread; sh needs blockDim.x ints
 __device__ __forceinline__ int block_exscan(int v, int* sh, int* total) {
   int t = threadIdx.x, n = blockDim.x;
@@ -45,6 +47,23 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
     if (lane >= off) v += x;
   }
   return v;
+}
+// exclusive scan of one value per thread over the workgroup (blockDim.x a multiple of 64); sh
+// needs blockDim.x / 64 ints
+__device__ __forceinline__ int tile_exscan(int v, int* sh, int* total) {
+  const int lane = (int)(threadIdx.x & 63), wv = (int)(threadIdx.x >> 6), nw = (int)(blockDim.x >> 6);
+  const int inc = wave_incl_scan(v);
+  if (lane == 63) sh[wv] = inc;
+  __syncthreads();
+  int before = 0, tot = 0;
+  for (int w = 0; w < nw; w++) {
+    const int x = sh[w];
+    before += w < wv ? x : 0;
+    tot += x;
+  }
+  __syncthreads();
+  *total = tot;
+  return before + inc - v;
 }
 __device__ __forceinline__ int array_exscan(int* data, int n, int* sh) {
   const int nw = (int)(blockDim.x >> 6), wv = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
@@ -188,122 +207,132 @@ template <typename R> __device__ __forceinline__ bool bp_sphere(const DevWorld<R
 }
 __device__ __forceinline__ float axis_of(f3 v, int ax) { return ax == 0 ? v.x : (ax == 1 ? v.y : v.z); }
 
-// NaiveBroadphase.collisionPairs (naive_broadphase.dart:14-33): pairs (i, j), j < i, in i-major
-// order.  One wave per row i (rows dealt round-robin to the waves): the lanes test 64
-// consecutive j at a time, a ballot gives each passing lane its rank, so pairs come out in j
-// order.  Pass 1 counts per row, a scan gives the row offsets, pass 2 writes.  The body data
-// the tests read (position, bounding radius, filter group / mask, static flag) is staged in LDS
-// when the world fits (BpLds), else read from the slab; in LDS, pass 1 also keeps every chunk's
-// ballot mask, and pass 2 writes from the masks instead of testing again.
-// Row i has ceil(i / 64) chunks; the masks of rows 0..i-1 take bp_chunks(i) words.
+// The bounding-sphere predicate of bp_sphere_at decided in FP32 where the margin allows: 1 it
+// holds, 0 it does not, -1 undecided.  The difference of two FP32 coordinates rounded to FP32 is
+// the same through FP64 (twice the precision and two bits), so l2 and s2 are off their FP64 values
+// by a few FP32 roundings; the margin of 1e-5 is forty times that, and 1e-30 covers underflow.  An
+// infinite s2 (a plane's radius) holds for every finite l2, as it does in FP64.
+__device__ __forceinline__ int bp_screen(float4 a, float4 b) {
+  const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z, s = a.w + b.w;
+  const float l2 = dx * dx + dy * dy + dz * dz, s2 = s * s;
+  if (l2 < s2 * 0.99999f - 1e-30f) return 1;
+  return l2 > s2 * 1.00001f + 1e-30f ? 0 : -1;
+}
+
+// The broadphase data of a world of fewer than BP_BIG bodies, in LDS: position and radius (FP32),
+// filter group / mask / static-or-asleep flag / body, the radius in R when that is FP64, and the
+// naive pass's ballot masks or the SAP pass's sort keys.
+// Naive masks: row i has ceil(i / 64) words, those of rows 0..i-1 take bp_chunks(i).
 __host__ __device__ __forceinline__ int bp_chunks(int i) {
   if (i <= 1) return 0;
   const int a = (i - 1) >> 6, b = (i - 1) & 63;
   return (a + 1) * (32 * a + b);
 }
+__host__ __device__ __forceinline__ int bp_pow2(int n) {
+  int p = 1;
+  while (p < n) p <<= 1;
+  return p;
+}
 template <typename R> struct BpLds {
-  unsigned long long* masks;   // bp_chunks(n) words
-  float* pos;  // 3 per body
-  R* brad;
-  int* gm;     // group, mask per body
-  int* stat;   // 1: static or asleep
-  static __host__ __device__ size_t bytes(int n) {
-    return (size_t)bp_chunks(n) * sizeof(unsigned long long) + (size_t)n * (3 * sizeof(float) + sizeof(R) + 3 * sizeof(int));
+  float4* P;
+  int4* F;
+  unsigned long long* words;   // naive: bp_chunks(n); SAP: the keys, a power of two
+  R* rad;                      // FP64 only
+  int* cnt;                    // SAP: old positions, then pairs per row
+  static __host__ __device__ size_t bytes(int n, bool sap) {
+    return (size_t)n * (sizeof(float4) + sizeof(int4) + (sizeof(R) == 8 ? sizeof(R) : 0) + (sap ? sizeof(int) : 0)) +
+           (size_t)(sap ? bp_pow2(n) : bp_chunks(n)) * sizeof(unsigned long long);
   }
-  __device__ void carve(void* base, int cap) {
-    masks = (unsigned long long*)base;
-    brad = (R*)(masks + bp_chunks(cap));
-    pos = (float*)(brad + cap);
-    gm = (int*)(pos + 3 * cap);
-    stat = gm + 2 * cap;
+  __device__ void carve(void* base, int n, bool sap) {
+    P = (float4*)base;
+    F = (int4*)(P + n);
+    words = (unsigned long long*)(F + n);
+    rad = (R*)(words + (sap ? bp_pow2(n) : bp_chunks(n)));
+    cnt = (int*)(sizeof(R) == 8 ? rad + n : rad);
+  }
+  __device__ __forceinline__ double radius(int k) const {
+    if constexpr (sizeof(R) == 8) return (double)rad[k];
+    else return (double)P[k].w;
+  }
+  // body b's data at k
+  __device__ __forceinline__ void put(const DevWorld<R>& W, int k, int b) const {
+    const f3 p = F3<R>(W.pos, b);
+    const R r = W.brad[b];
+    P[k] = make_float4(p.x, p.y, p.z, (float)r);
+    F[k] = make_int4(W.group[b], W.mask[b], bp_passive(W, b) ? 1 : 0, b);
+    if constexpr (sizeof(R) == 8) rad[k] = r;
+  }
+  // needBroadphaseCollision of records x, y
+  static __device__ __forceinline__ bool need(int4 x, int4 y) {
+    return (x.x & y.y) != 0 && (y.x & x.y) != 0 && !(x.z && y.z);
   }
 };
-template <typename R, bool LDS>
-__device__ __forceinline__ bool bp_test(const DevWorld<R>& W, const BpLds<R>& L, int a, int b) {
-  if constexpr (LDS) {
-    if ((L.gm[2 * a] & L.gm[2 * b + 1]) == 0 || (L.gm[2 * b] & L.gm[2 * a + 1]) == 0) return false;
-    if (L.stat[a] && L.stat[b]) return false;
-    f3 pa = mk3(L.pos[3 * a], L.pos[3 * a + 1], L.pos[3 * a + 2]), pb = mk3(L.pos[3 * b], L.pos[3 * b + 1], L.pos[3 * b + 2]);
-    return bp_sphere_at(pa, (double)L.brad[a], pb, (double)L.brad[b]);
-  } else {
-    return bp_need(W, a, b) && bp_sphere(W, a, b);
-  }
-}
-template <typename R, bool LDS>
-__device__ __forceinline__ unsigned long long bp_row_chunk(const DevWorld<R>& W, const BpLds<R>& L, int i, int j0) {
-  int j = j0 + (int)(threadIdx.x & 63);
-  bool hit = j < i && bp_test<R, LDS>(W, L, i, j);
-  return __ballot(hit);
-}
-// body i's broadphase data from LDS, read once per row (the chunk loop stores ballot masks to
-// LDS, so the compiler could not keep these loads out of it)
-template <typename R> struct BpRowBody {
-  int group, mask, stat;
-  f3 p;
-  R r;
-  __device__ BpRowBody(const BpLds<R>& L, int i)
-      : group(L.gm[2 * i]), mask(L.gm[2 * i + 1]), stat(L.stat[i]), p(mk3(L.pos[3 * i], L.pos[3 * i + 1], L.pos[3 * i + 2])),
-        r(L.brad[i]) {}
-};
-// bp_test<R, true> (i, j) with body i's data held
-template <typename R>
-__device__ __forceinline__ unsigned long long bp_row_chunk_lds(const BpLds<R>& L, const BpRowBody<R>& A, int i, int j0) {
-  const int j = j0 + (int)(threadIdx.x & 63);
-  bool hit = false;
-  if (j < i && (A.group & L.gm[2 * j + 1]) != 0 && (L.gm[2 * j] & A.mask) != 0 && !(A.stat && L.stat[j])) {
-    const f3 pb = mk3(L.pos[3 * j], L.pos[3 * j + 1], L.pos[3 * j + 2]);
-    hit = bp_sphere_at(A.p, (double)A.r, pb, (double)L.brad[j]);
-  }
-  return __ballot(hit);
-}
-template <typename R, bool LDS> __device__ bool st_bp_naive(const DevWorld<R>& W, int* sh, const BpLds<R>& L) {
-  const int n = W.nb, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
-  if constexpr (LDS) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      f3 p = F3<R>(W.pos, i);
-      L.pos[3 * i] = p.x; L.pos[3 * i + 1] = p.y; L.pos[3 * i + 2] = p.z;
-      L.brad[i] = W.brad[i];
-      L.gm[2 * i] = W.group[i];
-      L.gm[2 * i + 1] = W.mask[i];
-      L.stat[i] = bp_passive(W, i);
-    }
-    __syncthreads();
-  }
-  for (int i = wave; i < n; i += nwave) {
-    int c = 0;
-    if constexpr (LDS) {
-      const BpRowBody<R> A(L, i);
-      for (int j0 = 0; j0 < i; j0 += 64) {
-        const unsigned long long m = bp_row_chunk_lds<R>(L, A, i, j0);
-        if (lane == 0) L.masks[bp_chunks(i) + (j0 >> 6)] = m;
-        c += __popcll(m);
+
+// NaiveBroadphase.collisionPairs (naive_broadphase.dart:14-33): pairs (i, j), j < i, in i-major
+// order.  A wave keeps 64 bodies j in registers and walks the rows i dealt to it, each row's data
+// read once for all 64 from LDS: 14 FP32 instructions screen a row, and only where one of its 64
+// spheres is near are the filters (and, undecided, the FP64 predicate) looked at.  The ballots
+// of a row's hits stay in LDS; in row order their set bits are the pairs in the reference's
+// order, so a scan of the population counts places them.
+template <typename R> __device__ bool st_bp_naive(const DevWorld<R>& W, int* sh, const BpLds<R>& L) {
+  const int n = W.nb, tid = (int)threadIdx.x, bd = (int)blockDim.x;
+  const int lane = tid & 63, wave = uni(tid >> 6), nwave = bd >> 6, nw = bp_chunks(n);
+  for (int i = tid; i < n; i += bd) L.put(W, i, i);
+  for (int w = tid; w < nw; w += bd) L.words[w] = 0ull;
+  __syncthreads();
+  for (int j0 = 0; j0 < n - 1; j0 += 64) {
+    const int j = j0 + lane;
+    const float4 pj = L.P[min(j, n - 1)];
+    const int4 fj = L.F[min(j, n - 1)];
+    int i = j0 + 1 + wave;
+    float4 pn = L.P[min(i, n - 1)];
+    for (; i < n; i += nwave) {
+      const float4 pi = pn;
+      pn = L.P[min(i + nwave, n - 1)];
+      const int scr = bp_screen(pi, pj);
+      if (!__any(j < i && scr != 0)) continue;
+      bool hit = j < i && scr != 0 && BpLds<R>::need(L.F[i], fj);
+      if (__any(hit && scr < 0)) {
+        const bool exact = bp_sphere_at(mk3(pi.x, pi.y, pi.z), L.radius(i), mk3(pj.x, pj.y, pj.z), L.radius(min(j, n - 1)));
+        hit = hit && (scr > 0 || exact);
       }
-    } else {
-      for (int j0 = 0; j0 < i; j0 += 64) c += __popcll(bp_row_chunk<R, LDS>(W, L, i, j0));
+      const unsigned long long m = __ballot(hit);
+      if (lane == 0 && m) L.words[bp_chunks(i) + (j0 >> 6)] = m;
     }
-    if (lane == 0) W.cnt[i] = c;
   }
   __syncthreads();
-  int P = array_exscan(W.cnt, n, sh);
+  const int K = (nw + bd - 1) / bd, w0 = min(nw, tid * K), w1 = min(nw, w0 + K);
+  int c = 0;
+  for (int w = w0; w < w1; w++) c += __popcll(L.words[w]);
+  int P;
+  int o = tile_exscan(c, sh, &P);
   if (P > W.pair_cap) {
-    if (threadIdx.x == 0) { W.counters[C_PAIRS] = P; ws_fail(W.counters, WS_PAIRS); }
+    if (tid == 0) { W.counters[C_PAIRS] = P; ws_fail(W.counters, WS_PAIRS); }
     return false;
   }
-  for (int i = wave; i < n; i += nwave) {
-    int o = W.cnt[i];
-    for (int j0 = 0; j0 < i; j0 += 64) {
-      unsigned long long m;
-      if constexpr (LDS) m = L.masks[bp_chunks(i) + (j0 >> 6)];
-      else m = bp_row_chunk<R, LDS>(W, L, i, j0);
-      if ((m >> lane) & 1ull) {
-        int k = o + __popcll(m & ((1ull << lane) - 1ull));
-        W.pair_i[k] = i;
-        W.pair_j[k] = j0 + lane;
+  if (c) {
+    int lo = 1, hi = n - 1;   // the row of word w0: the last i with bp_chunks(i) <= w0
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (bp_chunks(mid) <= w0) lo = mid;
+      else hi = mid - 1;
+    }
+    int i = lo, next = bp_chunks(i + 1), j0 = 64 * (w0 - bp_chunks(i));
+    for (int w = w0; w < w1; w++) {
+      if (w == next) {
+        i++;
+        next = bp_chunks(i + 1);
+        j0 = 0;
       }
-      o += __popcll(m);
+      for (unsigned long long m = L.words[w]; m; m &= m - 1) {
+        W.pair_i[o] = i;
+        W.pair_j[o] = j0 + __builtin_ctzll(m);
+        o++;
+      }
+      j0 += 64;
     }
   }
-  if (threadIdx.x == 0) W.counters[C_PAIRS] = P;
+  if (tid == 0) W.counters[C_PAIRS] = P;
   __syncthreads();
   return true;
 }
@@ -349,37 +378,76 @@ template <typename R> __device__ void sap_sort(const DevWorld<R>& W) {
   for (int k = threadIdx.x; k < n; k += blockDim.x) W.order[k] = W.tmp[(int)(key[k] & 0xffffffffu)];
   __syncthreads();
 }
-template <typename R> __device__ bool st_bp_sap(const DevWorld<R>& W, int* sh) {
-  int n = W.nb, ax = W.sap_axis;
-  sap_sort(W);
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    int bi = W.order[k], c = 0;
-    double A2 = (double)axis_of(F3<R>(W.pos, bi), ax) + (double)W.brad[bi];
-    for (int m = k + 1; m < n; m++) {
-      int bj = W.order[m];
-      if (!bp_need(W, bi, bj)) continue;
-      if (!((double)axis_of(F3<R>(W.pos, bj), ax) - (double)W.brad[bj] < A2)) break;
-      if (bp_sphere(W, bi, bj)) c++;
+// The whole of it for a world of fewer than BP_BIG bodies, from LDS: the bitonic sort, then one
+// wave per row over the sorted records, 64 candidates at a time, once to count and once to write.
+template <typename R> __device__ bool st_bp_sap(const DevWorld<R>& W, int* sh, const BpLds<R>& L) {
+  const int n = W.nb, ax = W.sap_axis, np2 = bp_pow2(n), tid = (int)threadIdx.x, bd = (int)blockDim.x;
+  const int lane = tid & 63, wave = uni(tid >> 6), nwave = bd >> 6;
+  for (int k = tid; k < np2; k += bd) {
+    unsigned long long key = ~0ull;
+    if (k < n) {
+      const int b = W.order[k];
+      key = ((unsigned long long)order_key(axis_of(F3<R>(W.aabb_lo, b), ax)) << 32) | (unsigned)k;
+      L.cnt[k] = b;
     }
-    W.cnt[k] = c;
+    L.words[k] = key;
   }
   __syncthreads();
-  int P = array_exscan(W.cnt, n, sh);
-  if (P > W.pair_cap) {
-    if (threadIdx.x == 0) { W.counters[C_PAIRS] = P; ws_fail(W.counters, WS_PAIRS); }
-    return false;
+  for (int size = 2; size <= np2; size <<= 1)
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      for (int t = tid; t < np2 / 2; t += bd) {
+        const int lo = ((t & ~(stride - 1)) << 1) | (t & (stride - 1)), hi = lo + stride;
+        const unsigned long long a = L.words[lo], b = L.words[hi];
+        if ((a > b) == ((lo & size) == 0)) { L.words[lo] = b; L.words[hi] = a; }
+      }
+      __syncthreads();
+    }
+  for (int k = tid; k < n; k += bd) {
+    const int b = L.cnt[(int)(L.words[k] & 0xffffffffu)];
+    W.order[k] = b;
+    L.put(W, k, b);
   }
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    int bi = W.order[k], o = W.cnt[k];
-    double A2 = (double)axis_of(F3<R>(W.pos, bi), ax) + (double)W.brad[bi];
-    for (int m = k + 1; m < n; m++) {
-      int bj = W.order[m];
-      if (!bp_need(W, bi, bj)) continue;
-      if (!((double)axis_of(F3<R>(W.pos, bj), ax) - (double)W.brad[bj] < A2)) break;
-      if (bp_sphere(W, bi, bj)) { W.pair_i[o] = bi; W.pair_j[o] = bj; o++; }
+  __syncthreads();
+  int P = 0;
+  for (int pass = 0; pass < 2; pass++) {
+    for (int k = wave; k < n; k += nwave) {
+      const float4 p4 = L.P[k];
+      const int4 gi = L.F[k];
+      const f3 pi = mk3(p4.x, p4.y, p4.z);
+      const double ri = L.radius(k), A2 = (double)axis_of(pi, ax) + ri;
+      int o = pass ? L.cnt[k] : 0;
+      for (int m0 = k + 1; m0 < n; m0 += 64) {
+        const int m = min(m0 + lane, n - 1);
+        const float4 q4 = L.P[m];
+        const int4 gj = L.F[m];
+        const f3 pj = mk3(q4.x, q4.y, q4.z);
+        const double rj = L.radius(m);
+        const bool need = m0 + lane < n && BpLds<R>::need(gi, gj);
+        const bool brk = need && !((double)axis_of(pj, ax) - rj < A2);
+        const bool hit = need && !brk && bp_sphere_at(pi, ri, pj, rj);
+        const unsigned long long bm = __ballot(brk);
+        unsigned long long hm = __ballot(hit);
+        if (bm) hm &= (1ull << __builtin_ctzll(bm)) - 1ull;
+        if (pass && ((hm >> lane) & 1ull)) {
+          const int r = o + __popcll(hm & ((1ull << lane) - 1ull));
+          W.pair_i[r] = gi.w;
+          W.pair_j[r] = gj.w;
+        }
+        o += __popcll(hm);
+        if (bm) break;
+      }
+      if (!pass && lane == 0) L.cnt[k] = o;
+    }
+    __syncthreads();
+    if (!pass) {
+      P = array_exscan(L.cnt, n, sh);
+      if (P > W.pair_cap) {
+        if (tid == 0) { W.counters[C_PAIRS] = P; ws_fail(W.counters, WS_PAIRS); }
+        return false;
+      }
     }
   }
-  if (threadIdx.x == 0) W.counters[C_PAIRS] = P;
+  if (tid == 0) W.counters[C_PAIRS] = P;
   __syncthreads();
   return true;
 }
@@ -481,8 +549,10 @@ template <typename R> __device__ int big_row(const DevWorld<R>& W, int k, bool e
       if (stop) break;
     }
   } else {
-    BpLds<R> L;
-    for (int j0 = 0; j0 < k; j0 += 64) put(bp_row_chunk<R, false>(W, L, k, j0), k, j0 + lane);
+    for (int j0 = 0; j0 < k; j0 += 64) {
+      const int j = j0 + lane;
+      put(__ballot(j < k && bp_need(W, k, j) && bp_sphere(W, k, j)), k, j);
+    }
   }
   return c;
 }
@@ -685,9 +755,17 @@ template <typename R> __device__ __forceinline__ int pair_class(const DevWorld<R
   return NP_OTHER;
 }
 
-// pass 1: per-class pair counts of the group's world (class c's count at cnt[c * stride])
-template <typename R> __device__ void st_narrow_count(const DevWorld<R>& W, int* cnt, int stride, int* sh) {
-  int P = W.counters[C_PAIRS];
+// The queue's words: class totals and cursors (zero between steps: k_rows clears them once the
+// step's queue is placed), the class bounds (bounds[c] = first entry of class c, bounds[NP_NCLS] =
+// total), the wave classes' tickets, then NP_NCLS pair counts per listed world.
+constexpr int QW_TOT = 0, QW_CUR = NP_NCLS, QW_BOUNDS = 2 * NP_NCLS, QW_TICKETS = QW_BOUNDS + NP_NCLS + 1,
+              QW_COUNTS = QW_TICKETS + NP_NTICKET;
+__host__ __device__ constexpr size_t queue_words(size_t nworlds) { return QW_COUNTS + nworlds * NP_NCLS; }
+
+// pass 1 (at the end of the broadphase): the pair counts of the workgroup's world by class, into
+// its words and the totals
+template <typename R> __device__ void st_narrow_count(const DevWorld<R>& W, int* qw, int idx, int* sh) {
+  const int P = W.counters[C_PAIRS];
   if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = 0;
   __syncthreads();
   for (int p = threadIdx.x; p < P; p += blockDim.x) {
@@ -696,106 +774,38 @@ template <typename R> __device__ void st_narrow_count(const DevWorld<R>& W, int*
     atomicAdd(&sh[pair_class(W, bi, bj)], 1);
   }
   __syncthreads();
-  if (threadIdx.x < NP_NCLS) cnt[threadIdx.x * stride] = sh[threadIdx.x];
+  if (threadIdx.x < NP_NCLS) {
+    const int c = sh[threadIdx.x];
+    qw[QW_COUNTS + idx * NP_NCLS + threadIdx.x] = c;
+    if (c) atomicAdd(&qw[QW_TOT + threadIdx.x], c);
+  }
 }
-
-// pass 2: the world's pairs into the queue at its offsets (class c's at off[c * stride])
+// the first queue entry of this thread's class (threads 0..NP_NCLS-1): the totals of the classes
+// before it
+__device__ __forceinline__ int queue_base(const int* qw) {
+  int base = 0;
+  for (int c = 0; c < NP_NCLS; c++) base += c < (int)threadIdx.x ? qw[QW_TOT + c] : 0;
+  return base;
+}
+// the class bounds and the tickets (one workgroup of the placement)
+__device__ __forceinline__ void queue_bounds(int* qw) {
+  if (threadIdx.x <= NP_NCLS) qw[QW_BOUNDS + threadIdx.x] = queue_base(qw);
+  if (threadIdx.x < NP_NTICKET) qw[QW_TICKETS + threadIdx.x] = 0;
+}
+// pass 2: the world's pairs into the queue, each class in a range reserved by its cursor (the
+// order of the worlds within a class is free)
 template <typename R>
-__device__ void st_narrow_place(const DevWorld<R>& W, int wid, const int* off, int stride, int2* q, int* sh) {
-  int P = W.counters[C_PAIRS];
-  if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = off[threadIdx.x * stride];
+__device__ void st_narrow_place(const DevWorld<R>& W, int wid, int* qw, int idx, int2* q, int* sh) {
+  const int P = W.counters[C_PAIRS];
+  if (threadIdx.x < NP_NCLS) {
+    const int c = qw[QW_COUNTS + idx * NP_NCLS + threadIdx.x];
+    sh[threadIdx.x] = c ? queue_base(qw) + atomicAdd(&qw[QW_CUR + threadIdx.x], c) : 0;
+  }
   __syncthreads();
   for (int p = threadIdx.x; p < P; p += blockDim.x) {
     int bi = W.pair_i[p], bj = W.pair_j[p];
     if (bi < 0) continue;
     q[atomicAdd(&sh[pair_class(W, bi, bj)], 1)] = make_int2(wid, p);
-  }
-}
-
-// between the passes: offsets class-major over the listed worlds.  cnt[c * n + w] holds world
-// w's count of class c and becomes its offset; bounds[c] = first entry of class c,
-// bounds[NP_NCLS] = total.  One workgroup: the class totals first, then rounds of bd worlds
-// (lane t of round j takes world j * bd + t: coalesced), each scanned at once for every class
-// by wave shuffles and one exchange of the wave totals.
-__device__ inline void st_narrow_scan(int* cnt, int n, int* bounds, int* sh) {
-  const int tid = threadIdx.x, bd = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = bd >> 6;
-  // the first RC rounds' counts are loaded once, all at the start, and kept in registers for the
-  // second pass (the block is alone on its CU: each round's loads would be a round trip)
-  constexpr int RC = 4;
-  int cache[RC][NP_NCLS];
-  int base[NP_NCLS];
-  {
-    int part[NP_NCLS];
-#pragma unroll
-    for (int c = 0; c < NP_NCLS; c++) part[c] = 0;
-#pragma unroll
-    for (int r = 0; r < RC; r++) {
-      const int w = r * bd + tid;
-#pragma unroll
-      for (int c = 0; c < NP_NCLS; c++) {
-        cache[r][c] = w < n ? cnt[c * n + w] : 0;
-        part[c] += cache[r][c];
-      }
-    }
-    for (int w = RC * bd + tid; w < n; w += bd)
-#pragma unroll
-      for (int c = 0; c < NP_NCLS; c++) part[c] += cnt[c * n + w];
-#pragma unroll
-    for (int c = 0; c < NP_NCLS; c++) {
-      for (int off = 32; off > 0; off >>= 1) part[c] += __shfl_xor(part[c], off, 64);
-      if (lane == 0) sh[wave * NP_NCLS + c] = part[c];
-    }
-    __syncthreads();
-    int run = 0;
-#pragma unroll
-    for (int c = 0; c < NP_NCLS; c++) {
-      int tot = 0;
-      for (int v = 0; v < nw; v++) tot += sh[v * NP_NCLS + c];
-      base[c] = run;
-      if (tid == 0) bounds[c] = run;
-      run += tot;
-    }
-    if (tid == 0) {
-      bounds[NP_NCLS] = run;
-      for (int t = 0; t < NP_NTICKET; t++) bounds[NP_NCLS + 1 + t] = 0;   // the wave classes' tickets
-    }
-    __syncthreads();
-  }
-  // one round: the counts v of world w (one per thread) become offsets
-  auto scan_round = [&](int w, const int (&v)[NP_NCLS]) {
-    int incl[NP_NCLS];
-#pragma unroll
-    for (int c = 0; c < NP_NCLS; c++) {
-      incl[c] = v[c];
-      for (int off = 1; off < 64; off <<= 1) {
-        int x = __shfl_up(incl[c], off, 64);
-        if (lane >= off) incl[c] += x;
-      }
-      if (lane == 63) sh[wave * NP_NCLS + c] = incl[c];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < NP_NCLS; c++) {
-      int woff = 0, tot = 0;
-      for (int u = 0; u < nw; u++) {
-        int t = sh[u * NP_NCLS + c];
-        woff += u < wave ? t : 0;
-        tot += t;
-      }
-      if (w < n) cnt[c * n + w] = base[c] + woff + incl[c] - v[c];
-      base[c] += tot;
-    }
-    __syncthreads();
-  };
-#pragma unroll
-  for (int r = 0; r < RC; r++)
-    if (r * bd < n) scan_round(r * bd + tid, cache[r]);
-  for (int w0 = RC * bd; w0 < n; w0 += bd) {
-    const int w = w0 + tid;
-    int v[NP_NCLS];
-#pragma unroll
-    for (int c = 0; c < NP_NCLS; c++) v[c] = w < n ? cnt[c * n + w] : 0;
-    scan_round(w, v);
   }
 }
 
@@ -1388,8 +1398,6 @@ template <typename R> __device__ __forceinline__ void gs_store(typename GsWord<R
 //         each chunk sees the previous chunk's values)
 //   hist: hist_cap ints of LDS for the level histogram (global scratch when L + 1 > hist_cap
 //         or not LDS)
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
 // gather: the rows are in their row records and go to GS records here; else the row builders
 // write the GS records afterwards, at the positions rpos this leaves
 template <typename R, typename G, bool LDS>
