@@ -990,6 +990,27 @@ template <typename R> static void launch_big_bp(const StepView& V, hipStream_t s
   k_big_rows<R><<<4 * ns, 256, 0, st>>>(dw, V.list, V.spans(), 1);
 }
 
+// the resolver kernels over the placed queue: one kernel per class that the listed worlds can fill
+// (each compiles only its resolver), the thread classes up to 4 waves per SIMD.  qcap: a bound of
+// the queue's length; clip_cap: points a wave pair's clip polygon may have
+template <typename R> static void launch_classes(const StepView& V, double dt, int qcap, int clip_cap, hipStream_t st) {
+  const DevWorld<R>* dw = (const DevWorld<R>*)V.worlds;
+  int* bounds = V.qcls + QW_BOUNDS;
+  const int blocks = (std::max(64, std::min(qcap, 256 * 4 * 4 * 64)) + 63) / 64;
+  auto has = [&](int c) { return (V.classes >> c) & 1u; };
+  if (has(NP_SS)) k_narrow_cls<R, NP_SS><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  if (has(NP_SP)) k_narrow_cls<R, NP_SP><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  if (has(NP_SB)) k_narrow_cls<R, NP_SB><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  if (has(NP_SC)) k_narrow_cls<R, NP_SC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  if (has(NP_PC)) k_narrow_cls<R, NP_PC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  if (has(NP_CC)) k_narrow_cls<R, NP_CC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  if (has(NP_OTHER)) k_narrow_cls<R, NP_OTHER><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  const int waves = std::max(1, std::min(qcap, 4096));
+  if (has(NP_WHC)) k_narrow_wave<R, NP_WHC><<<(waves + 3) / 4, 256, 0, st>>>(dw, V.q, bounds, dt, clip_cap);
+  // compound-body pairs are rare: a small grid, strided over however many there are
+  if (has(NP_WAVE)) k_narrow_wave<R, NP_WAVE><<<32, 256, 0, st>>>(dw, V.q, bounds, dt, clip_cap);
+}
+
 enum { K_BP = 0, K_NARROW, K_ROWS, K_LEVELS, K_GSROWS, K_GS, K_POST, K_NSTAGE };
 static const char* kStageNames[K_NSTAGE] = {"k_bp", "k_narrow", "k_rows", "k_levels", "k_gsrows", "k_gs", "k_post"};
 
@@ -1004,8 +1025,6 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
                                              hipEvent_t* ev, bool tune = false) {
   const DevWorld<R>* dw = (const DevWorld<R>*)V.worlds;
   const int* d_list = V.list;
-  auto groups = [&](int bd) { return nbig + (n - nbig + bd / 64 - 1) / (bd / 64); };
-  const int lcap = levels_lds_cap(nbig, max_nb, ctx->max_lds);
   hipStream_t st = ctx->stream;
   if (ev) HIPCHK(ctx, hipEventRecord(ev[0], st));
   {
@@ -1014,26 +1033,10 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
   }
   if (ev) HIPCHK(ctx, hipEventRecord(ev[1], st));
   {
-    const int qcap = (int)V.qcap;
-    int* bounds = V.qcls + QW_BOUNDS;
     if (V.nw) k_big_ncount<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls);
     k_narrow<R><<<n, 256, 0, st>>>(dw, d_list, V.qcls, V.q);
     if (V.nw) k_big_nplace<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls, V.q);
-    // one kernel per thread class that the listed worlds can fill (each compiles only its
-    // resolver), up to 4 waves per SIMD
-    const int blocks = (std::max(64, std::min(qcap, 256 * 4 * 4 * 64)) + 63) / 64;
-    auto has = [&](int c) { return (V.classes >> c) & 1u; };
-    if (has(NP_SS)) k_narrow_cls<R, NP_SS><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    if (has(NP_SP)) k_narrow_cls<R, NP_SP><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    if (has(NP_SB)) k_narrow_cls<R, NP_SB><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    if (has(NP_SC)) k_narrow_cls<R, NP_SC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    if (has(NP_PC)) k_narrow_cls<R, NP_PC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    if (has(NP_CC)) k_narrow_cls<R, NP_CC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    if (has(NP_OTHER)) k_narrow_cls<R, NP_OTHER><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-    const int waves = std::max(1, std::min(qcap, 4096));
-    if (has(NP_WHC)) k_narrow_wave<R, NP_WHC><<<(waves + 3) / 4, 256, 0, st>>>(dw, V.q, bounds, dt);
-    // compound-body pairs are rare: a small grid, strided over however many there are
-    if (has(NP_WAVE)) k_narrow_wave<R, NP_WAVE><<<32, 256, 0, st>>>(dw, V.q, bounds, dt);
+    launch_classes<R>(V, dt, (int)V.qcap, CLIP_WAVE, st);
     if (V.n_sleep) k_wake<R><<<n, 256, 0, st>>>(dw, d_list);
     if (V.n_events) k_events<R><<<n, 1024, 0, st>>>(dw, d_list, 0);
   }
@@ -1060,7 +1063,7 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
     for (int c = 0; c < 3; c++) {
       const int b = kTuneBlocks[c];
       HIPCHK(ctx, hipEventRecord(ctx->tev[3 * c], st));
-      k_levels<R><<<groups(b), b, lds_levels(b, lcap), st>>>(dw, d_list, nbig, n, lcap, 0);
+      launch_levels<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, b, st);
       build_rows();   // at the positions this schedule gave (the order inside a level may differ)
       HIPCHK(ctx, hipEventRecord(ctx->tev[3 * c + 1], st));
       launch_gs<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, b, keep, st);
@@ -1073,7 +1076,7 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
     }
   } else {
     const int bl = ctx->levels_block, bg = ctx->solve_block;
-    k_levels<R><<<groups(bl), bl, lds_levels(bl, lcap), st>>>(dw, d_list, nbig, n, lcap, 0);
+    launch_levels<R>(dw, d_list, n, V.gsg, max_nb, ctx->max_lds, bl, st);
     if (ev) HIPCHK(ctx, hipEventRecord(ev[4], st));
     build_rows();
     if (ev) HIPCHK(ctx, hipEventRecord(ev[5], st));
@@ -1651,7 +1654,7 @@ static int raycast_t(chp_ctx* ctx, uint32_t id, const chp_ray* rays, uint32_t nr
   const DevWorld<R>* dw = (const DevWorld<R>*)ctx->d_worlds;
   DevWorld<R>& D = dev_of<R>(S);
   HIPCHK(ctx, hipMemcpyAsync(d_rays, rays, nr * sizeof(chp_ray), hipMemcpyHostToDevice, st));
-  const int blocks = (int)std::min<uint32_t>((nr + 63) / 64, 4096);
+  const int blocks = (int)std::min<uint32_t>((nr + 3) / 4, 65536), icap = (int)std::min<uint32_t>(cap, 0x7fffffffu);
   // the world's ray has no heightfield cell index yet: the first ray (in order) whose walk calls
   // the heightfield intersection sets it
   if (!((HostWorld<R>*)S.host.get())->hf_nx.empty()) {
@@ -1714,20 +1717,31 @@ static int narrowphase_t(chp_ctx* ctx, uint32_t id, const int32_t* pi, const int
   if (r != CHP_OK) return r;
   r = ensure_eq(ctx, S.row_cap);
   if (r != CHP_OK) return r;
+  r = ensure_queue(ctx, &id, 1);
+  if (r != CHP_OK) return r;
+  r = upload_list(ctx, {(int)id});
+  if (r != CHP_OK) return r;
   DevWorld<R>& D = dev_of<R>(S);
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  hipStream_t hs = ctx->stream;
   if (np) {
-    HIPCHK(ctx, hipMemcpy(D.pair_i, pi, np * 4, hipMemcpyHostToDevice));
-    HIPCHK(ctx, hipMemcpy(D.pair_j, pj, np * 4, hipMemcpyHostToDevice));
+    HIPCHK(ctx, hipMemcpyAsync(D.pair_i, pi, np * 4, hipMemcpyHostToDevice, hs));
+    HIPCHK(ctx, hipMemcpyAsync(D.pair_j, pj, np * 4, hipMemcpyHostToDevice, hs));
   }
-  int c[C_COUNT];
-  HIPCHK(ctx, hipMemcpy(c, D.counters, sizeof c, hipMemcpyDeviceToHost));
-  c[C_PAIRS] = (int)np; c[C_STATUS] = 0; c[C_STAGING] = 0; c[C_ROWS] = 0;
-  HIPCHK(ctx, hipMemcpy(D.counters, c, sizeof c, hipMemcpyHostToDevice));
-  k_np_slot<R><<<1, 64, 0, ctx->stream>>>((const DevWorld<R>*)ctx->d_worlds, (int)id, dt, ctx->d_eq, S.row_cap);
+  // the step's queue and resolver kernels on the given pairs (450 bodies: 180 us, where one wave
+  // took every pair 1786 us), then the equations.  Clip polygons keep the thread path's capacity,
+  // the slot's limit
+  const StepView V = ctx_view(ctx);
+  const DevWorld<R>* dw = (const DevWorld<R>*)V.worlds;
+  k_np_queue<R><<<1, 1024, 0, hs>>>(dw, (int)id, (int)np, V.qcls, V.q);
+  if (np) launch_classes<R>(V, dt, (int)np, CLIP_THREAD, hs);
+  k_np_offsets<R><<<1, 1024, 0, hs>>>(dw, (int)id, S.row_cap);
+  if (np) k_np_equations<R><<<std::min<uint32_t>((np + 63) / 64, 16384), 64, 0, hs>>>(dw, (int)id, dt, ctx->d_eq);
   HIPCHK(ctx, hipGetLastError());
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  HIPCHK(ctx, hipMemcpy(c, D.counters, sizeof c, hipMemcpyDeviceToHost));
+  std::vector<int> cv;
+  r = read_status(ctx, &id, 1, cv);
+  if (r != CHP_OK) return r;
+  int c[C_COUNT];
+  memcpy(c, cv.data(), sizeof c);
   if (c[C_STATUS]) {
     int st = c[C_STATUS];
     c[C_STATUS] = 0;
@@ -1781,29 +1795,24 @@ static int solve_t(chp_ctx* ctx, uint32_t id, const chp_equation* eqs, uint32_t 
   if (r != CHP_OK) return r;
   r = upload_list(ctx, {(int)id});
   if (r != CHP_OK) return r;
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  if (n) HIPCHK(ctx, hipMemcpy(ctx->d_eq, eqs, n * sizeof(chp_equation), hipMemcpyHostToDevice));
-  const DevWorld<R>* dw = (const DevWorld<R>*)ctx->d_worlds;
-  const int bl = ctx->levels_block, bg = ctx->solve_block, nbig = S.nb > SMALL_NB ? 1 : 0;
   hipStream_t st = ctx->stream;
-  k_solve_rows<R><<<1, 256, 0, st>>>(dw, (int)id, ctx->d_eq, (int)n, dt);
-  const int lcap = levels_lds_cap(nbig, S.nb, ctx->max_lds);
-  k_levels<R><<<1, bl, lds_levels(bl, lcap), st>>>(dw, ctx->d_list, nbig, 1, lcap, 1);
+  if (n) HIPCHK(ctx, hipMemcpyAsync(ctx->d_eq, eqs, n * sizeof(chp_equation), hipMemcpyHostToDevice, st));
+  const DevWorld<R>* dw = (const DevWorld<R>*)ctx->d_worlds;
+  const int bl = ctx->levels_block, bg = ctx->solve_block, rb = ((int)n + 63) / 64;
+  k_solve_bodies<R><<<(S.nb + 255) / 256, 256, 0, st>>>(dw, (int)id, (int)n);
+  if (n) k_solve_rows<R><<<rb, 64, 0, st>>>(dw, (int)id, ctx->d_eq, (int)n, dt);
+  launch_levels<R>(dw, ctx->d_list, 1, ctx->gsg, S.nb, ctx->max_lds, bl, st);
+  if (n) k_solve_records<R><<<rb, 64, 0, st>>>(dw, (int)id, (int)n);
   if (self) launch_gs<R, true>(dw, ctx->d_list, 1, ctx->gsg, S.nb, ctx->max_lds, bg, 1, st);
   else launch_gs<R>(dw, ctx->d_list, 1, ctx->gsg, S.nb, ctx->max_lds, bg, 1, st);
-  k_solve_finish<R><<<1, 256, 0, st>>>(dw, (int)id);
+  double* d_mult = mult && n ? (double*)ctx->d_eq : nullptr;   // the equations have been read
+  k_solve_finish<R><<<(std::max(S.nb, (int)n) + 255) / 256, 256, 0, st>>>(dw, (int)id, (int)n, dt, d_mult);
   HIPCHK(ctx, hipGetLastError());
-  HIPCHK(ctx, hipStreamSynchronize(st));
-  DevWorld<R>& D = dev_of<R>(S);
-  int c[C_COUNT];
-  HIPCHK(ctx, hipMemcpy(c, D.counters, sizeof c, hipMemcpyDeviceToHost));
+  std::vector<int> c;
+  r = read_status(ctx, &id, 1, c);
+  if (r != CHP_OK) return r;
   *iters = c[C_ITERS];
-  if (mult && n) {
-    std::vector<RowRec<R>> rr(n);
-    HIPCHK(ctx, hipMemcpy(rr.data(), D.rows, n * sizeof(RowRec<R>), hipMemcpyDeviceToHost));
-    R invDt = (R)1 / (R)dt;   // gs_solver.dart:124-129
-    for (uint32_t k = 0; k < n; k++) mult[k] = (double)(rr[k].lambda * invDt);
-  }
+  if (d_mult) HIPCHK(ctx, hipMemcpy(mult, d_mult, n * sizeof(double), hipMemcpyDeviceToHost));
   return CHP_OK;
 }
 

@@ -221,13 +221,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 }
 template <typename R, int CLS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_narrow_wave(const DevWorld<R>* __restrict__ worlds, const int2* __restrict__ q,
-                                                     int* __restrict__ bounds, double dt) {
+                                                     int* __restrict__ bounds, double dt, int clip_cap) {
   __shared__ f3 ws[4][NPCtx<R, true>::WS_F3];            // one LDS workspace per wave
   __shared__ ContactRec<R> loc[4][WAVE_KMAX];             // and one contact buffer
   constexpr unsigned kinds = CLS == NP_WHC ? (NK_CC | NK_HC | NK_SH) : NK_ALL;
   st_narrow_wave<R, kinds>(worlds, q + bounds[CLS], bounds[CLS + 1] - bounds[CLS], bounds + NP_NCLS + 1 + (CLS - NP_WHC),
                            (R)dt, ws[threadIdx.x >> 6],
-                           loc[threadIdx.x >> 6], WAVE_KMAX);
+                           loc[threadIdx.x >> 6], WAVE_KMAX, clip_cap);
 }
 
 
@@ -267,64 +267,6 @@ __global__ __launch_bounds__(64) void k_joint_rows(const DevWorld<R>* __restrict
     constraint_rows<R, MODE>(W, c, F + C + W.c_row_off[c], (R)dt, keep != 0);
 }
 
-// The level stage runs one large world per workgroup (the first nbig entries of the list) and one
-// small world (at most SMALL_NB bodies) per wave, blockDim / 64 of them per workgroup.
-constexpr int SMALL_NB = 128;        // bodies of a world run by one wave
-constexpr int LS_SMALL = 1024;                  // level histogram of a small world in LDS
-constexpr int LS_LEVELS = 4096;                 // of a large world's level stage
-
-// bodies of a large world whose level walk keeps each body's last level in LDS (4 bytes per
-// body): up to the largest large world of the launch, at most what a workgroup's LDS holds beside
-// the level histogram and the static arrays (4 KiB kept free)
-constexpr int BIG_NB_LDS_MIN = 512;
-static int levels_lds_cap(int nbig, int max_nb, size_t max_lds) {
-  const int most = (int)((max_lds - 4096 - (size_t)LS_LEVELS * sizeof(int)) / sizeof(int));
-  return nbig ? std::max(BIG_NB_LDS_MIN, std::min(max_nb, most)) : BIG_NB_LDS_MIN;
-}
-
-// dynamic LDS of k_levels for a workgroup of bd threads (big_cap: as levels_lds_cap)
-static size_t lds_levels(int bd, int big_cap) {
-  size_t big = (size_t)(big_cap + LS_LEVELS) * sizeof(int), small = (size_t)(SMALL_NB + LS_SMALL) * sizeof(int);
-  return std::max(big, (bd / 64) * small);
-}
-
-// the world of this workgroup (large) or of this wave (small); -1: none / quarantined
-template <typename R>
-__device__ __forceinline__ int group_world(const DevWorld<R>* worlds, const int* list, int nbig, int n, int* sh,
-                                           int& wave) {
-  if ((int)blockIdx.x < nbig) {
-    wave = -1;
-    int id = list[blockIdx.x];
-    return block_bcast(worlds[id].counters[C_STATUS], sh) != 0 ? -1 : id;
-  }
-  wave = threadIdx.x >> 6;
-  int idx = nbig + ((int)blockIdx.x - nbig) * (int)(blockDim.x >> 6) + wave;
-  if (idx >= n) return -1;
-  int id = list[idx];
-  return worlds[id].counters[C_STATUS] != 0 ? -1 : id;
-}
-
-// GS dependency levels of the step's rows and the level-ordered GS records
-template <typename R>
-__global__ __launch_bounds__(256) void k_levels(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                int nbig, int n, int big_cap, int gather) {
-  __shared__ int sh[256];
-  extern __shared__ int lds_i[];
-  int wave;
-  int id = group_world(worlds, list, nbig, n, sh, wave);
-  if (id < 0) return;
-  const DevWorld<R>& W = worlds[id];
-  if (W.solver_kind == CHP_SOLVER_SPLIT) return;   // k_split_prep orders its rows
-  if (wave < 0) {
-    if (W.nb <= big_cap) st_levels<R, GBlock, true>(W, GBlock(), sh, lds_i, lds_i + big_cap, LS_LEVELS, gather != 0);
-    else st_levels<R, GBlock, false>(W, GBlock(), sh, W.tmp, nullptr, 0, gather != 0);
-  } else {
-    int* base = lds_i + wave * (SMALL_NB + LS_SMALL);
-    if (W.nb <= SMALL_NB) st_levels<R, GWave, true>(W, GWave(), sh, base, base + SMALL_NB, LS_SMALL, gather != 0);
-    else st_levels<R, GWave, false>(W, GWave(), sh, W.tmp, nullptr, 0, gather != 0);
-  }
-}
-
 // GS sweeps.  Worlds of at most GS_WAVE_NB bodies run one per wave, four to a workgroup; those of
 // at most GS_SUB_MAX_NB one per workgroup of four waves, all of them in one launch; larger ones
 // one per workgroup of their own launch.  vlambda / wlambda and the step tables live in LDS where
@@ -352,6 +294,75 @@ static size_t lds_gs_sub(const GsSegs& g) {
 static int big_lds_cap(int max_nb, size_t max_lds) {
   const int most = (int)((max_lds - 4096 - GS_SS_BIG * sizeof(int)) / (8 * sizeof(float))) - 1;
   return std::min(max_nb, most);
+}
+
+// GS dependency levels of the step's rows.  Worlds of at most GS_WAVE_NB bodies run one per wave,
+// those of at most GS_SUB_MAX_NB one per workgroup, all in one launch and with their rows in LDS
+// (up to LV_ROWS_WAVE / LV_ROWS_SUB rows: 217 bodies 31 -> 12 us, half a batch of 2048 worlds
+// 149 -> 51 us); larger ones in a workgroup of 1024 threads of their own launch, whose passes over
+// the rows are what takes the time (16,384 bodies 2.35 -> 0.75 ms, with 256 threads before).
+constexpr int SMALL_NB = GS_WAVE_NB;
+constexpr int LV_ROWS_WAVE = 1024, LV_ROWS_SUB = 6144, LV_TB_SUB = 512, LV_TB_BIG = 1024;
+constexpr int LV_HIST_BIG = 4096;                // of a large world's level histogram in LDS
+static size_t lds_levels_sub(const GsSegs& g, int bd) {
+  return std::max(g.nb_sub ? lev_lds_bytes(g.nb_sub, LV_TB_SUB, LV_ROWS_SUB) : 0,
+                  g.nb_wave ? (bd / 64) * lev_lds_bytes(GS_WAVE_NB, GS_WAVE_NB, LV_ROWS_WAVE) : 0);
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_levels_sub(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                    GsSegs g, int n) {
+  __shared__ int sh[8];
+  extern __shared__ float4 lds_f4[];
+  const int b = (int)blockIdx.x, nsub = g.wave - g.blk;
+  if (b < nsub) {
+    const DevWorld<R>& W = worlds[list[g.blk + b]];
+    if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;   // k_split_prep orders its rows
+    if (W.counters[C_ROWS] <= LV_ROWS_SUB) {
+      st_levels_lds<R>(W, GBlock(), sh, lds_f4, g.nb_sub, LV_TB_SUB, LV_ROWS_SUB);
+    } else {
+      unsigned long long* tb = (unsigned long long*)lds_f4;
+      int* last = (int*)(tb + LV_TB_SUB);
+      st_levels<R, GBlock, true>(W, GBlock(), sh, last, last + g.nb_sub, LV_ROWS_SUB, tb, LV_TB_SUB);
+    }
+  } else {
+    const int wave = uni((int)(threadIdx.x >> 6)), idx = g.wave + (b - nsub) * (int)(blockDim.x >> 6) + wave;
+    if (idx >= n) return;
+    const DevWorld<R>& W = worlds[list[idx]];
+    if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;
+    char* lds = (char*)lds_f4 + wave * lev_lds_bytes(GS_WAVE_NB, GS_WAVE_NB, LV_ROWS_WAVE);
+    if (W.counters[C_ROWS] <= LV_ROWS_WAVE) {
+      st_levels_lds<R>(W, GWave(), sh, lds, GS_WAVE_NB, GS_WAVE_NB, LV_ROWS_WAVE);
+    } else {
+      unsigned long long* tb = (unsigned long long*)lds;
+      int* last = (int*)(tb + GS_WAVE_NB);
+      st_levels<R, GWave, true>(W, GWave(), sh, last, last + GS_WAVE_NB, LV_ROWS_WAVE, tb, GS_WAVE_NB);
+    }
+  }
+}
+// big_cap: bodies whose last levels fit in the launch's LDS
+template <typename R>
+__global__ __launch_bounds__(1024) void k_levels(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
+                                                 int big_cap) {
+  __shared__ int sh[32];
+  extern __shared__ float4 lds_f4[];
+  const DevWorld<R>& W = worlds[list[blockIdx.x]];
+  if (W.counters[C_STATUS] != 0 || W.solver_kind == CHP_SOLVER_SPLIT) return;
+  unsigned long long* tb = (unsigned long long*)lds_f4;
+  int* hist = (int*)(tb + LV_TB_BIG);
+  if (W.nb <= big_cap) st_levels<R, GBlock, true>(W, GBlock(), sh, hist + LV_HIST_BIG, hist, LV_HIST_BIG, tb, LV_TB_BIG);
+  else st_levels<R, GBlock, false>(W, GBlock(), sh, W.tmp, hist, LV_HIST_BIG, tb, LV_TB_BIG);
+}
+// bd: workgroup size of k_levels_sub, and a quarter of k_levels'
+template <typename R>
+static void launch_levels(const DevWorld<R>* dw, const int* d_list, int n, const GsSegs& g, int max_nb, size_t max_lds, int bd,
+                          hipStream_t st) {
+  if (g.blk) {
+    const size_t fixed = LV_TB_BIG * 8 + LV_HIST_BIG * 4;
+    const int cap = std::min(max_nb, (int)((max_lds - 4096 - fixed) / sizeof(int)));
+    k_levels<R><<<g.blk, 4 * bd, fixed + (size_t)cap * sizeof(int), st>>>(dw, d_list, cap);
+  }
+  const int nsub = (g.wave - g.blk) + (n - g.wave + bd / 64 - 1) / (bd / 64);
+  if (nsub) k_levels_sub<R><<<nsub, bd, lds_levels_sub(g, bd), st>>>(dw, d_list, g, n);
 }
 
 template <typename R, int NW, bool SELF>
@@ -513,26 +524,79 @@ __global__ __launch_bounds__(256) void k_post(const DevWorld<R>* __restrict__ wo
   st_post(W, dt);
 }
 
-// Narrowphase slot: contacts for the pairs in the world's pair slab, then the equations
+// Narrowphase slot: the given pairs (in the pair slab) queued by class, for the class kernels; then
+// the offsets of their equations, then the equations.  One workgroup of one world each, the
+// equations over the grid.
 template <typename R>
-__global__ __launch_bounds__(64) void k_np_slot(const DevWorld<R>* __restrict__ worlds, int id, double dt,
-                                                chp_equation* __restrict__ out, int cap) {
-  __shared__ int sh[64];
-  __shared__ f3 cb[2 * CLIP_THREAD * 64];
+__global__ __launch_bounds__(1024) void k_np_queue(const DevWorld<R>* __restrict__ worlds, int id, int np,
+                                                   int* __restrict__ qw, int2* __restrict__ q) {
+  __shared__ int sh[16];
   const DevWorld<R>& W = worlds[id];
-  st_narrow(W, (R)dt, cb);
-  st_equations(W, (R)dt, out, cap, sh);
+  if (threadIdx.x == 0) {
+    W.counters[C_PAIRS] = np;
+    W.counters[C_STATUS] = W.counters[C_STAGING] = W.counters[C_ROWS] = 0;
+  }
+  __threadfence_block();
+  __syncthreads();
+  st_narrow_count(W, qw, 0, sh);
+  __threadfence();
+  __syncthreads();
+  queue_bounds(qw);
+  st_narrow_place(W, id, qw, 0, q, sh);
+  __syncthreads();
+  if (threadIdx.x < 2 * NP_NCLS) qw[QW_TOT + threadIdx.x] = 0;
+}
+template <typename R>
+__global__ __launch_bounds__(1024) void k_np_offsets(const DevWorld<R>* __restrict__ worlds, int id, int cap) {
+  __shared__ int sh[32];
+  st_equation_offsets(worlds[id], cap, sh);
+}
+template <typename R>
+__global__ __launch_bounds__(64) void k_np_equations(const DevWorld<R>* __restrict__ worlds, int id, double dt,
+                                                     chp_equation* __restrict__ out) {
+  const DevWorld<R>& W = worlds[id];
+  if (W.counters[C_STATUS] & WS_ROWS) return;
+  const int P = W.counters[C_PAIRS];
+  for (int p = (int)(blockIdx.x * blockDim.x + threadIdx.x); p < P; p += (int)(gridDim.x * blockDim.x))
+    pair_equations(W, p, (R)dt, out);
 }
 
-// Solver slot: rows from given equations; then k_levels / k_gs; then the velocity update
+// Solver slot: the bodies' solve masses, rows from the given equations, their GS records at the
+// schedule's positions (after k_levels), and at the end the velocity update and the multipliers
+// (Equation.multiplier = lambda / dt, gs_solver.dart:124-129)
 template <typename R>
-__global__ __launch_bounds__(256) void k_solve_rows(const DevWorld<R>* __restrict__ worlds, int id,
-                                                    const chp_equation* __restrict__ eq, int n, double dt) {
-  st_solve_rows(worlds[id], eq, n, (R)dt);
+__global__ __launch_bounds__(256) void k_solve_bodies(const DevWorld<R>* __restrict__ worlds, int id, int n) {
+  const DevWorld<R>& W = worlds[id];
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < W.nb) solve_body(W, i);
+  if (i == 0) { W.counters[C_ROWS] = n; W.counters[C_STATUS] = 0; }
 }
 template <typename R>
-__global__ __launch_bounds__(256) void k_solve_finish(const DevWorld<R>* __restrict__ worlds, int id) {
-  st_solve_finish(worlds[id]);
+__global__ __launch_bounds__(64) void k_solve_rows(const DevWorld<R>* __restrict__ worlds, int id,
+                                                   const chp_equation* __restrict__ eq, int n, double dt) {
+  const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (r < n) solve_row(worlds[id], eq, r, (R)dt);
+}
+template <typename R>
+__global__ __launch_bounds__(64) void k_solve_records(const DevWorld<R>* __restrict__ worlds, int id, int n) {
+  const DevWorld<R>& W = worlds[id];
+  const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (r >= n) return;
+  const int k = W.rpos[r];
+  const int2 x = ((const int2*)W.row_ab)[r];
+  gs_store<R>((typename GsWord<R>::T*)W.gsr, k, W.rows[r], (unsigned)x.x, (unsigned)x.y);
+  W.glam[2 * (size_t)k] = (R)0;
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_solve_finish(const DevWorld<R>* __restrict__ worlds, int id, int n, double dt,
+                                                      double* __restrict__ mult) {
+  const DevWorld<R>& W = worlds[id];
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < W.nb && n > 0) solve_finish_body(W, i);
+  if (i < n && mult) {
+    const R invDt = (R)1 / (R)dt;
+    mult[i] = (double)(W.glam[2 * (size_t)W.rpos[i]] * invDt);
+  }
 }
 
 // the kernels instantiated in chp_narrow_kernels.hip
@@ -544,7 +608,7 @@ __global__ __launch_bounds__(256) void k_solve_finish(const DevWorld<R>* __restr
   X void k_narrow_cls<R, NP_PC>(const DevWorld<R>*, const int2*, const int*, double);                  \
   X void k_narrow_cls<R, NP_CC>(const DevWorld<R>*, const int2*, const int*, double);                  \
   X void k_narrow_cls<R, NP_OTHER>(const DevWorld<R>*, const int2*, const int*, double);               \
-  X void k_narrow_wave<R, NP_WHC>(const DevWorld<R>*, const int2*, int*, double);                      \
-  X void k_narrow_wave<R, NP_WAVE>(const DevWorld<R>*, const int2*, int*, double);
+  X void k_narrow_wave<R, NP_WHC>(const DevWorld<R>*, const int2*, int*, double, int);                      \
+  X void k_narrow_wave<R, NP_WAVE>(const DevWorld<R>*, const int2*, int*, double, int);
 
 }  // namespace chp

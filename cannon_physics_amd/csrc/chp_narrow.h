@@ -116,6 +116,7 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   // thread path: this lane's two clip polygons in an LDS area of 2 * CLIP_THREAD * 64 f3 shared
   // by the wave (element k of polygon b at cb[(b * CLIP_THREAD + k) * 64 + lane])
   f3* cb = nullptr;
+  int clip_cap = CLIP_WAVE;   // WAVE: points a clip polygon may have
   CHP_HD NPCtx(const DevWorld<R>& w, R dt_, Sink<R, WAVE>* s, f3* ws_ = nullptr, f3* cb_ = nullptr)
       : W(w), dt(dt_), cm(0), sink(s), status(0), ws(ws_), cb(cb_) {}
 
@@ -586,7 +587,7 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     if constexpr (WAVE) {
       bufA = Poly{ws + WS_CA, 1};
       bufB = Poly{ws + WS_CB, 1};
-      cap = CLIP_WAVE;
+      cap = clip_cap;
     } else {
       const int lane = (int)(threadIdx.x & 63);
       bufA = Poly{cb + lane, 64};

@@ -711,15 +711,6 @@ __device__ __forceinline__ void narrow_pair(const DevWorld<R>& W, int p, R dt, f
   pair_counts(W, p, n, base);
 }
 
-// narrowphase of one world on one workgroup, one thread per pair (the slot entry point)
-// (cb: 2 * CLIP_THREAD * 64 f3 of LDS per wave of the workgroup)
-template <typename R> __device__ void st_narrow(const DevWorld<R>& W, R dt, f3* cb) {
-  int P = W.counters[C_PAIRS];
-  f3* wcb = cb + (threadIdx.x >> 6) * (2 * CLIP_THREAD * 64);
-  for (int p = threadIdx.x; p < P; p += blockDim.x) narrow_pair(W, p, dt, wcb);
-  __syncthreads();
-}
-
 // The batched narrowphase sorts the pairs of every listed world by resolver class, so that a
 // wave of the thread kernel runs one resolver on neighbouring data.  Classes 0..NP_WAVE-1 run one
 // pair per thread, class NP_WAVE one pair per wave.
@@ -840,10 +831,11 @@ constexpr int WAVE_KMAX = 64;
 // falling clear of a heightfield against one resting on a dozen pillars).  Waves numbered at or
 // beyond the queue's length leave at once, so an empty or short queue costs few atomics on the
 // one counter.
-// (ws: the wave's LDS workspace; loc: its LDS contact buffer of kmax records)
+// (ws: the wave's LDS workspace; loc: its LDS contact buffer of kmax records; clip_cap: points a
+// clip polygon may have)
 template <typename R, unsigned KINDS>
 __device__ void st_narrow_wave(const DevWorld<R>* worlds, const int2* queue, int cnt, int* ticket, R dt, f3* ws,
-                               ContactRec<R>* loc, int kmax) {
+                               ContactRec<R>* loc, int kmax, int clip_cap) {
   const int lane = threadIdx.x & 63;
   if ((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6) >= cnt) return;
   for (;;) {
@@ -857,6 +849,7 @@ __device__ void st_narrow_wave(const DevWorld<R>* worlds, const int2* queue, int
     const int bi = W.pair_i[p], bj = W.pair_j[p];
     Sink<R, true> s{loc, kmax, 0, 0};
     NPCtx<R, true, KINDS> ctx(W, dt, &s, ws);
+    ctx.clip_cap = clip_cap;
     ctx.pair(bi, bj);
     int n = s.n, base = 0;
     if (lane == 0) {
@@ -870,6 +863,7 @@ __device__ void st_narrow_wave(const DevWorld<R>* worlds, const int2* queue, int
     } else if (n > kmax) {  // more contacts than the local buffer: run the pair again into the slab
       Sink<R, true> s2{W.contacts + base, n, 0, 0};
       NPCtx<R, true, KINDS> ctx2(W, dt, &s2, ws);
+      ctx2.clip_cap = clip_cap;
       ctx2.pair(bi, bj);
     } else if (lane == 0) {
       for (int k = 0; k < n; k++) W.contacts[base + k] = loc[k];
@@ -1124,16 +1118,23 @@ template <typename R> __device__ bool st_rowscan(const DevWorld<R>& W, int* sh) 
 // Narrowphase slot with World's row assembly, world_class.dart:539-635, without the joints):
 // friction equations then contact equations in generation order, disabled and trigger ones
 // dropped, the body-material restitution override applied.  B and 1/C are the solver's.
-template <typename R> __device__ void st_equations(const DevWorld<R>& W, R h, chp_equation* out, int cap, int* sh) {
-  int P = W.counters[C_PAIRS];
-  int F = array_exscan(W.pf_cnt, P, sh);
-  int C = array_exscan(W.pc_off, P, sh);
-  if (F + C > cap) {
-    if (threadIdx.x == 0) { W.counters[C_ROWS] = F + C; ws_fail(W.counters, WS_ROWS); }
-    return;
+// The offsets of a pair's equations (one workgroup); false when they outgrow the buffer.
+template <typename R> __device__ bool st_equation_offsets(const DevWorld<R>& W, int cap, int* sh) {
+  const int P = W.counters[C_PAIRS];
+  const int F = array_exscan(W.pf_cnt, P, sh);
+  const int C = array_exscan(W.pc_off, P, sh);
+  const bool ok = F + C <= cap;
+  if (threadIdx.x == 0) {
+    W.counters[C_ROWS] = F + C;
+    if (ok) { W.counters[C_FROWS] = F; W.counters[C_CROWS] = C; }
+    else ws_fail(W.counters, WS_ROWS);
   }
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
-    int fo = W.pf_cnt[p], co = F + W.pc_off[p];
+  return ok;
+}
+// the equations of pair p
+template <typename R> __device__ void pair_equations(const DevWorld<R>& W, int p, R h, chp_equation* out) {
+  {
+    int fo = W.pf_cnt[p], co = W.counters[C_FROWS] + W.pc_off[p];
     for (int k = 0; k < W.pc_cnt[p]; k++) {
       const ContactRec<R>& c = W.contacts[W.pc_base[p] + k];
       if (!(c.flags & 1)) continue;
@@ -1168,58 +1169,47 @@ template <typename R> __device__ void st_equations(const DevWorld<R>& W, R h, ch
       out[co++] = e;
     }
   }
-  if (threadIdx.x == 0) { W.counters[C_ROWS] = F + C; W.counters[C_FROWS] = F; W.counters[C_CROWS] = C; }
-  __syncthreads();
 }
 
 // GSSolver.solve's set-up for given equations (gs_solver.dart:27-75): solve masses, the applied
 // force as the body holds it (the World added gravity before calling the solver), and each
 // equation's B and 1/C from its own spook parameters.
-template <typename R> __device__ void st_solve_rows(const DevWorld<R>& W, const chp_equation* eq, int n, R h) {
-  for (int i = threadIdx.x; i < W.nb; i += blockDim.x) {
-    S3<R>(W.feff, i, F3<R>(W.force, i));
-    const bool kin = solve_massless(W, i);
-    W.ims[i] = kin ? (R)0 : W.inv_mass[i];
-    for (int k = 0; k < 9; k++) W.iiws[9 * i + k] = kin ? 0.f : W.iiw[9 * i + k];
-    S3<R>(W.vl, i, mk3(0.f, 0.f, 0.f));
-    S3<R>(W.wl, i, mk3(0.f, 0.f, 0.f));
-  }
-  __syncthreads();
-  // one pass per equation kind, each with a single row builder: the builders are not merged
-  // into one body
+template <typename R> __device__ __forceinline__ void solve_body(const DevWorld<R>& W, int i) {
+  S3<R>(W.feff, i, F3<R>(W.force, i));
+  const bool kin = solve_massless(W, i);
+  W.ims[i] = kin ? (R)0 : W.inv_mass[i];
+  for (int k = 0; k < 9; k++) W.iiws[9 * i + k] = kin ? 0.f : W.iiw[9 * i + k];
+  S3<R>(W.vl, i, mk3(0.f, 0.f, 0.f));
+  S3<R>(W.wl, i, mk3(0.f, 0.f, 0.f));
+}
+// row r.  One pass per equation kind, each with a single row builder: the builders are not merged
+// into one body
+template <typename R> __device__ void solve_row(const DevWorld<R>& W, const chp_equation* eq, int r, R h) {
+  const chp_equation& e = eq[r];
+  const f3 ri = mk3(e.ri[0], e.ri[1], e.ri[2]), rj = mk3(e.rj[0], e.rj[1], e.rj[2]);
+  const f3 nn = mk3(e.n[0], e.n[1], e.n[2]);
+  const R sa_ = (R)e.a, sb_ = (R)e.b, se = (R)e.eps, mn = (R)e.min_force, mx = (R)e.max_force;
+  const int ps = e.kind == CHP_ROW_CONTACT ? 0 : e.kind == CHP_ROW_FRICTION ? 1 : e.kind == CHP_ROW_MOTOR ? 3 : 2;
   for (int pass = 0; pass < 4; pass++) {
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-      const chp_equation& e = eq[r];
-      const f3 ri = mk3(e.ri[0], e.ri[1], e.ri[2]), rj = mk3(e.rj[0], e.rj[1], e.rj[2]);
-      const f3 nn = mk3(e.n[0], e.n[1], e.n[2]);
-      const R sa_ = (R)e.a, sb_ = (R)e.b, se = (R)e.eps, mn = (R)e.min_force, mx = (R)e.max_force;
-      const int ps = e.kind == CHP_ROW_CONTACT ? 0 : e.kind == CHP_ROW_FRICTION ? 1 : e.kind == CHP_ROW_MOTOR ? 3 : 2;
-      if (ps != pass) continue;
-      const RowBody<R> A = row_body(W, e.body_i), B = row_body(W, e.body_j);
-      if (pass == 0)
-        contact_row(W, r, A, B, ri, rj, nn, (R)e.restitution, sa_, sb_, se, h, mn, mx);
-      else if (pass == 1)
-        friction_row(W, r, A, B, ri, rj, nn, sb_, se, h, mn, mx);
-      else if (pass == 2 && (e.kind == CHP_ROW_ROTATIONAL || e.kind == CHP_ROW_CONE))
-        rot_row(W, r, e.kind, A, B, ri, rj, (R)e.angle_cos, h, mn, mx, sa_, sb_, se);
-      else if (pass == 3)
-        motor_row(W, r, A, B, ri, rj, (R)e.target_velocity, h, mn, mx, sb_, se);
-    }
-    __syncthreads();
+    if (ps != pass) continue;
+    const RowBody<R> A = row_body(W, e.body_i), B = row_body(W, e.body_j);
+    if (pass == 0)
+      contact_row(W, r, A, B, ri, rj, nn, (R)e.restitution, sa_, sb_, se, h, mn, mx);
+    else if (pass == 1)
+      friction_row(W, r, A, B, ri, rj, nn, sb_, se, h, mn, mx);
+    else if (pass == 2 && (e.kind == CHP_ROW_ROTATIONAL || e.kind == CHP_ROW_CONE))
+      rot_row(W, r, e.kind, A, B, ri, rj, (R)e.angle_cos, h, mn, mx, sa_, sb_, se);
+    else if (pass == 3)
+      motor_row(W, r, A, B, ri, rj, (R)e.target_velocity, h, mn, mx, sb_, se);
   }
-  if (threadIdx.x == 0) { W.counters[C_ROWS] = n; W.counters[C_STATUS] = 0; }
-  __syncthreads();
 }
 
 // end of GSSolver.solve: v += vlambda * linearFactor, w += wlambda * angularFactor
 // (gs_solver.dart:111-121)
-template <typename R> __device__ void st_solve_finish(const DevWorld<R>& W) {
-  if (W.counters[C_ROWS] == 0) return;
-  for (int i = threadIdx.x; i < W.nb; i += blockDim.x) {
-    f3 v = F3<R>(W.vel, i), w = F3<R>(W.avel, i);
-    S3<R>(W.vel, i, add3<R>(v, mul3<R>(F3<R>(W.vl, i), F3<R>(W.lin_factor, i))));
-    S3<R>(W.avel, i, add3<R>(w, mul3<R>(F3<R>(W.wl, i), F3<R>(W.ang_factor, i))));
-  }
+template <typename R> __device__ __forceinline__ void solve_finish_body(const DevWorld<R>& W, int i) {
+  f3 v = F3<R>(W.vel, i), w = F3<R>(W.avel, i);
+  S3<R>(W.vel, i, add3<R>(v, mul3<R>(F3<R>(W.vl, i), F3<R>(W.lin_factor, i))));
+  S3<R>(W.avel, i, add3<R>(w, mul3<R>(F3<R>(W.wl, i), F3<R>(W.ang_factor, i))));
 }
 
 // ---- Gauss-Seidel -------------------------------------------------------------------------------
@@ -1388,27 +1378,198 @@ template <typename R> __device__ __forceinline__ void gs_store(typename GsWord<R
 // Levels.  Consecutive rows on the same two bodies (a contact's two friction rows, the rows of
 // one box-box contact patch, a joint's rows) form a run; inside a run each row depends on the
 // one before it and on nothing later outside the run, so the run's rows take consecutive levels
-// from the run's start level.  One wave walks the runs in solver order, 64 at a time: a run
-// starts one level above the last level of each of its dynamic bodies (last[], from the earlier
-// chunks); inside the chunk lane j's start is final once lanes 0..j-1 are done, so a uniform
-// pass over j hands its end level to the later lanes sharing a body.  Rows without a dynamic body
-// depend on nothing and take level 0.  The rows are then counting-sorted by level and gathered
-// into the GS records in level order.
+// from the run's start level.  One wave walks the runs in solver order, 64 at a time (lev_walk).
+// Rows without a dynamic body depend on nothing and take level 0.  The rows are then
+// counting-sorted by level; the row builders write the GS records at the positions rpos this
+// leaves.
+
+// The walk of NR runs by the wave of lanes tid < 64.  A run starts one level above the last level
+// of each of its dynamic bodies: last[] for the earlier chunks of 64, and inside the chunk the
+// latest earlier lane on each body, whose end it waits for (the runs of a body have increasing
+// levels, so its latest is its highest).  Those lanes come from a table of 64-bit lane masks by
+// body, and the ends are relaxed until they stand; a chunk that is one long chain (joints) is
+// finished by the pass over the lanes instead.  A relaxation round is two lane permutes where the
+// pass is sixty-three dependent broadcasts, and a chunk of a pile takes three or four rounds.
+//   tb: TB masks (a power of two; bodies share an entry when nb > TB), all zero and left so
+//   rs(q): first and one past the last row of run q; put(q, v): the start level, -1 when not dynamic
+// Returns the lane's part of the number of levels.
+template <bool LDS, class RS, class PUT>
+__device__ __forceinline__ int lev_walk(const int2* ab, int NR, int nb, int* last, unsigned long long* tb, int TB, RS rs, PUT put) {
+  const int lane = (int)threadIdx.x & 63;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const bool shared = nb > TB;
+  int lmax = 0;
+  auto load_rs = [&](int c) { return c + lane < NR ? rs(c + lane) : make_int2(0, 0); };
+  auto load_ab = [&](int2 r, int c) { return c + lane < NR ? ab[r.x] : make_int2(0, 0); };
+  int2 rs_next = load_rs(0), x_next = load_ab(rs_next, 0), rs_after = load_rs(64);
+  for (int c0 = 0; c0 < NR; c0 += 64) {
+    const int q = c0 + lane;
+    const bool act = q < NR;
+    const int2 r = rs_next, x = x_next;
+    x_next = load_ab(rs_after, c0 + 64);   // the runs' bounds are loaded two chunks ahead, their bodies one
+    rs_next = rs_after;
+    rs_after = load_rs(c0 + 128);
+    const bool da = act && (x.x & GS_DYN), db = act && (x.y & GS_DYN), dyn = da || db;
+    const int a = x.x & GS_IDX, b = x.y & GS_IDX, len = r.y - r.x;
+    const int ka = da ? a : -1 - 2 * lane, kb = db ? b : -2 - 2 * lane;   // non-dynamic keys never match
+    const int span = dyn ? len : 1;   // levels a run occupies
+    unsigned long long *ta = tb + (a & (TB - 1)), *tbb = tb + (b & (TB - 1));
+    if (da) atomicOr(ta, 1ull << lane);
+    if (db) atomicOr(tbb, 1ull << lane);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local");
+    unsigned long long ma = da ? *ta & below : 0ull, mb = db ? *tbb & below : 0ull;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local");
+    if (da) *ta = 0ull;
+    if (db) *tbb = 0ull;
+    int lev = 0;
+    if constexpr (LDS) {
+      if (da) lev = max(lev, last[a] + 1);
+      if (db) lev = max(lev, last[b] + 1);
+    } else {
+      if (da) lev = max(lev, atomicAdd(&last[a], 0) + 1);
+      if (db) lev = max(lev, atomicAdd(&last[b], 0) + 1);
+    }
+    if (shared) {   // drop the lanes of other bodies from the top of the masks
+      for (;;) {
+        const int ja = ma ? 63 - __clzll(ma) : lane, jb = mb ? 63 - __clzll(mb) : lane;
+        const int aa = __shfl(ka, ja, 64), ab_ = __shfl(kb, ja, 64), ba = __shfl(ka, jb, 64), bb = __shfl(kb, jb, 64);
+        const bool xa = ma != 0 && aa != a && ab_ != a, xb = mb != 0 && ba != b && bb != b;
+        if (xa) ma ^= 1ull << ja;
+        if (xb) mb ^= 1ull << jb;
+        if (!__any(xa || xb)) break;
+      }
+    }
+    const int pa = ma ? 63 - __clzll(ma) : lane, pb = mb ? 63 - __clzll(mb) : lane;
+    bool more = __any(pa != lane || pb != lane);
+    for (int round = 0; more && round < 12; round++) {
+      const int e = lev + span;   // one past the run's last level
+      const int ea = __shfl(e, pa, 64), eb = __shfl(e, pb, 64);
+      int nl = lev;
+      if (pa != lane) nl = max(nl, ea);
+      if (pb != lane) nl = max(nl, eb);
+      more = __any(nl != lev);
+      lev = nl;
+    }
+    if (more) {
+      const int n = uni(min(64, NR - c0));
+      int endv = lev + span - 1;
+      for (int j = 0; j < n - 1; j++) {   // branch-free: exec-mask switches would sit on the chain
+        const int kaj = __builtin_amdgcn_readlane(ka, j), kbj = __builtin_amdgcn_readlane(kb, j);
+        const int endj = __builtin_amdgcn_readlane(endv, j);
+        const int hit = (int)(lane > j) & ((int)(ka == kaj) | (int)(ka == kbj) | (int)(kb == kaj) | (int)(kb == kbj));
+        lev = max(lev, hit ? endj + 1 : 0);
+        endv = lev + span - 1;
+      }
+    }
+    // the chain through a body has increasing levels: the chunk's last run on it wins
+    if (da) atomicMax(&last[a], lev + span - 1);
+    if (db) atomicMax(&last[b], lev + span - 1);
+    if (act) {
+      put(q, dyn ? lev : -1);
+      lmax = max(lmax, lev + span);
+    }
+  }
+  return lmax;
+}
+
+// Rows in LDS: a world of at most `cap` rows keeps its runs, levels and histogram there, so that
+// the passes around the walk cost LDS accesses instead of a memory round trip each.
+//   lds: lev_lds_bytes(nbcap, TB, cap)
+__host__ __device__ constexpr size_t lev_lds_bytes(int nbcap, int TB, int cap) {
+  return ((((size_t)TB + cap / 64) * 8 + (size_t)nbcap * 4 + ((size_t)cap + 2) * 6) + 15) & ~(size_t)15;
+}
+template <typename R, typename G>
+__device__ __forceinline__ void st_levels_lds(const DevWorld<R>& W, const G& g, int* sh, void* lds, int nbcap, int TB, int cap) {
+  const int E = uni(W.counters[C_ROWS]), nb = W.nb, tid = g.tid, bd = g.n;
+  const int lane = tid & 63, wv = uni(tid >> 6), nw = bd >> 6;
+  const int2* ab = (const int2*)W.row_ab;
+  unsigned long long* tb = (unsigned long long*)lds;
+  unsigned long long* first = tb + TB;   // bit r: row r starts a run
+  int* last = (int*)(first + cap / 64);
+  unsigned short* rid = (unsigned short*)(last + nbcap);   // run of each row, then its level
+  unsigned short* rst = rid + cap + 2;                     // first row of each run (+ E at the end)
+  unsigned short* rlv = rst + cap + 2;                     // start level of each run, 0xffff: not dynamic
+  int* hist = (int*)rst;                                   // after the levels: cap + 2 ints in their place
+  for (int k = tid; k < TB; k += bd) tb[k] = 0ull;
+  for (int b = tid; b < nb; b += bd) last[b] = -1;
+  // runs: a row starts one when its body pair differs from the previous row's.  Each wave takes a
+  // contiguous stretch of 64-row words
+  const int words = (E + 63) >> 6, per = (words + nw - 1) / nw, w0 = min(words, wv * per), w1 = min(words, w0 + per);
+  int c = 0;
+  for (int w = w0; w < w1; w++) {
+    const int r = 64 * w + lane;
+    const int2 x = r < E ? ab[r] : make_int2(0, 0), y = r > 0 && r < E ? ab[r - 1] : make_int2(-1, -1);
+    const unsigned long long m = __ballot(r < E && (r == 0 || x.x != y.x || x.y != y.y));
+    if (lane == 0) first[w] = m;
+    c += __popcll(m);
+  }
+  int before = 0, NR = c;
+  if (nw > 1) {
+    if (lane == 0) sh[wv] = c;
+    g.lds_sync();
+    NR = 0;
+    for (int u = 0; u < nw; u++) {
+      const int t = sh[u];
+      before += u < wv ? t : 0;
+      NR += t;
+    }
+  }
+  g.lds_sync();
+  NR = uni(NR);
+  for (int w = w0; w < w1; w++) {
+    const int r = 64 * w + lane;
+    const unsigned long long m = first[w];
+    const int id = before + __popcll(m & (~0ull >> (63 - lane))) - 1;
+    if (r < E) {
+      rid[r] = (unsigned short)id;
+      if ((m >> lane) & 1ull) rst[id] = (unsigned short)r;
+    }
+    before += __popcll(m);
+  }
+  if (tid == 0) rst[NR] = (unsigned short)E;
+  g.lds_sync();
+  int lmax = 0;
+  if (tid < 64)
+    lmax = lev_walk<true>(ab, NR, nb, last, tb, TB, [&](int q) { return make_int2(rst[q], rst[q + 1]); },
+                          [&](int q, int v) { rlv[q] = (unsigned short)v; });
+  const int L = uni(g.imax(lmax, sh));   // (a barrier for the whole group)
+  g.lds_sync();
+  for (int r = tid; r < E; r += bd) {
+    const int id = rid[r], l0 = rlv[id];
+    rid[r] = (unsigned short)(l0 == 0xffff ? 0 : l0 + (r - (int)rst[id]));
+  }
+  g.lds_sync();
+  // counting sort by level; the order inside a level is free (its rows are independent)
+  for (int l = tid; l <= L; l += bd) hist[l] = 0;
+  g.lds_sync();
+  for (int r = tid; r < E; r += bd) atomicAdd(&hist[rid[r]], 1);
+  g.lds_sync();
+  g.exscan(hist, L + 1, sh);
+  for (int l = tid; l <= L; l += bd) W.lvl_start[l] = hist[l];
+  g.lds_sync();
+  for (int r = tid; r < E; r += bd) {
+    const int k = atomicAdd(&hist[rid[r]], 1);
+    W.sched[k] = r;
+    W.rpos[r] = k;
+  }
+  if (tid == 0) W.counters[C_LEVELS] = L;
+}
+
+// Rows in memory (any number of them).
 //   last: nb ints (LDS when LDS, else the world's global scratch, read with atomics so that
 //         each chunk sees the previous chunk's values)
-//   hist: hist_cap ints of LDS for the level histogram (global scratch when L + 1 > hist_cap
-//         or not LDS)
-// gather: the rows are in their row records and go to GS records here; else the row builders
-// write the GS records afterwards, at the positions rpos this leaves
+//   hist: hist_cap ints of LDS for the level histogram (global scratch when L + 1 > hist_cap)
+//   tb: TB lane masks in LDS
 template <typename R, typename G, bool LDS>
 __device__ __forceinline__ void st_levels(const DevWorld<R>& W, const G& g, int* sh, int* last, int* hist, int hist_cap,
-                                          bool gather) {
+                                          unsigned long long* tb, int TB) {
   const int E = uni(W.counters[C_ROWS]), nb = W.nb;
   const int tid = g.tid, bd = g.n;
   const int2* ab = (const int2*)W.row_ab;
   int* runid = W.level;     // run of each row, then its level
   int* rstart = W.rpos;     // first row of each run (+ E at the end), until the sort below
   int* rlev = W.sched;      // start level of each run, until the sort below
+  for (int k = tid; k < TB; k += bd) tb[k] = 0ull;
   for (int b = tid; b < nb; b += bd) last[b] = -1;
   // The passes over the rows take LU rows per thread per turn, loading all of them before any
   // store: each turn then waits for one round of loads rather than one per row.
@@ -1454,62 +1615,11 @@ __device__ __forceinline__ void st_levels(const DevWorld<R>& W, const G& g, int*
   if (tid == 0) rstart[NR] = E;
   g.sync();
   int lmax = 0;
-  if (tid < 64) {
-    const int lane = tid;
-    // the runs' bounds and body pairs are loaded ahead (bounds two chunks, pairs one chunk), so
-    // the walk does not wait for them
-    auto load_rs = [&](int c) { const int q = c + lane; return q < NR ? make_int2(rstart[q], rstart[q + 1]) : make_int2(0, 0); };
-    auto load_ab = [&](int2 rs, int c) { return c + lane < NR ? ab[rs.x] : make_int2(0, 0); };
-    int2 rs_next = load_rs(0);
-    int2 x_next = load_ab(rs_next, 0);
-    int2 rs_after = load_rs(64);
-    for (int c0 = 0; c0 < NR; c0 += 64) {
-      const int q = c0 + lane;
-      const bool act = q < NR;
-      const int2 rs = rs_next, x = x_next;
-      x_next = load_ab(rs_after, c0 + 64);
-      rs_next = rs_after;
-      rs_after = load_rs(c0 + 128);
-      int a = 0, b = 0, len = 0;
-      bool da = false, db = false;
-      if (act) {
-        len = rs.y - rs.x;
-        da = x.x & GS_DYN;
-        db = x.y & GS_DYN;
-        a = x.x & GS_IDX;
-        b = x.y & GS_IDX;
-      }
-      const bool dyn = da || db;
-      const int ka = da ? a : -1 - 2 * lane, kb = db ? b : -2 - 2 * lane;   // non-dynamic keys never match
-      const int span = dyn ? len : 1;   // levels a run occupies
-      int lev = 0;
-      if constexpr (LDS) {
-        if (da) lev = max(lev, last[a] + 1);
-        if (db) lev = max(lev, last[b] + 1);
-      } else {
-        if (da) lev = max(lev, atomicAdd(&last[a], 0) + 1);
-        if (db) lev = max(lev, atomicAdd(&last[b], 0) + 1);
-      }
-      const int n = uni(min(64, NR - c0));
-      // branch-free: a branch per lane costs exec-mask switches on this loop's dependent chain
-      int endv = lev + span - 1;
-      for (int j = 0; j < n - 1; j++) {
-        const int kaj = __builtin_amdgcn_readlane(ka, j), kbj = __builtin_amdgcn_readlane(kb, j);
-        const int endj = __builtin_amdgcn_readlane(endv, j);
-        const int hit = (int)(lane > j) & ((int)(ka == kaj) | (int)(ka == kbj) | (int)(kb == kaj) | (int)(kb == kbj));
-        lev = max(lev, hit ? endj + 1 : 0);
-        endv = lev + span - 1;
-      }
-      // the chain through a body has increasing levels: the chunk's last run on it wins
-      if (da) atomicMax(&last[a], lev + span - 1);
-      if (db) atomicMax(&last[b], lev + span - 1);
-      if (act) {
-        rlev[q] = dyn ? lev : -1;
-        lmax = max(lmax, lev + span);
-      }
-    }
-  }
+  if (tid < 64)
+    lmax = lev_walk<LDS>(ab, NR, nb, last, tb, TB, [&](int q) { return make_int2(rstart[q], rstart[q + 1]); },
+                         [&](int q, int v) { rlev[q] = v; });
   const int L = uni(g.imax(lmax, sh));
+  g.sync();
   for (int r0 = tid; r0 < E; r0 += LU * bd) {
     int id[LU], l0[LU], rs[LU];
 #pragma unroll
@@ -1557,21 +1667,9 @@ __device__ __forceinline__ void st_levels(const DevWorld<R>& W, const G& g, int*
     }
     g.sync();
   };
-  if (LDS && L + 1 <= hist_cap) sort(hist);
+  if (L + 1 <= hist_cap) sort(hist);
   else sort(W.last_level);
-  if (gather) {
-    typedef typename GsWord<R>::T T;
-    T* gsr = (T*)W.gsr;
-    for (int k = tid; k < E; k += bd) {
-      int r = W.sched[k];
-      RowRec<R> o = W.rows[r];
-      int2 x = ab[r];
-      gs_store<R>(gsr, k, o, (unsigned)x.x, (unsigned)x.y);
-      W.glam[2 * k] = (R)0;
-    }
-  }
   if (tid == 0) W.counters[C_LEVELS] = L;
-  g.sync();
 }
 
 // GSSolver.solve iterations (gs_solver.dart:76-108) + Equation.computeGWlambda /
