@@ -292,7 +292,7 @@ struct chp_ctx {
     bool keep = false;
     double dt = 0;
     const void *dq = nullptr, *dqcls = nullptr, *dlist = nullptr, *dworlds = nullptr, *dbig = nullptr;
-    std::array<int, 10> big{};
+    std::array<int, 11> big{};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
   } sg;
@@ -880,6 +880,7 @@ static int upload_list(chp_ctx* ctx, const std::vector<int>& list) {
   }
   std::vector<int> spans, tiles, bigw;
   int max_tiles = 1;
+  size_t bodies = 0;
   ctx->n_sap = 0;
   ctx->n_sleep = 0;
   ctx->n_events = 0;
@@ -894,6 +895,7 @@ static int upload_list(chp_ctx* ctx, const std::vector<int>& list) {
     if (S.split) ctx->n_split++;
     if (S.joints) ctx->n_joints++;
     ctx->classes |= step_classes(S);
+    bodies += (size_t)S.nb;
     if (S.nb < BP_BIG) continue;
     bigw.push_back((int)li);
     for (int s0 = 0; s0 < S.nb; s0 += BP_SPAN) { spans.push_back((int)li); spans.push_back(s0); }
@@ -1529,7 +1531,7 @@ template <typename R> static int broadphase_t(chp_ctx* ctx, uint32_t id, int32_t
   r = upload_list(ctx, {(int)id});
   if (r != CHP_OK) return r;
   if (ctx->worlds[id].nb >= BP_BIG) launch_big_bp<R>(ctx_view(ctx), ctx->stream);
-  else launch_bp<R>((const DevWorld<R>*)ctx->d_worlds, ctx->d_list, 1, ctx->worlds[id].nb, ctx->n_sap, nullptr, ctx->stream);
+  else launch_bp<R>((const DevWorld<R>*)ctx->d_worlds, ctx->d_list, 1, ctx->worlds[id].nb, ctx->n_sap, nullptr, 0, ctx->stream);
   HIPCHK(ctx, hipGetLastError());
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   DevWorld<R>& D = dev_of<R>(ctx->worlds[id]);
@@ -1637,19 +1639,20 @@ static int raycast_t(chp_ctx* ctx, uint32_t id, const chp_ray* rays, uint32_t nr
   if (r != CHP_OK) return r;
   *n = 0;
   if (nr == 0) return CHP_OK;
-  // staging: rays | probe (int4) | counts | offsets | hits
+  if (nr > 0x7fffffffu / 2) return fail(ctx, CHP_E_CAPACITY, "too many rays in one call");
+  // staging: rays | probe (int4) | counts, then offsets | one hit per ray | hits
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   const size_t o_rays = 0, o_probe = up(nr * sizeof(chp_ray)), o_cnt = up(o_probe + nr * sizeof(int4)),
-               o_off = up(o_cnt + nr * sizeof(int)), o_hits = up(o_off + nr * sizeof(int));
+               o_one = up(o_cnt + nr * sizeof(int)), o_hits = up(o_one + nr * sizeof(chp_ray_hit));
   const size_t hcap = std::max<uint32_t>(cap, 1);
   r = ensure_qbuf(ctx, o_hits + hcap * sizeof(chp_ray_hit));
+  if (r == CHP_OK) r = ensure_stage(ctx, sizeof(long long));
   if (r != CHP_OK) return r;
   char* q = (char*)ctx->d_qbuf;
   chp_ray* d_rays = (chp_ray*)(q + o_rays);
   int4* d_probe = (int4*)(q + o_probe);
   int* d_cnt = (int*)(q + o_cnt);
-  int* d_off = (int*)(q + o_off);
-  chp_ray_hit* d_hits = (chp_ray_hit*)(q + o_hits);
+  chp_ray_hit *d_one = (chp_ray_hit*)(q + o_one), *d_hits = (chp_ray_hit*)(q + o_hits);
   hipStream_t st = ctx->stream;
   const DevWorld<R>* dw = (const DevWorld<R>*)ctx->d_worlds;
   DevWorld<R>& D = dev_of<R>(S);
@@ -1662,7 +1665,7 @@ static int raycast_t(chp_ctx* ctx, uint32_t id, const chp_ray* rays, uint32_t nr
     HIPCHK(ctx, hipMemcpyAsync(rs, D.ray_state, sizeof rs, hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
     if (!rs[RS_SET]) {
-      k_rays<R, 0><<<blocks, 64, 0, st>>>(dw, (int)id, d_rays, (int)nr, d_probe, nullptr, nullptr, nullptr);
+      k_rays<R, 0><<<blocks, 256, 0, st>>>(dw, (int)id, d_rays, (int)nr, d_probe, nullptr, nullptr, nullptr, nullptr, 0);
       HIPCHK(ctx, hipGetLastError());
       std::vector<int4> pr(nr);
       HIPCHK(ctx, hipMemcpyAsync(pr.data(), d_probe, nr * sizeof(int4), hipMemcpyDeviceToHost, st));
@@ -1675,21 +1678,19 @@ static int raycast_t(chp_ctx* ctx, uint32_t id, const chp_ray* rays, uint32_t nr
         }
     }
   }
-  k_rays<R, 1><<<blocks, 64, 0, st>>>(dw, (int)id, d_rays, (int)nr, nullptr, d_cnt, nullptr, nullptr);
+  bool any_all = false;
+  for (uint32_t k = 0; k < nr && !any_all; k++) any_all = rays[k].mode == CHP_RAY_ALL;
+  long long* h_total = (long long*)ctx->h_stage;   // pinned: the scan writes it
+  k_rays<R, 1><<<blocks, 256, 0, st>>>(dw, (int)id, d_rays, (int)nr, nullptr, d_cnt, nullptr, d_one, nullptr, 0);
+  k_ray_scan<<<1, 1024, 0, st>>>(d_cnt, (int)nr, h_total);
+  k_ray_hits<<<(nr + 255) / 256, 256, 0, st>>>(d_rays, (int)nr, d_cnt, h_total, d_one, d_hits, icap);
+  if (any_all) k_rays<R, 2><<<blocks, 256, 0, st>>>(dw, (int)id, d_rays, (int)nr, nullptr, nullptr, d_cnt, nullptr, d_hits, icap);
   HIPCHK(ctx, hipGetLastError());
-  std::vector<int> cnt(nr), off(nr);
-  HIPCHK(ctx, hipMemcpyAsync(cnt.data(), d_cnt, nr * sizeof(int), hipMemcpyDeviceToHost, st));
   HIPCHK(ctx, hipStreamSynchronize(st));
-  size_t total = 0;
-  for (uint32_t k = 0; k < nr; k++) { off[k] = (int)total; total += (size_t)cnt[k]; }
+  const size_t total = (size_t)*h_total;
   *n = (uint32_t)std::min<size_t>(total, UINT32_MAX);
   if (total > cap) return fail(ctx, CHP_E_CAPACITY, "hit buffer too small: need " + std::to_string(total));
-  if (total == 0) return CHP_OK;
-  HIPCHK(ctx, hipMemcpyAsync(d_off, off.data(), nr * sizeof(int), hipMemcpyHostToDevice, st));
-  k_rays<R, 2><<<blocks, 64, 0, st>>>(dw, (int)id, d_rays, (int)nr, nullptr, nullptr, d_off, d_hits);
-  HIPCHK(ctx, hipGetLastError());
-  HIPCHK(ctx, hipMemcpyAsync(hits, d_hits, total * sizeof(chp_ray_hit), hipMemcpyDeviceToHost, st));
-  HIPCHK(ctx, hipStreamSynchronize(st));
+  if (total) HIPCHK(ctx, hipMemcpy(hits, d_hits, total * sizeof(chp_ray_hit), hipMemcpyDeviceToHost));
   return CHP_OK;
 }
 

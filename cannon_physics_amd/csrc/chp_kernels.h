@@ -462,10 +462,40 @@ __global__ __launch_bounds__(1024) void k_aabb_query(const DevWorld<R>* __restri
   if (threadIdx.x == 0) *total = carry;
 }
 template <typename R, int PASS>
-__global__ __launch_bounds__(64) void k_rays(const DevWorld<R>* __restrict__ worlds, int id, const chp_ray* __restrict__ rays,
-                                             int nr, int4* __restrict__ probe, int* __restrict__ cnt,
-                                             const int* __restrict__ off, chp_ray_hit* __restrict__ out) {
-  st_rays<R, PASS>(worlds[id], rays, nr, probe, cnt, off, out);
+__global__ __launch_bounds__(256) void k_rays(const DevWorld<R>* __restrict__ worlds, int id, const chp_ray* __restrict__ rays,
+                                              int nr, int4* __restrict__ probe, int* __restrict__ cnt,
+                                              const int* __restrict__ off, chp_ray_hit* __restrict__ one,
+                                              chp_ray_hit* __restrict__ out, int cap) {
+  __shared__ int list[4][RAY_LIST];
+  const int wave = uni((int)(threadIdx.x >> 6));
+  for (int r = (int)blockIdx.x * 4 + wave; r < nr; r += (int)gridDim.x * 4) {
+    if (PASS == 2 && rays[r].mode != CHP_RAY_ALL) continue;
+    wave_ray<R, PASS>(worlds[id], rays[r], r, list[wave], probe, cnt, off, one, out, cap);
+  }
+}
+// the rays' counts become offsets, with their total
+static __global__ __launch_bounds__(1024) void k_ray_scan(int* __restrict__ cnt, int nr, long long* __restrict__ total) {
+  __shared__ int sh[32];
+  __shared__ long long big[16];
+  long long s = 0;   // the offsets are ints: a total beyond them is told apart here
+  for (int r = (int)threadIdx.x; r < nr; r += 1024) s += cnt[r];
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((threadIdx.x & 63) == 0) big[threadIdx.x >> 6] = s;
+  __syncthreads();
+  s = 0;
+  for (int w = 0; w < 16; w++) s += big[w];
+  if (threadIdx.x == 0) *total = s;
+  if (s <= 0x7fffffffLL) array_exscan(cnt, nr, sh);
+}
+// the one hit of each closest / any ray to its place
+static __global__ __launch_bounds__(256) void k_ray_hits(const chp_ray* __restrict__ rays, int nr, const int* __restrict__ off,
+                                                         const long long* __restrict__ total,
+                                                         const chp_ray_hit* __restrict__ one, chp_ray_hit* __restrict__ out,
+                                                         int cap) {
+  const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (r >= nr || rays[r].mode == CHP_RAY_ALL) return;
+  const long long end = r + 1 < nr ? (long long)off[r + 1] : *total;
+  if (off[r] < end && off[r] < cap) out[off[r]] = one[r];
 }
 
 // SplitSolver: ids, islands and row positions (after the rows' body pairs), then the islands'

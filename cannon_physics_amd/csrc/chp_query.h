@@ -1,9 +1,9 @@
 // chp_query.h -- queries against a world's device state between steps: Broadphase.aabbQuery
 // (naive_broadphase.dart:39-56, sap_broadphase.dart:239-261) and World.raycastClosest / Any / All
-// (world_class.dart:245-276, ray_class.dart).  One thread per ray; each ray walks the bodies in
-// the broadphase's query order (body order; SAP: the sorted axis list), as Ray.intersectWorld
-// does, so that the first hit (any), the kept hit among equal distances (closest) and the order
-// of all hits (all) are the reference's.
+// (world_class.dart:245-276, ray_class.dart).  One wave per ray; the hits are merged in the
+// broadphase's query order (body order; SAP: the sorted axis list), in which Ray.intersectWorld
+// walks the bodies, so that the first hit (any), the kept hit among equal distances (closest) and
+// the order of all hits (all) are the reference's.
 #pragma once
 #include "chp_stages.h"
 
@@ -248,52 +248,123 @@ template <typename R> struct RayRun {
     }
   }
 
-  // Ray.intersectWorld (:176-204): the bodies that aabbQuery returns for the ray's AABB, in
-  // its order
-  CHP_HD void world(const chp_ray& r) {
+  // Ray.intersectWorld's set-up (:176-204)
+  CHP_HD void begin(const chp_ray& r) {
     from = mk3(r.from[0], r.from[1], r.from[2]);
     to = mk3(r.to[0], r.to[1], r.to[2]);
     mode = r.mode; skip_back = r.skip_backfaces; check_cr = r.check_collision_response;
     group = r.collision_filter_group; mask = r.collision_filter_mask;
     dir = normalize3<R>(sub3<R>(to, from));
-    const f3 lo = mk3(fminf(to.x, from.x), fminf(to.y, from.y), fminf(to.z, from.z));
-    const f3 hi = mk3(fmaxf(to.x, from.x), fmaxf(to.y, from.y), fmaxf(to.z, from.z));
-    for (int k = 0; k < W.nb && !should_stop; k++) {
-      const int b = query_body(W, k);
-      if (!aabb_overlaps(F3<R>(W.aabb_lo, b), F3<R>(W.aabb_hi, b), lo, hi)) continue;
-      body(b);
-    }
   }
 };
 
-// one ray per thread.  PASS 0: the probe for the heightfield cell index (first call per ray,
-// into probe[r] = (called, x, y)); 1: count the hits per ray (closest / any: 0 or 1); 2: write
-// them from off[r]
+// One ray on one wave.  The lanes test 64 bodies' AABBs at a time against the ray's
+// (Ray.intersectWorld walks the bodies aabbQuery returns for it, in its order); the overlapping
+// bodies go, in that order, to a list in LDS, and each full list of 64 is intersected a body per
+// lane and the lanes' hits merged in list order.  Nearly every body fails the AABB test, so a ray
+// costs a coalesced pass over the AABBs and one or two rounds of intersections; with a thread per
+// ray a wave of 64 rays paid for every body any of them came near (16,384 rays into 2,000 bodies:
+// 947 us to count and 1,110 us to write, now 163 us in all).
+// PASS 0: the probe for the heightfield cell index (first call per ray, into probe[r] = (called, x,
+// y)); 1: the hits per ray counted, and the one hit of a closest / any ray into one[r]; 2: an
+// all-mode ray's hits written from off[r], as far as cap reaches.
+constexpr int RAY_LIST = 128;
 template <typename R, int PASS>
-__device__ void st_rays(const DevWorld<R>& W, const chp_ray* rays, int nr, int4* probe, int* cnt, const int* off,
-                        chp_ray_hit* out) {
-  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < nr; r += gridDim.x * blockDim.x) {
-    RayRun<R> run(W);
-    run.ray_index = r;
-    run.probe = PASS == 0;
-    run.hx = W.ray_state[RS_X];
-    run.hy = W.ray_state[RS_Y];
-    if (PASS == 2 && rays[r].mode == CHP_RAY_ALL) run.out = out + off[r];
-    run.world(rays[r]);
-    if (PASS == 0) {
-      probe[r] = make_int4(run.probed ? 1 : 0, run.px, run.py, 0);
-      continue;
+__device__ void wave_ray(const DevWorld<R>& W, const chp_ray& ray, int r, int* list, int4* probe, int* cnt, const int* off,
+                         chp_ray_hit* one, chp_ray_hit* out, int cap) {
+  const int lane = (int)threadIdx.x & 63;
+  RayRun<R> base(W);
+  base.begin(ray);
+  base.ray_index = r;
+  base.probe = PASS == 0;
+  base.hx = W.ray_state[RS_X];
+  base.hy = W.ray_state[RS_Y];
+  const f3 lo = mk3(fminf(base.to.x, base.from.x), fminf(base.to.y, base.from.y), fminf(base.to.z, base.from.z));
+  const f3 hi = mk3(fmaxf(base.to.x, base.from.x), fmaxf(base.to.y, base.from.y), fmaxf(base.to.z, base.from.z));
+  const bool all = base.mode == CHP_RAY_ALL;
+  bool stop = false, has = false;
+  int n = 0, kept_body = -1, kept_shape = -1, face = -1;
+  f3 kn{}, kp{};
+  R kd = (R)-1;
+  // the first m bodies of the list, one per lane
+  auto intersect = [&](int m) {
+    RayRun<R> run = base;
+    if (lane < m) run.body(list[lane]);
+    if constexpr (PASS == 2) {
+      const int inc = wave_incl_scan(run.n), at = off[r] + n + inc - run.n;
+      if (run.n > 0 && at + run.n <= cap) {
+        RayRun<R> w = base;
+        w.out = out + at;
+        w.body(list[lane]);
+      }
+      n += __shfl(inc, 63, 64);
+      return;
     }
-    const int n = rays[r].mode == CHP_RAY_ALL ? run.n : (run.has_hit ? 1 : 0);
-    if (PASS == 1) {
-      cnt[r] = n;
-    } else if (rays[r].mode != CHP_RAY_ALL && run.has_hit) {
-      chp_ray_hit& h = out[off[r]];
-      h.ray = r; h.body = run.hbody; h.shape = W.si_shape[run.hshape]; h.face = run.face_last;
-      h.normal[0] = run.hn.x; h.normal[1] = run.hn.y; h.normal[2] = run.hn.z;
-      h.point[0] = run.hp.x; h.point[1] = run.hp.y; h.point[2] = run.hp.z;
-      h.distance = (double)run.hdist;
+    if (PASS == 0) {   // in order: the first heightfield call, or the hit that ends the walk before it
+      const unsigned long long pm = __ballot(run.probed), hm = base.mode == CHP_RAY_ANY ? __ballot(run.has_hit) : 0ull;
+      const int fp = pm ? __builtin_ctzll(pm) : 64, fh = hm ? __builtin_ctzll(hm) : 64;
+      if (fp < 64 && fp <= fh) {
+        base.px = __shfl(run.px, fp, 64);
+        base.py = __shfl(run.py, fp, 64);
+        base.probed = true;
+      }
+      stop = fp < 64 || fh < 64;
+      return;
     }
+    if (all) {
+      n += __shfl(wave_incl_scan(run.n), 63, 64);
+      return;
+    }
+    for (unsigned long long h = __ballot(run.has_hit); h; h &= h - 1) {
+      const int l = __builtin_ctzll(h);
+      const R d = __shfl(run.hdist, l, 64);
+      face = __shfl(run.face_last, l, 64);   // of the last intersection reported
+      if (d < kd || !has) {
+        has = true;
+        kd = d;
+        kept_body = __shfl(run.hbody, l, 64);
+        kept_shape = __shfl(run.hshape, l, 64);
+        kn = mk3(__shfl(run.hn.x, l, 64), __shfl(run.hn.y, l, 64), __shfl(run.hn.z, l, 64));
+        kp = mk3(__shfl(run.hp.x, l, 64), __shfl(run.hp.y, l, 64), __shfl(run.hp.z, l, 64));
+      }
+      if (base.mode != CHP_RAY_CLOSEST) {   // any: the first hit ends the walk
+        stop = true;
+        break;
+      }
+    }
+  };
+  int have = 0;
+  for (int k0 = 0; k0 < W.nb && !stop; k0 += 64) {
+    const int k = k0 + lane;
+    const int b = k < W.nb ? query_body(W, k) : 0;
+    const unsigned long long m = __ballot(k < W.nb && aabb_overlaps(F3<R>(W.aabb_lo, b), F3<R>(W.aabb_hi, b), lo, hi));
+    if (!m) continue;
+    if ((m >> lane) & 1ull) list[have + __popcll(m & ((1ull << lane) - 1ull))] = b;
+    have += __popcll(m);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local");
+    if (have >= 64) {
+      intersect(64);
+      have -= 64;
+      const int t = list[64 + lane];
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local");
+      list[lane] = t;
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local");
+    }
+  }
+  if (have > 0 && !stop) intersect(have);
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local");   // the next ray reuses the list
+  if (lane != 0 || PASS == 2) return;
+  if (PASS == 0) {
+    probe[r] = make_int4(base.probed ? 1 : 0, base.px, base.py, 0);
+    return;
+  }
+  cnt[r] = all ? n : (has ? 1 : 0);
+  if (!all && has) {
+    chp_ray_hit& h = one[r];
+    h.ray = r; h.body = kept_body; h.shape = W.si_shape[kept_shape]; h.face = face;
+    h.normal[0] = kn.x; h.normal[1] = kn.y; h.normal[2] = kn.z;
+    h.point[0] = kp.x; h.point[1] = kp.y; h.point[2] = kp.z;
+    h.distance = (double)kd;
   }
 }
 
