@@ -228,6 +228,7 @@ struct ListState {
   int big_nspans = 0, big_ntiles = 0, big_nw = 0, big_rounds = 0;
   int n_sap = 0, n_sleep = 0, n_events = 0, n_split = 0, n_joints = 0;
   unsigned classes = 0;
+  bool few = false;
   GsSegs gsg;
   int2* d_q = nullptr;
   size_t d_q_cap = 0;
@@ -266,6 +267,7 @@ struct chp_ctx {
   int n_split = 0;  // worlds in the current list with a SplitSolver
   int n_joints = 0; // worlds in the current list with constraints
   unsigned classes = 0;   // narrowphase classes the current list's pairs can have
+  bool few = false;       // the current list has at most NP_FEW_BODIES bodies
   GsSegs gsg;       // the GS kernels' segments of the current list
   ListState second;          // the second stream's list state (see ListState)
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -346,6 +348,7 @@ static void swap_lists(chp_ctx* ctx) {
   std::swap(ctx->n_split, o.n_split);
   std::swap(ctx->n_joints, o.n_joints);
   std::swap(ctx->classes, o.classes);
+  std::swap(ctx->few, o.few);
   std::swap(ctx->gsg, o.gsg);
   std::swap(ctx->d_q, o.d_q);
   std::swap(ctx->d_q_cap, o.d_q_cap);
@@ -848,6 +851,12 @@ static int ensure_queue(chp_ctx* ctx, const uint32_t* ids, uint32_t n) {
 // the narrowphase classes of a step of the world
 static unsigned step_classes(const WorldSlot& S) { return S.classes | (S.ev.mask && S.kinematic ? 1u << NP_WAVE : 0u); }
 
+// A list of at most this many bodies has so few pairs that a class's time is one pair's: its hull
+// pairs run on the wave path (one 300-body pile: 84 us a thread each, 40 us a wave each) and its
+// other thread classes in one launch (80 us one after the other, 31 us together).  Beyond it the
+// thread classes fill the chip and do the same pairs in fewer instructions.
+constexpr int NP_FEW_BODIES = 4096;
+
 // uploads the world list of the next launches and the large-world tables that go with it (the
 // host copies stay alive in the context until the next upload)
 static int upload_list(chp_ctx* ctx, const std::vector<int>& list) {
@@ -904,6 +913,7 @@ static int upload_list(chp_ctx* ctx, const std::vector<int>& list) {
       max_tiles = std::max(max_tiles, (S.nb + SAP_TILE - 1) / SAP_TILE);
     }
   }
+  ctx->few = bodies <= (size_t)NP_FEW_BODIES;
   ctx->big_nspans = (int)spans.size() / 2;
   ctx->big_ntiles = (int)tiles.size() / 2;
   ctx->big_nw = (int)bigw.size();
@@ -939,6 +949,7 @@ struct StepView {
   const int* big = nullptr;
   int nspans = 0, ntiles = 0, nw = 0, rounds = 0, n_sap = 0, n_sleep = 0, n_events = 0, n_split = 0, n_joints = 0;
   unsigned classes = 0;
+  bool few = false;
   GsSegs gsg;
   int2* q = nullptr;
   size_t qcap = 0;
@@ -959,6 +970,7 @@ static StepView ctx_view(const chp_ctx* ctx) {
   v.n_split = ctx->n_split;
   v.n_joints = ctx->n_joints;
   v.classes = ctx->classes;
+  v.few = ctx->few;
   v.gsg = ctx->gsg;
   v.q = ctx->d_q;
   v.qcap = ctx->d_q_cap;
@@ -970,10 +982,10 @@ static StepView ctx_view(const chp_ctx* ctx) {
 // world has a workgroup: of 1024 threads while the worlds leave CUs idle, else of 256, four to a
 // CU (one 300-body world 108 us with the 256 threads and FP64 tests it had before)
 template <typename R>
-static void launch_bp(const DevWorld<R>* dw, const int* list, int n, int max_nb, int n_sap, int* qw, hipStream_t st) {
+static void launch_bp(const DevWorld<R>* dw, const int* list, int n, int max_nb, int n_sap, int* qw, int wcc, hipStream_t st) {
   const int lds_nb = std::min(max_nb, BP_BIG - 1), bd = n <= 256 ? 1024 : 256;
-  if (n_sap < n) k_bp<R, false><<<n, bd, BpLds<R>::bytes(lds_nb, false), st>>>(dw, list, lds_nb, qw);
-  if (n_sap) k_bp<R, true><<<n, bd, BpLds<R>::bytes(lds_nb, true), st>>>(dw, list, lds_nb, qw);
+  if (n_sap < n) k_bp<R, false><<<n, bd, BpLds<R>::bytes(lds_nb, false), st>>>(dw, list, lds_nb, qw, wcc);
+  if (n_sap) k_bp<R, true><<<n, bd, BpLds<R>::bytes(lds_nb, true), st>>>(dw, list, lds_nb, qw, wcc);
 }
 
 // the broadphase of the large worlds of the list (after k_bp, which leaves them alone)
@@ -994,21 +1006,27 @@ template <typename R> static void launch_big_bp(const StepView& V, hipStream_t s
 
 // the resolver kernels over the placed queue: one kernel per class that the listed worlds can fill
 // (each compiles only its resolver), the thread classes up to 4 waves per SIMD.  qcap: a bound of
-// the queue's length; clip_cap: points a wave pair's clip polygon may have
-template <typename R> static void launch_classes(const StepView& V, double dt, int qcap, int clip_cap, hipStream_t st) {
+// the queue's length; clip_cap: points a wave pair's clip polygon may have; few: see above (the
+// queue was placed so)
+template <typename R> static void launch_classes(const StepView& V, double dt, int qcap, int clip_cap, bool few, hipStream_t st) {
   const DevWorld<R>* dw = (const DevWorld<R>*)V.worlds;
   int* bounds = V.qcls + QW_BOUNDS;
   const int blocks = (std::max(64, std::min(qcap, 256 * 4 * 4 * 64)) + 63) / 64;
   auto has = [&](int c) { return (V.classes >> c) & 1u; };
-  if (has(NP_SS)) k_narrow_cls<R, NP_SS><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-  if (has(NP_SP)) k_narrow_cls<R, NP_SP><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-  if (has(NP_SB)) k_narrow_cls<R, NP_SB><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-  if (has(NP_SC)) k_narrow_cls<R, NP_SC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-  if (has(NP_PC)) k_narrow_cls<R, NP_PC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-  if (has(NP_CC)) k_narrow_cls<R, NP_CC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  if (few) {
+    if (V.classes & (1u << NP_SS | 1u << NP_SP | 1u << NP_SB | 1u << NP_SC | 1u << NP_PC))
+      k_narrow_threads<R><<<std::min(blocks + 5, 2048), 64, 0, st>>>(dw, V.q, bounds, dt);
+  } else {
+    if (has(NP_SS)) k_narrow_cls<R, NP_SS><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_SP)) k_narrow_cls<R, NP_SP><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_SB)) k_narrow_cls<R, NP_SB><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_SC)) k_narrow_cls<R, NP_SC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_PC)) k_narrow_cls<R, NP_PC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+    if (has(NP_CC)) k_narrow_cls<R, NP_CC><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
+  }
   if (has(NP_OTHER)) k_narrow_cls<R, NP_OTHER><<<blocks, 64, 0, st>>>(dw, V.q, bounds, dt);
-  const int waves = std::max(1, std::min(qcap, 4096));
-  if (has(NP_WHC)) k_narrow_wave<R, NP_WHC><<<(waves + 3) / 4, 256, 0, st>>>(dw, V.q, bounds, dt, clip_cap);
+  const int waves = std::max(1, std::min(qcap, few ? 2048 : 4096));
+  if (has(NP_WHC) || (few && has(NP_CC))) k_narrow_wave<R, NP_WHC><<<(waves + 3) / 4, 256, 0, st>>>(dw, V.q, bounds, dt, clip_cap);
   // compound-body pairs are rare: a small grid, strided over however many there are
   if (has(NP_WAVE)) k_narrow_wave<R, NP_WAVE><<<32, 256, 0, st>>>(dw, V.q, bounds, dt, clip_cap);
 }
@@ -1028,17 +1046,18 @@ template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, in
   const DevWorld<R>* dw = (const DevWorld<R>*)V.worlds;
   const int* d_list = V.list;
   hipStream_t st = ctx->stream;
+  const int wcc = V.few ? 1 : 0;
   if (ev) HIPCHK(ctx, hipEventRecord(ev[0], st));
   {
-    launch_bp<R>(dw, d_list, n, max_nb, V.n_sap, V.qcls, st);
+    launch_bp<R>(dw, d_list, n, max_nb, V.n_sap, V.qcls, wcc, st);
     launch_big_bp<R>(V, st);
   }
   if (ev) HIPCHK(ctx, hipEventRecord(ev[1], st));
   {
-    if (V.nw) k_big_ncount<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls);
-    k_narrow<R><<<n, 256, 0, st>>>(dw, d_list, V.qcls, V.q);
-    if (V.nw) k_big_nplace<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls, V.q);
-    launch_classes<R>(V, dt, (int)V.qcap, CLIP_WAVE, st);
+    if (V.nw) k_big_ncount<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls, wcc);
+    k_narrow<R><<<n, 256, 0, st>>>(dw, d_list, V.qcls, V.q, wcc);
+    if (V.nw) k_big_nplace<R><<<V.nspans, 256, 0, st>>>(dw, d_list, V.spans(), V.qcls, V.q, wcc);
+    launch_classes<R>(V, dt, (int)V.qcap, CLIP_WAVE, wcc != 0, st);
     if (V.n_sleep) k_wake<R><<<n, 256, 0, st>>>(dw, d_list);
     if (V.n_events) k_events<R><<<n, 1024, 0, st>>>(dw, d_list, 0);
   }
@@ -1100,9 +1119,9 @@ static void drop_graph(chp_ctx* ctx) {
 }
 
 // what of the list decides which kernels a step launches, and their grids
-static std::array<int, 10> step_shape(const chp_ctx* ctx) {
+static std::array<int, 11> step_shape(const chp_ctx* ctx) {
   return {ctx->big_nspans, ctx->big_ntiles, ctx->big_nw, ctx->big_rounds, ctx->n_sap, ctx->n_sleep, ctx->n_events, ctx->n_split,
-          ctx->n_joints, (int)ctx->classes};
+          ctx->n_joints, (int)ctx->classes, ctx->few ? 1 : 0};
 }
 
 // the captured step for this configuration (captured anew when anything baked into its kernel
@@ -1375,6 +1394,7 @@ template <typename R> static int step_noalloc_t(chp_ctx* ctx, uint32_t id, doubl
   V.n_split = S.split ? 1 : 0;
   V.n_joints = S.joints ? 1 : 0;
   V.classes = step_classes(S);
+  V.few = S.nb <= NP_FEW_BODIES;
   V.gsg.blk = S.nb > GS_SUB_MAX_NB ? 1 : 0;
   V.gsg.wave = S.nb > GS_WAVE_NB ? 1 : 0;
   V.gsg.nb_sub = V.gsg.wave > V.gsg.blk ? S.nb : 0;
@@ -1733,8 +1753,8 @@ static int narrowphase_t(chp_ctx* ctx, uint32_t id, const int32_t* pi, const int
   // the slot's limit
   const StepView V = ctx_view(ctx);
   const DevWorld<R>* dw = (const DevWorld<R>*)V.worlds;
-  k_np_queue<R><<<1, 1024, 0, hs>>>(dw, (int)id, (int)np, V.qcls, V.q);
-  if (np) launch_classes<R>(V, dt, (int)np, CLIP_THREAD, hs);
+  k_np_queue<R><<<1, 1024, 0, hs>>>(dw, (int)id, (int)np, V.qcls, V.q, V.few);
+  if (np) launch_classes<R>(V, dt, (int)np, CLIP_THREAD, V.few, hs);
   k_np_offsets<R><<<1, 1024, 0, hs>>>(dw, (int)id, S.row_cap);
   if (np) k_np_equations<R><<<std::min<uint32_t>((np + 63) / 64, 16384), 64, 0, hs>>>(dw, (int)id, dt, ctx->d_eq);
   HIPCHK(ctx, hipGetLastError());

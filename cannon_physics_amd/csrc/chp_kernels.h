@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/cannon_hip.h"
 #include "chp_build.h"
@@ -28,7 +29,7 @@ namespace chp {
 // pairs alone).
 template <typename R, bool SAP>
 __global__ __launch_bounds__(1024) void k_bp(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                             int lds_nb, int* __restrict__ qw) {
+                                             int lds_nb, int* __restrict__ qw, int wcc) {
   __shared__ int sh[32];
   extern __shared__ float4 lds_bp[];
   const DevWorld<R>& W = worlds[list[blockIdx.x]];
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(1024) void k_bp(const DevWorld<R>* __restrict__ wor
   else ok = st_bp_naive(W, sh, L);
   if (!ok || !qw) return;
   st_filter(W);
-  st_narrow_count(W, qw, (int)blockIdx.x, sh);
+  st_narrow_count(W, qw, (int)blockIdx.x, wcc != 0, sh);
 }
 
 // large worlds (at least BP_BIG bodies): prestep, SAP sort and pair passes over the grid.
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(1024) void k_big_scan(const DevWorld<R>* __restrict
 // its K workers, worker k takes pairs k * 256 + t, stride K * 256.  Counts add into the class
 // totals; placement reserves each class range per workgroup.
 template <typename R>
-__device__ __forceinline__ void big_pair_classes(const DevWorld<R>& W, int2 sp, int* sh, bool mark_filtered) {
+__device__ __forceinline__ void big_pair_classes(const DevWorld<R>& W, int2 sp, int* sh, bool wcc, bool mark_filtered) {
   const int K = (W.nb + BP_SPAN - 1) / BP_SPAN, k = sp.y / BP_SPAN, P = W.counters[C_PAIRS];
   for (int p = k * 256 + (int)threadIdx.x; p < P; p += K * 256) {
     int bi = W.pair_i[p], bj = W.pair_j[p];
@@ -130,29 +131,29 @@ __device__ __forceinline__ void big_pair_classes(const DevWorld<R>& W, int2 sp, 
       if (mark_filtered) pair_counts(W, p, 0, 0);
       continue;
     }
-    atomicAdd(&sh[pair_class(W, bi, bj)], 1);
+    atomicAdd(&sh[pair_class(W, bi, bj, wcc)], 1);
   }
 }
 template <typename R>
 __global__ __launch_bounds__(256) void k_big_ncount(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                    const int2* __restrict__ spans, int* __restrict__ qw) {
+                                                    const int2* __restrict__ spans, int* __restrict__ qw, int wcc) {
   __shared__ int sh[NP_NCLS];
   CHP_SPAN_PROLOGUE(spans)
   if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = 0;
   __syncthreads();
-  big_pair_classes(W, sp, sh, true);
+  big_pair_classes(W, sp, sh, wcc != 0, true);
   __syncthreads();
   if (threadIdx.x < NP_NCLS && sh[threadIdx.x]) atomicAdd(&qw[QW_TOT + threadIdx.x], sh[threadIdx.x]);
 }
 template <typename R>
 __global__ __launch_bounds__(256) void k_big_nplace(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
                                                     const int2* __restrict__ spans, int* __restrict__ qw,
-                                                    int2* __restrict__ q) {
+                                                    int2* __restrict__ q, int wcc) {
   __shared__ int sh[NP_NCLS];
   CHP_SPAN_PROLOGUE(spans)
   if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = 0;
   __syncthreads();
-  big_pair_classes(W, sp, sh, false);
+  big_pair_classes(W, sp, sh, wcc != 0, false);
   __syncthreads();
   if (threadIdx.x < NP_NCLS)
     sh[threadIdx.x] = sh[threadIdx.x] ? queue_base(qw) + atomicAdd(&qw[QW_CUR + threadIdx.x], sh[threadIdx.x]) : 0;
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(256) void k_big_nplace(const DevWorld<R>* __restric
   for (int p = k * 256 + (int)threadIdx.x; p < P; p += K * 256) {
     int bi = W.pair_i[p], bj = W.pair_j[p];
     if (bi < 0) continue;
-    q[atomicAdd(&sh[pair_class(W, bi, bj)], 1)] = make_int2(wid, p);
+    q[atomicAdd(&sh[pair_class(W, bi, bj, wcc)], 1)] = make_int2(wid, p);
   }
 }
 
@@ -203,21 +204,27 @@ __global__ __launch_bounds__(64) void k_big_post(const DevWorld<R>* __restrict__
 // grid-wide over the whole batch.
 template <typename R>
 __global__ __launch_bounds__(256) void k_narrow(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
-                                                int* __restrict__ qw, int2* __restrict__ q) {
+                                                int* __restrict__ qw, int2* __restrict__ q, int wcc) {
   __shared__ int sh[64];
   if (blockIdx.x == 0) queue_bounds(qw);
   CHP_WORLD_PROLOGUE
   if (W.nb >= BP_BIG) return;  // k_big_nplace
-  st_narrow_place(W, list[blockIdx.x], qw, (int)blockIdx.x, q, sh);
+  st_narrow_place(W, list[blockIdx.x], qw, (int)blockIdx.x, wcc != 0, q, sh);
 }
-// classes whose resolvers clip polygons (convex-convex, and the mixed class) hold the clip
-// polygons of the block's 64 lanes in LDS
-constexpr bool cls_clips(int c) { return c == NP_CC || c == NP_OTHER; }
+// LDS of the 64 lanes of a thread class, in f3: the clip polygons of convex-convex (and the mixed
+// class), the side vectors of sphere-box
+constexpr int cls_lds(int c) { return c == NP_CC || c == NP_OTHER ? 2 * CLIP_THREAD * 64 : c == NP_SB ? 6 * 64 : 1; }
 template <typename R, int CLS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_narrow_cls(const DevWorld<R>* __restrict__ worlds, const int2* __restrict__ q,
                                                    const int* __restrict__ bounds, double dt) {
-  __shared__ f3 cb[cls_clips(CLS) ? 2 * CLIP_THREAD * 64 : 1];
+  __shared__ f3 cb[cls_lds(CLS)];
   st_narrow_class<R, CLS>(worlds, q, bounds, (R)dt, cb);
+}
+template <typename R>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_narrow_threads(const DevWorld<R>* __restrict__ worlds,
+                                                     const int2* __restrict__ q, const int* __restrict__ bounds, double dt) {
+  __shared__ f3 cb[cls_lds(NP_SB)];
+  st_narrow_threads<R>(worlds, q, bounds, (R)dt, cb);
 }
 template <typename R, int CLS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_narrow_wave(const DevWorld<R>* __restrict__ worlds, const int2* __restrict__ q,
@@ -559,7 +566,7 @@ __global__ __launch_bounds__(256) void k_post(const DevWorld<R>* __restrict__ wo
 // equations over the grid.
 template <typename R>
 __global__ __launch_bounds__(1024) void k_np_queue(const DevWorld<R>* __restrict__ worlds, int id, int np,
-                                                   int* __restrict__ qw, int2* __restrict__ q) {
+                                                   int* __restrict__ qw, int2* __restrict__ q, int wcc) {
   __shared__ int sh[16];
   const DevWorld<R>& W = worlds[id];
   if (threadIdx.x == 0) {
@@ -568,11 +575,11 @@ __global__ __launch_bounds__(1024) void k_np_queue(const DevWorld<R>* __restrict
   }
   __threadfence_block();
   __syncthreads();
-  st_narrow_count(W, qw, 0, sh);
+  st_narrow_count(W, qw, 0, wcc != 0, sh);
   __threadfence();
   __syncthreads();
   queue_bounds(qw);
-  st_narrow_place(W, id, qw, 0, q, sh);
+  st_narrow_place(W, id, qw, 0, wcc != 0, q, sh);
   __syncthreads();
   if (threadIdx.x < 2 * NP_NCLS) qw[QW_TOT + threadIdx.x] = 0;
 }
@@ -631,6 +638,7 @@ __global__ __launch_bounds__(256) void k_solve_finish(const DevWorld<R>* __restr
 
 // the kernels instantiated in chp_narrow_kernels.hip
 #define CHP_NARROW_KERNELS(X, R)                                                                       \
+  X void k_narrow_threads<R>(const DevWorld<R>*, const int2*, const int*, double);                     \
   X void k_narrow_cls<R, NP_SS>(const DevWorld<R>*, const int2*, const int*, double);                  \
   X void k_narrow_cls<R, NP_SP>(const DevWorld<R>*, const int2*, const int*, double);                  \
   X void k_narrow_cls<R, NP_SB>(const DevWorld<R>*, const int2*, const int*, double);                  \

@@ -3,6 +3,8 @@
 // per-body stages of the whole batch, and of large worlds, run over the grid.  The kernels in
 // chp_api.hip launch each stage once over every listed world.
 #pragma once
+#include <type_traits>
+
 #include "chp_narrow.h"
 
 namespace chp {
@@ -721,7 +723,9 @@ enum { NP_SS = 0, NP_SP, NP_SB, NP_SC, NP_SH, NP_PC, NP_CC, NP_OTHER, NP_WHC, NP
 // after the class bounds: one pair ticket per wave class (NP_WHC, NP_WAVE)
 constexpr int NP_NTICKET = 2;
 static_assert(NP_WAVE == NP_WHC + 1, "the tickets follow the wave classes' order");
-template <typename R> __device__ __forceinline__ int pair_class(const DevWorld<R>& W, int bi, int bj) {
+// wcc: hull pairs of the batch run on the wave path whatever their size (few of them: a pair takes a
+// wave a fraction of the time it takes a thread)
+template <typename R> __device__ __forceinline__ int pair_class(const DevWorld<R>& W, int bi, int bj, bool wcc) {
   if (W.ev_mask) {   // justTest pairs (narrow_phase.dart:665-668): their overlap probe is on the wave path
     const int ti = W.type[bi], tj = W.type[bj];
     if ((ti == CHP_BODY_KINEMATIC && tj != CHP_BODY_DYNAMIC) || (tj == CHP_BODY_KINEMATIC && ti != CHP_BODY_DYNAMIC))
@@ -741,7 +745,7 @@ template <typename R> __device__ __forceinline__ int pair_class(const DevWorld<R
   if (lo == CHP_SHAPE_PLANE && (hi == CHP_SHAPE_BOX || hi == CHP_SHAPE_CONVEX)) return NP_PC;
   if (lo == CHP_SHAPE_BOX || lo == CHP_SHAPE_CONVEX) {
     if (hi == CHP_SHAPE_HEIGHTFIELD) return NP_WHC;
-    if (hi == CHP_SHAPE_BOX || hi == CHP_SHAPE_CONVEX) return wave_pair(W, bi, bj) ? NP_WHC : NP_CC;
+    if (hi == CHP_SHAPE_BOX || hi == CHP_SHAPE_CONVEX) return wcc || wave_pair(W, bi, bj) ? NP_WHC : NP_CC;
   }
   return NP_OTHER;
 }
@@ -755,14 +759,14 @@ __host__ __device__ constexpr size_t queue_words(size_t nworlds) { return QW_COU
 
 // pass 1 (at the end of the broadphase): the pair counts of the workgroup's world by class, into
 // its words and the totals
-template <typename R> __device__ void st_narrow_count(const DevWorld<R>& W, int* qw, int idx, int* sh) {
+template <typename R> __device__ void st_narrow_count(const DevWorld<R>& W, int* qw, int idx, bool wcc, int* sh) {
   const int P = W.counters[C_PAIRS];
   if (threadIdx.x < NP_NCLS) sh[threadIdx.x] = 0;
   __syncthreads();
   for (int p = threadIdx.x; p < P; p += blockDim.x) {
     int bi = W.pair_i[p], bj = W.pair_j[p];
     if (bi < 0) { pair_counts(W, p, 0, 0); continue; }
-    atomicAdd(&sh[pair_class(W, bi, bj)], 1);
+    atomicAdd(&sh[pair_class(W, bi, bj, wcc)], 1);
   }
   __syncthreads();
   if (threadIdx.x < NP_NCLS) {
@@ -786,7 +790,7 @@ __device__ __forceinline__ void queue_bounds(int* qw) {
 // pass 2: the world's pairs into the queue, each class in a range reserved by its cursor (the
 // order of the worlds within a class is free)
 template <typename R>
-__device__ void st_narrow_place(const DevWorld<R>& W, int wid, int* qw, int idx, int2* q, int* sh) {
+__device__ void st_narrow_place(const DevWorld<R>& W, int wid, int* qw, int idx, bool wcc, int2* q, int* sh) {
   const int P = W.counters[C_PAIRS];
   if (threadIdx.x < NP_NCLS) {
     const int c = qw[QW_COUNTS + idx * NP_NCLS + threadIdx.x];
@@ -796,7 +800,7 @@ __device__ void st_narrow_place(const DevWorld<R>& W, int wid, int* qw, int idx,
   for (int p = threadIdx.x; p < P; p += blockDim.x) {
     int bi = W.pair_i[p], bj = W.pair_j[p];
     if (bi < 0) continue;
-    q[atomicAdd(&sh[pair_class(W, bi, bj)], 1)] = make_int2(wid, p);
+    q[atomicAdd(&sh[pair_class(W, bi, bj, wcc)], 1)] = make_int2(wid, p);
   }
 }
 
@@ -819,6 +823,30 @@ __device__ void st_narrow_class(const DevWorld<R>* worlds, const int2* q, const 
   for (int i = bounds[CLS] + g; i < b1; i += ng) {
     const int2 e = q[i];
     narrow_pair<R, cls_kinds(CLS), cls_kmax(CLS), cls_direct(CLS)>(worlds[e.x], e.y, dt, cb);
+  }
+}
+
+// the thread classes without clip polygons in one launch, 64 queue entries of one class at a time
+template <typename R>
+__device__ void st_narrow_threads(const DevWorld<R>* worlds, const int2* q, const int* bounds, R dt, f3* cb) {
+  constexpr int CLS[5] = {NP_SB, NP_SC, NP_PC, NP_SS, NP_SP};   // the longest first
+  int first[6];
+  first[0] = 0;
+#pragma unroll
+  for (int k = 0; k < 5; k++) first[k + 1] = first[k] + (bounds[CLS[k] + 1] - bounds[CLS[k]] + 63) / 64;
+  for (int b = (int)blockIdx.x; b < first[5]; b += (int)gridDim.x) {
+    auto run = [&](auto cls, int k) {
+      constexpr int C = decltype(cls)::value;
+      const int i = bounds[C] + 64 * (b - first[k]) + (int)threadIdx.x;
+      if (i >= bounds[C + 1]) return;
+      const int2 e = q[i];
+      narrow_pair<R, cls_kinds(C), cls_kmax(C), cls_direct(C)>(worlds[e.x], e.y, dt, cb);
+    };
+    if (b < first[1]) run(std::integral_constant<int, NP_SB>(), 0);
+    else if (b < first[2]) run(std::integral_constant<int, NP_SC>(), 1);
+    else if (b < first[3]) run(std::integral_constant<int, NP_PC>(), 2);
+    else if (b < first[4]) run(std::integral_constant<int, NP_SS>(), 3);
+    else run(std::integral_constant<int, NP_SP>(), 4);
   }
 }
 
