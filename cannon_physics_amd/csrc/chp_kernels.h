@@ -528,10 +528,11 @@ __global__ __launch_bounds__(256) void k_split_gs(const DevWorld<R>* __restrict_
 template <typename R>
 __global__ __launch_bounds__(1024) void k_events(const DevWorld<R>* __restrict__ worlds, const int* __restrict__ list,
                                                  int seed) {
-  __shared__ int sh[1024];
+  __shared__ int sh[32];
+  __shared__ u64 lk[EV_LDS];
   CHP_WORLD_PROLOGUE
   if (!W.ev_mask) return;
-  st_events(W, seed != 0, sh);
+  st_events(W, seed != 0, sh, lk);
 }
 
 // the wake-up pass after the narrowphase (worlds that may hold sleeping bodies)
