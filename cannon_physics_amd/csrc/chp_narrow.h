@@ -123,13 +123,14 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   // Narrowphase.createContactEquation (narrow_phase.dart:492-528) +
   // createFrictionEquationsFromContact (:530-586) + the World's body-material restitution
   // override (world_class.dart:556-560), folded into one record
-  CHP_HD void emit(int bi, int bj, SRef si, SRef sj, SRef rsi, SRef rsj, f3 ri, f3 rj, f3 ni) {
-    ContactRec<R> c;
-    c.bi = bi; c.bj = bj; c.cm = cm;
-    c.si = rsi.id; c.sj = rsj.id;   // createContactEquation: c.si = overrideShapeA ?? si
-    c.ri = ri; c.rj = rj; c.ni = ni;
+  // The flags, restitution and slip are the same for every contact of one resolver call: they are
+  // looked up (a dozen dependent loads) at its first contact and kept for the rest.
+  bool em_known = false;
+  int em_flags = 0;
+  R em_rest = 0, em_slip = 0;
+  CHP_HD void contact_params(int bi, int bj, SRef si, SRef sj, SRef rsi, SRef rsj) {
     const R* cmp = W.cm_params + 6 * cm;
-    bool enabled = (W.flags[bi] & BF_RESPONSE) && (W.flags[bj] & BF_RESPONSE) && si.resp && sj.resp;
+    const bool enabled = (W.flags[bi] & BF_RESPONSE) && (W.flags[bj] & BF_RESPONSE) && si.resp && sj.resp;
     R rest = cmp[1];
     int ma = si.mat >= 0 ? si.mat : W.material[bi];
     int mb = sj.mat >= 0 ? sj.mat : W.material[bj];
@@ -141,7 +142,7 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     if (fa >= 0 && fb >= 0 && W.mat_friction[fa] >= (R)0 && W.mat_friction[fb] >= (R)0)
       fric = W.mat_friction[fa] * W.mat_friction[fb];
     R slip = 0;
-    bool hasf = fric > (R)0;
+    const bool hasf = fric > (R)0;
     if (hasf) {
       R mug = fric * W.fric_grav_len;
       R rm = W.inv_mass[bi] + W.inv_mass[bj];
@@ -151,10 +152,21 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     int bmi = W.material[bi], bmj = W.material[bj];
     if (bmi >= 0 && bmj >= 0 && W.mat_restitution[bmi] >= (R)0 && W.mat_restitution[bmj] >= (R)0)
       rest = W.mat_restitution[bmi] * W.mat_restitution[bmj];
-    bool trig = (W.flags[bi] & BF_TRIGGER) || (W.flags[bj] & BF_TRIGGER);
-    c.flags = (enabled && !trig ? 1 : 0) | (hasf ? 2 : 0);
-    c.restitution = rest;
-    c.slip = slip;
+    const bool trig = (W.flags[bi] & BF_TRIGGER) || (W.flags[bj] & BF_TRIGGER);
+    em_flags = (enabled && !trig ? 1 : 0) | (hasf ? 2 : 0);
+    em_rest = rest;
+    em_slip = slip;
+    em_known = true;
+  }
+  CHP_HD void emit(int bi, int bj, SRef si, SRef sj, SRef rsi, SRef rsj, f3 ri, f3 rj, f3 ni) {
+    if (!em_known) contact_params(bi, bj, si, sj, rsi, rsj);
+    ContactRec<R> c;
+    c.bi = bi; c.bj = bj; c.cm = cm;
+    c.si = rsi.id; c.sj = rsj.id;   // createContactEquation: c.si = overrideShapeA ?? si
+    c.ri = ri; c.rj = rj; c.ni = ni;
+    c.flags = em_flags;
+    c.restitution = em_rest;
+    c.slip = em_slip;
     sink->push(c);
   }
   CHP_HD f3 P(int b) const { return ((const f3*)W.pos)[b]; }
@@ -896,6 +908,7 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
         // the resolvers take the lower shape type first; one call, so that each is compiled once
         auto ordered = [&]() {
           const bool sw = !(W.si_type[sa] < W.si_type[sb]);
+          em_known = false;
           dispatch(sw ? sb : sa, sw ? sa : sb, sw ? xj : xi, sw ? xi : xj, sw ? qj : qi, sw ? qi : qj, sw ? bj : bi,
                    sw ? bi : bj, rsi, rsj);
         };
