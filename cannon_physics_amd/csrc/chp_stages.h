@@ -1326,11 +1326,11 @@ struct GWave {
 };
 // GS record: 6 groups of 4 words, row position k at words [k * 24, k * 24 + 24)
 //   g0 sa.x sa.y sa.z ima  | g1 ra.x ra.y ra.z B    | g2 rb.x rb.y rb.z invC
-//   g3 ia.x ia.y ia.z eps  | g4 ib.x ib.y ib.z minF | g5 imb maxF a' b'
+//   g3 ia.x ia.y ia.z eps  | g4 ib.x ib.y ib.z minF | g5 a' maxF imb b'
 // a' = a | (a dynamic) << 31, b' = b | (b dynamic) << 31, as in row_ab; imb (never negative) has its
 // sign set when sb == -sa (else both spatial parts are +0).  The groups are
 // what the four lanes of a row load (st_gs): each a Jacobian part and the part its impulse moves
-// the velocity along, with one of the row's scalars in the fourth word.
+// the velocity along, with one of the row's scalars in the fourth word; and a word each of g5.
 template <typename R> struct GsWord;
 template <> struct GsWord<float> {
   typedef unsigned int T;
@@ -1371,9 +1371,9 @@ template <typename R> __device__ __forceinline__ void gs_load(const typename GsW
   auto S = [&](int i) { return GsWord<R>::get(w[i]); };
   o.sa = mk3(F(0), F(1), F(2)); o.ra = mk3(F(4), F(5), F(6)); o.rb = mk3(F(8), F(9), F(10));
   o.ia = mk3(F(12), F(13), F(14)); o.ib = mk3(F(16), F(17), F(18));
-  o.neg = flip_top<R>(w[20]);
-  o.ima = S(3); o.imb = o.neg ? -S(20) : S(20); o.B = S(7); o.invC = S(11); o.eps = S(15); o.minF = S(19); o.maxF = S(21);
-  o.a = (unsigned)w[22]; o.b = (unsigned)w[23];
+  o.neg = flip_top<R>(w[22]);
+  o.ima = S(3); o.imb = o.neg ? -S(22) : S(22); o.B = S(7); o.invC = S(11); o.eps = S(15); o.minF = S(19); o.maxF = S(21);
+  o.a = (unsigned)w[20]; o.b = (unsigned)w[23];
 }
 
 template <typename R> __device__ __forceinline__ void gs_store(typename GsWord<R>::T* base, int k,
@@ -1388,8 +1388,8 @@ template <typename R> __device__ __forceinline__ void gs_store(typename GsWord<R
   P(16, r.ib.x); P(17, r.ib.y); P(18, r.ib.z); P(19, r.minF);
   P(21, r.maxF);
   bool neg = !(r.kind == CHP_ROW_ROTATIONAL || r.kind == CHP_ROW_CONE || r.kind == CHP_ROW_MOTOR);
-  P(20, neg ? -r.imb : r.imb);
-  w[22] = (T)fa;
+  P(22, neg ? -r.imb : r.imb);
+  w[20] = (T)fa;
   w[23] = (T)fb;
 #pragma unroll
   for (int g = 0; g < GS_GROUPS; g++) {
@@ -1766,7 +1766,8 @@ template <int CTRL> __device__ __forceinline__ double quad(double v) {
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xf, 0xf, true);
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-constexpr int QP_SWAP1 = 0xB1, QP_SWAP2 = 0x4E, QP_LANE1 = 0x55, QP_LANE3 = 0xFF;   // [1,0,3,2] [2,3,0,1] [1,..] [3,..]
+constexpr int QP_SWAP1 = 0xB1, QP_SWAP2 = 0x4E;   // [1,0,3,2] [2,3,0,1]
+constexpr int QP_LANE0 = 0x00, QP_LANE1 = 0x55, QP_LANE3 = 0xFF, QP_LANES0033 = 0xF0;   // [0,..] [1,..] [3,..] [0,0,3,3]
 // v with its sign flipped where the top bit of m is set
 __device__ __forceinline__ float flip_sign(float v, unsigned m) { return __uint_as_float(__float_as_uint(v) ^ m); }
 __device__ __forceinline__ double flip_sign(double v, unsigned m) {
@@ -1867,7 +1868,16 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
     const unsigned negm = p == 2 ? 0x80000000u : 0u, half = (p & 1) * 16u, spare = 32u * nb + half;
     const bool first = p < 2, odd = p & 1;
     char* vb = (char*)vw;
-    GsQuad<R> qa[D], qk[D], qc[D];
+    GsQuad<R> qa[D], qk[D];
+    // g5: a word per lane, handed round the four (a quarter of the bytes the loads move, two
+    // permutations more), or all of it in each lane.  The word wins where the loads are what the
+    // steps wait for and loses where one world's four waves wait for each other: half a batch
+    // of 1024 chains 1167 -> 1063 us, of 2048 piles 334 -> 322, a 16,384-body world 4.01 -> 3.74 ms,
+    // a 300-body pile in double 290 -> 253, but in single 83 -> 92
+    constexpr bool WORD = sizeof(R) == 8 || NW != 4;
+    GsQuad<R> qc[WORD ? 1 : D];
+    WT qw[WORD ? D : 1];
+    const unsigned oc = (WORD ? 20u + p : 20u) * (unsigned)sizeof(R);
     R ql[D];
     unsigned qr[D];   // the row's position
     int pt = 0, s0, s1;   // the next step to load and its rows
@@ -1878,22 +1888,25 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
         const size_t o = (size_t)k * REC;
         qa[s].load((const WT*)(gsr + (o + oa)));
         qk[s].load((const WT*)(gsr + (o + ok)));
-        qc[s].load((const WT*)(gsr + (o + 20 * sizeof(R))));
+        if constexpr (WORD) qw[s] = *(const WT*)(gsr + (o + oc));
+        else qc[s].load((const WT*)(gsr + (o + oc)));
         ql[s] = *(const R*)(lam + (size_t)k * LAM);
       } else {
         qa[s].load((const WT*)(gsr + (__umul24(k, REC) + oa)));
         qk[s].load((const WT*)(gsr + (__umul24(k, REC) + ok)));
-        qc[s].load((const WT*)(gsr + (__umul24(k, REC) + 20u * (unsigned)sizeof(R))));
+        if constexpr (WORD) qw[s] = *(const WT*)(gsr + (__umul24(k, REC) + oc));
+        else qc[s].load((const WT*)(gsr + (__umul24(k, REC) + oc)));
         ql[s] = *(const R*)(lam + k * LAM);
       }
       qr[s] = k;
       pt = pt + 1 == Lpad ? 0 : pt + 1;
     };
-    // the body slot half this lane reads for slot s's row
-    auto body = [&](int s) {
-      const unsigned w = first ? (unsigned)qc[s].w[2] : (unsigned)qc[s].w[3];
-      return (w << 5) + half;
+    // a' or b' of slot s's row; the half of that body's slot this lane reads
+    auto word = [&](int s) {
+      if constexpr (WORD) return (unsigned)__builtin_amdgcn_update_dpp(0, (int)qw[s], QP_LANES0033, 0xf, 0xf, true);
+      else return first ? (unsigned)qc[s].w[0] : (unsigned)qc[s].w[3];
     };
+    auto body = [&](int s) { return (word(s) << 5) + half; };
     // The sweeps run in an inner loop whose only memory traffic is the ring's loads and the
     // lambda stores.  The rare undecided early-exit test reads the stored |dlambda| outside
     // it, and the ring then starts again at the first step of the next sweep.
@@ -1917,8 +1930,17 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
           // slot's row before its own step makes the wave wait for that row's loads, and the
           // ring then hides no latency
           __builtin_amdgcn_sched_barrier(0);
-          const unsigned wa = (unsigned)qc[s].w[2], wb = (unsigned)qc[s].w[3], w = first ? wa : wb;
-          const unsigned neg = (unsigned)(qc[s].w[0] >> (8 * sizeof(R) - 32)) & negm;
+          const unsigned w = word(s);
+          WT wi;       // imb: lane 2's
+          R maxF;
+          if constexpr (WORD) {
+            wi = qw[s];
+            maxF = quad<QP_LANE1>(GsWord<R>::get(wi));
+          } else {
+            wi = qc[s].w[2];
+            maxF = qc[s].get(1);
+          }
+          const unsigned neg = (unsigned)(wi >> (8 * sizeof(R) - 32)) & negm;
           const R jx = flip_sign(qa[s].get(0), neg), jy = flip_sign(qa[s].get(1), neg), jz = flip_sign(qa[s].get(2), neg);
           R d = (R)v4.x * jx;
           d += (R)v4.y * jy;
@@ -1927,19 +1949,21 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
           const R gwl = d + quad<QP_SWAP2>(d);
           const R own = qa[s].get(3);
           const R B = quad<QP_LANE1>(own), invC = quad<QP_LANE3>(own);
-          const R eps = quad<QP_LANE1>(qk[s].get(3)), minF = quad<QP_LANE3>(qk[s].get(3)), maxF = qc[s].get(1);
+          const R eps = quad<QP_LANE1>(qk[s].get(3)), minF = quad<QP_LANE3>(qk[s].get(3));
           const R clam = ql[s];
           R dl = invC * (B - gwl - eps * clam);
           // the clamp of gs_solver.dart:91-96 as selects; NaN compares false, as in the branches
           const R t = clam + dl;
           dl = t < minF ? minF - clam : (t > maxF ? maxF - clam : dl);
           // va += (ima dl) sa, wa += dl ia, vb += (imb dl) sb, wb += dl ib
-          const R c = odd ? (R)1 : (first ? own : (R)fabs(qc[s].get(0)));
+          const R c = odd ? (R)1 : (first ? own : (R)fabs(GsWord<R>::get(wi)));
           const R sc = flip_sign(c * dl, neg);
           const R kx = qk[s].get(0), ky = qk[s].get(1), kz = qk[s].get(2);
           float4 o = make_float4((float)((R)v4.x + sc * kx), (float)((R)v4.y + sc * ky), (float)((R)v4.z + sc * kz), 0.f);
           unsigned to = (w & GS_DYN) ? at : spare;
           if constexpr (SELF) {   // one body on both sides: its second impulse follows the first
+            const unsigned wa = (unsigned)__builtin_amdgcn_update_dpp(0, (int)w, QP_LANE0, 0xf, 0xf, true);
+            const unsigned wb = (unsigned)__builtin_amdgcn_update_dpp(0, (int)w, QP_LANE3, 0xf, 0xf, true);
             const bool same = ((wa ^ wb) & GS_IDX) == 0;
             const float ax = quad<0x44>(o.x), ay = quad<0x44>(o.y), az = quad<0x44>(o.z);   // lanes 0, 1, 0, 1
             if (same && !first && (wa & GS_DYN))
