@@ -21,6 +21,46 @@ struct HullVerts8 {
   int nv;
 };
 
+// the value of the lane a DPP control names, of lane l
+template <int CTRL> __device__ __forceinline__ int dpp(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true); }
+template <int CTRL> __device__ __forceinline__ float dpp(float v) { return __int_as_float(dpp<CTRL>(__float_as_int(v))); }
+template <int CTRL> __device__ __forceinline__ double dpp(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = dpp<CTRL>((int)x), hi = dpp<CTRL>((int)(x >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ int lane_of(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ float lane_of(float v, int l) { return __int_as_float(lane_of(__float_as_int(v), l)); }
+__device__ __forceinline__ double lane_of(double v, int l) {
+  const long long x = __double_as_longlong(v);
+  return __longlong_as_double(((long long)lane_of((int)(x >> 32), l) << 32) | (unsigned)lane_of((int)x, l));
+}
+__device__ __forceinline__ f3 lane_of(f3 v, int l) { return mk3(lane_of(v.x, l), lane_of(v.y, l), lane_of(v.z, l)); }
+// (key, index): the least key and its least index over each sixteen lanes, in all of them
+template <typename R> __device__ __forceinline__ void row_argmin(R& key, int& idx) {
+  auto take = [&](R k, int i) {
+    const bool t = k < key || (k == key && i < idx);
+    key = t ? k : key;
+    idx = t ? i : idx;
+  };
+  take(dpp<0x128>(key), dpp<0x128>(idx));   // rotations by 8, 4, 2, 1 lanes
+  take(dpp<0x124>(key), dpp<0x124>(idx));
+  take(dpp<0x122>(key), dpp<0x122>(idx));
+  take(dpp<0x121>(key), dpp<0x121>(idx));
+}
+
+// f3 values in LDS and vertices there, by an LDS pointer: through a pointer that may also be global
+// the loads are FLAT ones, which wait for both memories
+struct LdsF3 {
+  const __attribute__((address_space(3))) float* p;
+  __device__ __forceinline__ LdsF3(const f3* v) : p((const __attribute__((address_space(3))) float*)(const float*)v) {}
+  __device__ __forceinline__ f3 operator[](int i) const { return mk3(p[3 * i], p[3 * i + 1], p[3 * i + 2]); }
+};
+struct HullVertsLds {
+  LdsF3 v;
+  int nv;
+};
+
 template <typename R> CHP_HD HullView<R> hull_view(const DevWorld<R>& W, int h) {
   HullView<R> H;
   H.v = (const f3*)W.h_verts + W.h_vstart[h];
@@ -40,8 +80,8 @@ template <typename R> CHP_HD HullView<R> hull_view(const DevWorld<R>& W, int h) 
 
 struct SRef { int resp; int mat; int id; };   // Shape.collisionResponse / .material, instance
 
-// where resolvers put contacts.  WAVE: every lane of a wave computes the same contacts and
-// lane 0 stores them.  Two kinds:
+// where resolvers put contacts.  WAVE: every lane of a wave holds the same counts; push is given the
+// same contact by all lanes (lane 0 stores it), the hull resolvers store a contact per lane.  Two kinds:
 //  - buffered: into buf (a local or LDS array of cap records); writes beyond cap are counted,
 //    not stored, and the caller runs the pair again straight into the slab;
 //  - direct (slot != nullptr): a resolver that emits all of a pair's contacts in one go first
@@ -96,7 +136,7 @@ struct Poly {
 enum : unsigned { NK_SS = 1, NK_SP = 2, NK_SB = 4, NK_SC = 8, NK_SH = 16, NK_PC = 32, NK_CC = 64, NK_HC = 128,
                   NK_ALL = 255 };
 
-// A resolver context.  WAVE: a whole wave runs one pair, every lane on the same data (so every
+// A resolver context.  WAVE: a whole wave runs one pair, every lane on the same data unless said otherwise (so every
 // branch is uniform), and the separating-axis search splits its axes over the lanes.
 template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   const DevWorld<R>& W;
@@ -160,6 +200,9 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   }
   CHP_HD void emit(int bi, int bj, SRef si, SRef sj, SRef rsi, SRef rsj, f3 ri, f3 rj, f3 ni) {
     if (!em_known) contact_params(bi, bj, si, sj, rsi, rsj);
+    sink->push(record(bi, bj, rsi, rsj, ri, rj, ni));
+  }
+  CHP_HD ContactRec<R> record(int bi, int bj, SRef rsi, SRef rsj, f3 ri, f3 rj, f3 ni) const {
     ContactRec<R> c;
     c.bi = bi; c.bj = bj; c.cm = cm;
     c.si = rsi.id; c.sj = rsj.id;   // createContactEquation: c.si = overrideShapeA ?? si
@@ -167,7 +210,7 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     c.flags = em_flags;
     c.restitution = em_rest;
     c.slip = em_slip;
-    sink->push(c);
+    return c;
   }
   CHP_HD f3 P(int b) const { return ((const f3*)W.pos)[b]; }
 
@@ -334,19 +377,29 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   // sphereConvex (:1039-1257); returns the number of contacts added (0 or 1)
   CHP_HD int sphereConvex(R Rr, const HullView<R>& H, f3 xi, f3 xj, f4 qj, int bi, int bj, SRef si, SRef sj,
                           SRef rsi, SRef rsj) {
-    for (int i = 0; i != H.nv; i++) {
-      f3 wc = add3<R>(xj, qrot<R>(qj, H.v[i]));
-      f3 s2c = sub3<R>(wc, xi);
-      if (len2<R>(s2c) < Rr * Rr) {
-        f3 ri = normalize3<R>(s2c);
-        f3 n = ri;
-        ri = scale3<R>(ri, Rr);
-        f3 rj = sub3<R>(wc, xj);
-        ri = sub3<R>(add3<R>(ri, xi), P(bi));
-        rj = sub3<R>(add3<R>(rj, xj), P(bj));
-        emit(bi, bj, si, sj, rsi, rsj, ri, rj, n);
-        return 1;
-      }
+    int corner = -1;
+    f3 wc{}, s2c{};
+    auto in_sphere = [&](f3 v, int i) {
+      const f3 c = add3<R>(xj, qrot<R>(qj, v)), d = sub3<R>(c, xi);
+      if (corner < 0 && len2<R>(d) < Rr * Rr) { corner = i; wc = c; s2c = d; }
+    };
+    if (H.nv <= 8) {   // (the vertices' loads all in flight)
+      const HullVerts8 v = verts8(H);
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        if (i < H.nv) in_sphere(v.v[i], i);
+    } else {
+      for (int i = 0; i != H.nv && corner < 0; i++) in_sphere(H.v[i], i);
+    }
+    if (corner >= 0) {
+      f3 ri = normalize3<R>(s2c);
+      f3 n = ri;
+      ri = scale3<R>(ri, Rr);
+      f3 rj = sub3<R>(wc, xj);
+      ri = sub3<R>(add3<R>(ri, xi), P(bi));
+      rj = sub3<R>(add3<R>(rj, xj), P(bj));
+      emit(bi, bj, si, sj, rsi, rsj, ri, rj, n);
+      return 1;
     }
     for (int i = 0; i != H.nf; i++) {
       int f0 = H.fis[i], f1 = H.fis[i + 1];
@@ -422,7 +475,7 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   // ConvexPolyhedron.project (convex_polyhedron.dart:843-883).  lo is
   // Transform.pointToLocalFrame(pos, quat, 0), which depends only on the hull's pose: the
   // callers compute it once per hull and pass it in (same arithmetic, evaluated once).
-  CHP_HD static void project(const HullView<R>& H, f3 axis, f3 lo, f4 q, R& mx, R& mn) {
+  template <class VS> CHP_HD static void project(const VS& H, f3 axis, f3 lo, f4 q, R& mx, R& mn) {
     f3 la = vector_to_local<R>(q, axis);
     R add = dot3<R>(lo, la);
     R a = dot3<R>(H.v[0], la), b = a;
@@ -463,8 +516,8 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     return c;
   }
   // testSepAxis (:360-384): false when separated
-  template <class VS>
-  CHP_HD static bool testSepAxis(const VS& A, f3 axis, const VS& B, f3 loA, f4 qa, f3 loB, f4 qb, R& depth) {
+  template <class VSA, class VSB>
+  CHP_HD static bool testSepAxis(const VSA& A, f3 axis, const VSB& B, f3 loA, f4 qa, f3 loB, f4 qb, R& depth) {
     R maxA, minA, maxB, minB;
     project(A, axis, loA, qa, maxA, minA);
     project(B, axis, loB, qb, maxB, minB);
@@ -478,7 +531,8 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   CHP_HD static bool findSepAxis(const HullView<R>& A, const HullView<R>& B, f3 pa, f4 qa, f3 pb, f4 qb, bool face0_only,
                                  f3& target) {
     if constexpr (WAVE) {
-      return findSepAxisWave(A, B, pa, qa, pb, qb, face0_only, target);
+      return findSepAxisWave(A, B, A, B, pa, qa, pb, qb, face0_only, target, [&](int k) { return qrot<R>(qa, A.e[k]); },
+                             [&](int k) { return qrot<R>(qb, B.e[k]); });
     } else {
       if (A.nv <= 8 && B.nv <= 8) {
         const HullVerts8 va = verts8(A), vb = verts8(B);
@@ -531,9 +585,10 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   // wave.  The sequential search returns "separated" at the first separating axis, else the
   // first axis of least depth (strict <): here any lane's separating axis answers the first, a
   // (depth, axis index) minimum over the lanes the second.
-  __device__ static bool findSepAxisWave(const HullView<R>& A, const HullView<R>& B, f3 pa, f4 qa, f3 pb, f4 qb,
-                                         bool face0_only, f3& target, const f3* weA = nullptr,
-                                         const f3* weB = nullptr) {
+  // vA, vB: the vertices; eA, eB: the world edge directions
+  template <class VS, class EA, class EB>
+  __device__ static bool findSepAxisWave(const HullView<R>& A, const HullView<R>& B, const VS& vA, const VS& vB, f3 pa,
+                                         f4 qa, f3 pb, f4 qb, bool face0_only, f3& target, EA eA, EB eB) {
     const int lane = threadIdx.x & 63;
     const f3 zero = mk3(0.f, 0.f, 0.f);
     f3 loA = point_to_local<R>(pa, qa, zero), loB = point_to_local<R>(pb, qb, zero);
@@ -555,30 +610,31 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
           axis = qrot<R>(qb, B.fn[k - nA]);
         } else {
           int e = k - nA - nB, e0 = e / B.ne, e1 = e - e0 * B.ne;
-          const f3 ea = weA ? weA[e0] : qrot<R>(qa, A.e[e0]), eb = weB ? weB[e1] : qrot<R>(qb, B.e[e1]);
-          f3 cr = cross3<R>(ea, eb);
+          f3 cr = cross3<R>(eA(e0), eB(e1));
           valid = !almost_zero3<R>(cr);
           axis = valid ? normalize3<R>(cr) : zero;
         }
         if (valid) {
           R d;
-          if (!testSepAxis(A, axis, B, loA, qa, loB, qb, d)) sep = true;
+          if (!testSepAxis(vA, axis, vB, loA, qa, loB, qb, d)) sep = true;
           else if (d < best) { best = d; bestk = k; bax = axis; }
         }
       }
       if (__any(sep)) return false;
     }
-    // lexicographic (depth, axis index) minimum over the wave
-    int win = lane;
-    for (int off = 32; off > 0; off >>= 1) {
-      R ob = __shfl_xor(best, off, 64);
-      int ok = __shfl_xor(bestk, off, 64), ow = __shfl_xor(win, off, 64);
-      if (ob < best || (ob == best && ok < bestk)) { best = ob; bestk = ok; win = ow; }
+    // lexicographic (depth, axis index) minimum over the wave; an axis' lane is its index modulo 64
+    row_argmin(best, bestk);
+    R wk = lane_of(best, 0);
+    int wi = lane_of(bestk, 0);
+#pragma unroll
+    for (int r = 16; r < 64; r += 16) {
+      const R k = lane_of(best, r);
+      const int i = lane_of(bestk, r);
+      const bool t = k < wk || (k == wk && i < wi);
+      wk = t ? k : wk;
+      wi = t ? i : wi;
     }
-    win = __builtin_amdgcn_readfirstlane(win);
-    target = mk3(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bax.x), win)),
-                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bax.y), win)),
-                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bax.z), win)));
+    target = lane_of(bax, wi & 63);
     f3 dc = sub3<R>(pb, pa);
     if (dot3<R>(dc, target) > (R)0) target = neg3(target);
     return true;
@@ -607,19 +663,126 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     if (nout > cap) { status |= WS_STAGING; nout = cap; }
     return nout;
   }
+  // the same by a wave, a polygon vertex per lane (cap <= 64)
+  __device__ static int clipPlaneWave(Poly in, int nin, Poly out, int cap, f3 n, R c, int& status) {
+    if (nin < 2) return 0;
+    const int lane = (int)(threadIdx.x & 63);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    bool one = false, two = false;   // this vertex' output: its cut or itself, and itself after the cut
+    f3 o = mk3(0.f, 0.f, 0.f), last = o;
+    if (lane < nin) {
+      last = in[lane];
+      const f3 first = in[lane == 0 ? nin - 1 : lane - 1];
+      const R ndl = dot3<R>(n, last) + c, ndf = dot3<R>(n, first) + c;
+      one = ndf < (R)0 || ndl < (R)0;
+      two = !(ndf < (R)0) && ndl < (R)0;
+      o = ndf < (R)0 && ndl < (R)0 ? last : lerp3<R>(first, last, ndf / (ndf - ndl));
+    }
+    const unsigned long long m1 = __ballot(one), m2 = __ballot(two);
+    const int at = __popcll(m1 & below) + __popcll(m2 & below);
+    if (one && at < cap) out[at] = o;
+    if (two && at + 1 < cap) out[at + 1] = last;
+    wave_fence();
+    int nout = __popcll(m1) + __popcll(m2);
+    if (nout > cap) { status |= WS_STAGING; nout = cap; }
+    return nout;
+  }
   // convexConvex (narrow_phase.dart:1981-2043) with clipAgainstHull / clipFaceAgainstHull
   // (convex_polyhedron.dart:189-227, 417-541; their unused temporaries are omitted)
-  // WAVE: lanes copy n items (rotated by q when rot) into the workspace; then the wave sees them
-  __device__ static void stage(f3* dst, const f3* src, int n, bool rot, f4 q) {
-    for (int i = (int)(threadIdx.x & 63); i < n; i += 64) dst[i] = rot ? qrot<R>(q, src[i]) : src[i];
+  // WAVE: a hull's vertices and world edge directions into the workspace (at most 64 of each)
+  __device__ static void stage(f3* dv, f3* de, const HullView<R>& H, f4 q) {
+    const int lane = (int)(threadIdx.x & 63);
+    f3 v = mk3(0.f, 0.f, 0.f), e = v;
+    if (lane < H.nv) v = H.v[lane];
+    if (lane < H.ne) e = H.e[lane];
+    if (lane < H.nv) dv[lane] = v;
+    if (lane < H.ne) de[lane] = qrot<R>(q, e);
+  }
+  // A is the same hull at the same pose for every pillar of a heightfield pair: staged once
+  __device__ void stageA(const HullView<R>& A, f4 q) {
+    const bool same = ws_a == A.v && __float_as_uint(ws_qa.x) == __float_as_uint(q.x) &&
+                      __float_as_uint(ws_qa.y) == __float_as_uint(q.y) && __float_as_uint(ws_qa.z) == __float_as_uint(q.z) &&
+                      __float_as_uint(ws_qa.w) == __float_as_uint(q.w);
+    if (same) return;
+    stage(ws + WS_VA, ws + WS_EA, A, q);
+    ws_a = A.v;
+    ws_qa = q;
+  }
+  // what the lanes wrote to LDS before it, all of them read after it
+  __device__ static void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  CHP_HD void convexConvex(const HullView<R>& A0, SRef siRef, const HullView<R>& B0, SRef sjRef, f3 xi, f3 xj, f4 qi,
+  // the part of it after the axis search, by a wave: a face, polygon vertex, plane or contact per
+  // lane (faces of at most MAX_FACE_VERTS vertices, polygons of at most 64)
+  __device__ void clipWave(const HullView<R>& A, SRef siRef, const HullView<R>& B, SRef sjRef, f3 xi, f3 xj, f4 qi, f4 qj,
+                           int bi, int bj, SRef rsi, SRef rsj, f3 sep, Poly bufA, Poly bufB, int cap) {
+    const int lane = (int)(threadIdx.x & 63);
+    // lanes 0-15 look for B's face most aligned with the axis, 16-31 for A's most anti-aligned; the
+    // first face wins a tie, and NaN never
+    R key = (R)__builtin_huge_val();
+    int idx = 0x7fffffff;
+    const bool onB = lane < 16;
+    if (lane < 32) {
+      const int nf = onB ? B.nf : A.nf;
+      const f3* fn = onB ? B.fn : A.fn;
+      const f4 q = onB ? qj : qi;
+      for (int f = lane & 15; f < nf; f += 16) {
+        const R d = dot3<R>(qrot<R>(q, fn[f]), sep), k = onB ? -d : d;
+        if (k < key) { key = k; idx = f; }
+      }
+    }
+    row_argmin(key, idx);
+    const int cfb = lane_of(idx, 0), cfa = lane_of(idx, 16);
+    if (cfb == 0x7fffffff) return;
+    const int b0 = B.fis[cfb];
+    int nin = B.fis[cfb + 1] - b0;
+    if (nin > cap) { status |= WS_STAGING; return; }
+    if (lane < nin) bufA[lane] = add3<R>(qrot<R>(qj, B.v[B.fidx[b0 + lane]]), xj);
+    wave_fence();
+    if (cfa == 0x7fffffff) return;
+    const int pa0 = A.fis[cfa], nva = A.fis[cfa + 1] - pa0;
+    const int c0 = A.fcs[cfa], nconn = A.fcs[cfa + 1] - c0;
+    // lane i: the i-th clip plane; lane nva: the witness face's own
+    f3 pn = mk3(0.f, 0.f, 0.f);
+    R pe = 0;
+    if (lane <= nva) {
+      const int other = lane == nva ? cfa : (nconn > lane ? A.fconn[c0 + lane] : 0);
+      const f3 lpn = A.fn[other];
+      const R lpe = -dot3<R>(lpn, A.v[A.fidx[A.fis[other]]]);
+      pn = qrot<R>(qi, lpn);
+      pe = lpe - dot3<R>(pn, xi);
+    }
+    Poly pin = bufA, pout = bufB;
+    for (int i = 0; i < nva; i++) {
+      nin = clipPlaneWave(pin, nin, pout, cap, lane_of(pn, i), lane_of(pe, i), status);
+      Poly t = pin; pin = pout; pout = t;
+    }
+    const f3 pnws = lane_of(pn, nva);
+    const R pews = lane_of(pe, nva);
+    bool hit = false;
+    f3 ri = mk3(0.f, 0.f, 0.f), rj = ri;
+    if (lane < nin) {
+      const f3 v = pin[lane];
+      R depth = dot3<R>(pnws, v) + pews;
+      if (depth <= (R)-100) depth = (R)-100;
+      hit = depth <= (R)100 && depth <= (R)1e-6;
+      const f3 q = scale3<R>(neg3(pnws), depth);
+      ri = sub3<R>(add3<R>(sub3<R>(add3<R>(v, q), xi), xi), P(bi));
+      rj = sub3<R>(add3<R>(sub3<R>(v, xj), xj), P(bj));
+    }
+    const unsigned long long m = __ballot(hit);
+    if (m == 0) return;
+    if (!em_known) contact_params(bi, bj, siRef, sjRef, rsi, rsj);
+    const int at = sink->n + __popcll(m & ((1ull << lane) - 1ull));
+    if (hit && at < sink->cap) sink->buf[at] = record(bi, bj, rsi, rsj, ri, rj, neg3(sep));
+    sink->n += __popcll(m);
+    if (sink->n > sink->cap) sink->overflow = 1;
+  }
+  CHP_HD void convexConvex(const HullView<R>& A, SRef siRef, const HullView<R>& B, SRef sjRef, f3 xi, f3 xj, f4 qi,
                            f4 qj, int bi, int bj, SRef rsi, SRef rsj, bool face0_only) {
-    if (dist3<R>(xi, xj) > A0.bsr + B0.bsr) return;
-    HullView<R> A = A0, B = B0;
+    if (dist3<R>(xi, xj) > A.bsr + B.bsr) return;
     f3 sep = mk3(0.f, 0.f, 0.f);
     // the two clip polygons: the wave's workspace, or this lane's interleaved LDS area
     Poly bufA, bufB;
@@ -637,29 +800,24 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     if constexpr (WAVE) {
       // vertices and world edge directions from the workspace (the same values the global
       // tables give), clip polygons in it
-      const f3 *weA = nullptr, *weB = nullptr;
       if (A.nv <= WS_NV && B.nv <= WS_NV && A.ne <= WS_NE && B.ne <= WS_NE) {
-        // A is the same hull at the same pose for every pillar of a heightfield pair: staged once
-        const bool same = ws_a == A0.v && __float_as_uint(ws_qa.x) == __float_as_uint(qi.x) &&
-                          __float_as_uint(ws_qa.y) == __float_as_uint(qi.y) &&
-                          __float_as_uint(ws_qa.z) == __float_as_uint(qi.z) &&
-                          __float_as_uint(ws_qa.w) == __float_as_uint(qi.w);
-        if (!same) {
-          stage(ws + WS_VA, A0.v, A.nv, false, qi);
-          stage(ws + WS_EA, A0.e, A.ne, true, qi);
-          ws_a = A0.v;
-          ws_qa = qi;
-        }
-        stage(ws + WS_VB, B0.v, B.nv, false, qj);
-        stage(ws + WS_EB, B0.e, B.ne, true, qj);
-        A.v = ws + WS_VA;
-        B.v = ws + WS_VB;
-        weA = ws + WS_EA;
-        weB = ws + WS_EB;
+        stageA(A, qi);
+        stage(ws + WS_VB, ws + WS_EB, B, qj);
+        wave_fence();
+        const HullVertsLds vA{ws + WS_VA, A.nv}, vB{ws + WS_VB, B.nv};
+        const LdsF3 eA(ws + WS_EA), eB(ws + WS_EB);
+        if (!findSepAxisWave(A, B, vA, vB, xi, qi, xj, qj, face0_only, sep, [&](int k) { return eA[k]; },
+                             [&](int k) { return eB[k]; }))
+          return;
+      } else if (!findSepAxis(A, B, xi, qi, xj, qj, face0_only, sep)) {
+        return;
       }
-      if (!findSepAxisWave(A, B, xi, qi, xj, qj, face0_only, sep, weA, weB)) return;
     } else {
       if (!findSepAxis(A, B, xi, qi, xj, qj, face0_only, sep)) return;
+    }
+    if constexpr (WAVE) {
+      clipWave(A, siRef, B, sjRef, xi, xj, qi, qj, bi, bj, rsi, rsj, sep, bufA, bufB, cap);
+      return;
     }
     // clipAgainstHull: B's face most aligned with the axis
     int cfb = -1;
@@ -671,8 +829,6 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     if (cfb < 0) return;
     int nin = B.fis[cfb + 1] - B.fis[cfb];
     if (nin > cap) { status |= WS_STAGING; return; }
-    // (wave path: every lane computes and stores the same polygon; a wave's LDS accesses
-    // complete in program order, so each lane reads back what the wave wrote)
     for (int k = 0; k < nin; k++) bufA[k] = add3<R>(qrot<R>(qj, B.v[B.fidx[B.fis[cfb] + k]]), xj);
     // clipFaceAgainstHull: A's face most anti-aligned with the axis
     int cfa = -1;
@@ -744,9 +900,21 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     if (y0 >= ny) y0 = ny - 1;
     const R* d = W.hf_data + W.hf_dstart[hf];
     R m = W.hf_min[hf];  // Heightfield.getRectMinMax: min is the global minValue
-    for (int i = x0; i <= x1; i++)
-      for (int j = y0; j <= y1; j++)
-        if (d[i * ny + j] > m) m = d[i * ny + j];
+    if constexpr (WAVE) {   // the window's heights over the lanes
+      const int lane = (int)(threadIdx.x & 63), wy = y1 - y0 + 1, n = (x1 - x0 + 1) * wy;
+      for (int k = lane; k < n; k += 64) {
+        const R v = d[(x0 + k / wy) * ny + y0 + k % wy];
+        if (v > m) m = v;
+      }
+      for (int off = 32; off > 0; off >>= 1) {
+        const R v = __shfl_xor(m, off, 64);
+        if (v > m) m = v;
+      }
+    } else {
+      for (int i = x0; i <= x1; i++)
+        for (int j = y0; j <= y1; j++)
+          if (d[i * ny + j] > m) m = d[i * ny + j];
+    }
     mn = W.hf_min[hf];
     mx = m;
     return true;
@@ -776,7 +944,6 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
       // per pillar, two per cell.
       const int lane = (int)(threadIdx.x & 63);
       const int nyw = y1 - y0, ncand = (x1 - x0) * nyw * 2;
-      constexpr int NWORD = (int)(sizeof(ContactRec<R>) / sizeof(int));
       for (int c0 = 0; c0 < ncand; c0 += 64) {
         const int c = c0 + lane;
         ContactRec<R> rec{};
@@ -792,16 +959,11 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
             got = t.sphereConvex(Rr, H, xi, wpo, qj, bi, bj, si, pref, si, sj);
           }
         }
-        for (uint64_t m = __ballot(got != 0); m; m &= m - 1) {
-          const int l = __builtin_ctzll(m);
-          int w[NWORD];
-          __builtin_memcpy(w, &rec, sizeof(w));
-#pragma unroll
-          for (int k = 0; k < NWORD; k++) w[k] = __builtin_amdgcn_readlane(w[k], l);
-          ContactRec<R> o;
-          __builtin_memcpy(&o, w, sizeof(w));
-          sink->push(o);
-        }
+        const unsigned long long m = __ballot(got != 0);
+        const int at = sink->n + __popcll(m & ((1ull << lane) - 1ull));
+        if (got != 0 && at < sink->cap) sink->buf[at] = rec;
+        sink->n += __popcll(m);
+        if (sink->n > sink->cap) sink->overflow = 1;
       }
       return;
     }
@@ -817,6 +979,67 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
         if (sink->n - before > 2) return;
       }
   }
+  // heightfieldConvex and convexConvex by a wave: the second shape is the heightfield hf (hf >= 0), whose
+  // pillars near the hull are taken in turn, or the hull hullB.  One loop and one call for both:
+  // the resolvers' code, not their data, is what a launch of a few thousand pairs waits for
+  __device__ void hullPairsWave(const HullView<R>& A, SRef siRef, int hf, int hullB, SRef sjRef, f3 xi, f3 xj, f4 qi, f4 qj,
+                                int bi, int bj, SRef rsi, SRef rsj) {
+    const bool field = hf >= 0;
+    int x0 = 0, x1 = 0, y0 = 0, y1 = 0;
+    if (field) {
+      const f3 local = point_to_local<R>(xj, qj, xi);
+      const R radius = A.bsr;
+      R mn, mx;
+      if (!hfWindow(hf, local, radius, x0, x1, y0, y1, mn, mx)) return;
+      if (ld<R>(local.z) - radius > mx || ld<R>(local.z) + radius < mn) return;
+    }
+    const SRef pref{1, -1, sjRef.id};   // the pillar hull; its contacts name the heightfield
+    // The window's pillars (in the loop order i, j, lower/upper) are dealt to the lanes, 64 a
+    // round.  A lane drops its pillar when the bounding spheres miss, or when one of the face
+    // axes that findSeparatingAxis tests (the hull's face 0, then every pillar face;
+    // convex_polyhedron.dart:252-330) separates the two: the search then answers
+    // "separated" whatever the edge axes say, and convexConvex adds nothing.  The same
+    // projections of the same vertices decide it here, so the pillars left are exactly those
+    // that can add contacts; the wave takes them in loop order through convexConvex.
+    const int lane = (int)(threadIdx.x & 63);
+    const int nyw = y1 - y0, ncand = field ? (x1 - x0) * nyw * 2 : 1;
+    const f3 zero = mk3(0.f, 0.f, 0.f);
+    const f3 loA = point_to_local<R>(xi, qi, zero);
+    const bool staged = A.nv <= WS_NV && A.ne <= WS_NE;
+    if (staged) {
+      stageA(A, qi);
+      wave_fence();
+    }
+    for (int c0 = 0; c0 < ncand; c0 += 64) {
+      const int c = c0 + lane;
+      bool live = !field && lane == 0;
+      if (field && c < ncand) {
+        const int up = c & 1, ij = c >> 1, i = x0 + ij / nyw, j = y0 + ij % nyw;
+        const HullView<R> H = hull_view(W, pillarHull(hf, i, j, up));
+        const f3 wpo = point_to_world<R>(xj, qj, pillarOff(hf, i, j, up));
+        if (dist3<R>(xi, wpo) < H.bsr + A.bsr) {
+          live = true;
+          const f3 loB = point_to_local<R>(wpo, qj, zero);
+          R d;
+          auto faces = [&](const auto& va, const auto& vh) {
+            if (A.axes && !testSepAxis(va, qrot<R>(qi, A.fn[0]), vh, loA, qi, loB, qj, d)) live = false;
+            if (H.axes)
+              for (int f = 0; live && f < H.nf; f++)
+                if (!testSepAxis(va, qrot<R>(qj, H.fn[f]), vh, loA, qi, loB, qj, d)) live = false;
+          };
+          if (staged && H.nv <= 8) faces(HullVertsLds{ws + WS_VA, A.nv}, verts8(H));
+          else faces(A, H);
+        }
+      }
+      for (uint64_t m = __ballot(live); m; m &= m - 1) {
+        const int cc = c0 + __builtin_ctzll(m);
+        const int up = cc & 1, ij = cc >> 1, i = field ? x0 + ij / nyw : 0, j = field ? y0 + ij % nyw : 0;
+        const HullView<R> H = hull_view(W, field ? pillarHull(hf, i, j, up) : hullB);
+        const f3 wpo = field ? point_to_world<R>(xj, qj, pillarOff(hf, i, j, up)) : xj;
+        convexConvex(A, siRef, H, field ? pref : sjRef, xi, wpo, qi, qj, bi, bj, field ? siRef : rsi, field ? pref : rsj, field);
+      }
+    }
+  }
   // heightfieldConvex (:2044-2178): convexConvex against each pillar with faceListA = [0]
   CHP_HD void heightfieldConvex(const HullView<R>& A, SRef siRef, int hf, int hfId, f3 xi, f3 xj, f4 qi, f4 qj, int bi,
                                 int bj) {
@@ -827,45 +1050,6 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     if (!hfWindow(hf, local, radius, x0, x1, y0, y1, mn, mx)) return;
     if (ld<R>(local.z) - radius > mx || ld<R>(local.z) + radius < mn) return;
     SRef pref{1, -1, hfId};   // the pillar hull; its contacts name the heightfield
-    if constexpr (WAVE) {
-      // The window's pillars (in the loop order i, j, lower/upper) are dealt to the lanes, 64 a
-      // round.  A lane drops its pillar when the bounding spheres miss, or when one of the face
-      // axes that findSeparatingAxis tests (the hull's face 0, then every pillar face;
-      // convex_polyhedron.dart:252-330) separates the two: the search then answers
-      // "separated" whatever the edge axes say, and convexConvex adds nothing.  The same
-      // projections of the same vertices decide it here, so the pillars left are exactly those
-      // that can add contacts; the wave takes them in loop order through convexConvex.
-      const int lane = (int)(threadIdx.x & 63);
-      const int nyw = y1 - y0, ncand = (x1 - x0) * nyw * 2;
-      const f3 zero = mk3(0.f, 0.f, 0.f);
-      const f3 loA = point_to_local<R>(xi, qi, zero);
-      for (int c0 = 0; c0 < ncand; c0 += 64) {
-        const int c = c0 + lane;
-        bool live = false;
-        if (c < ncand) {
-          const int up = c & 1, ij = c >> 1, i = x0 + ij / nyw, j = y0 + ij % nyw;
-          const HullView<R> H = hull_view(W, pillarHull(hf, i, j, up));
-          const f3 wpo = point_to_world<R>(xj, qj, pillarOff(hf, i, j, up));
-          if (dist3<R>(xi, wpo) < H.bsr + A.bsr) {
-            live = true;
-            const f3 loB = point_to_local<R>(wpo, qj, zero);
-            R d;
-            if (A.axes && !testSepAxis(A, qrot<R>(qi, A.fn[0]), H, loA, qi, loB, qj, d)) live = false;
-            if (H.axes)
-              for (int f = 0; live && f < H.nf; f++)
-                if (!testSepAxis(A, qrot<R>(qj, H.fn[f]), H, loA, qi, loB, qj, d)) live = false;
-          }
-        }
-        for (uint64_t m = __ballot(live); m; m &= m - 1) {
-          const int cc = c0 + __builtin_ctzll(m);
-          const int up = cc & 1, ij = cc >> 1, i = x0 + ij / nyw, j = y0 + ij % nyw;
-          const HullView<R> H = hull_view(W, pillarHull(hf, i, j, up));
-          const f3 wpo = point_to_world<R>(xj, qj, pillarOff(hf, i, j, up));
-          convexConvex(A, siRef, H, pref, xi, wpo, qi, qj, bi, bj, siRef, pref, true);
-        }
-      }
-      return;
-    }
     for (int i = x0; i < x1; i++)
       for (int j = y0; j < y1; j++)
         for (int up = 0; up < 2; up++) {
@@ -905,36 +1089,32 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
         if (W.si_material[sa] >= 0 && W.si_material[sb] >= 0) shapeCM = W.cm_table[W.si_material[sa] * W.nmat + W.si_material[sb]];
         cm = shapeCM >= 0 ? shapeCM : (bodyCM >= 0 ? bodyCM : 0);
         SRef rsi{W.si_response[sa], W.si_material[sa], sa}, rsj{W.si_response[sb], W.si_material[sb], sb};
+        // the resolver's justTest answer: sphereSphere tests the distance (narrow_phase.dart:737-739),
+        // every other resolver whether it would create a contact
+        bool hit = false, resolve = true;
+        Sink<R, WAVE> held = *sink;
+        if constexpr (WAVE) if (justTest) {
+          resolve = !(W.si_type[sa] == CHP_SHAPE_SPHERE && W.si_type[sb] == CHP_SHAPE_SPHERE);
+          const R dx = ld<R>(xi.x) - ld<R>(xj.x), dy = ld<R>(xi.y) - ld<R>(xj.y), dz = ld<R>(xi.z) - ld<R>(xj.z);
+          const R rr = W.si_radius[sa] + W.si_radius[sb];
+          hit = dx * dx + dy * dy + dz * dz < rr * rr;
+          *sink = Sink<R, WAVE>{nullptr, 0, 0, 0};   // counts, stores nothing
+        }
         // the resolvers take the lower shape type first; one call, so that each is compiled once
-        auto ordered = [&]() {
+        if (resolve) {
           const bool sw = !(W.si_type[sa] < W.si_type[sb]);
           em_known = false;
           dispatch(sw ? sb : sa, sw ? sa : sb, sw ? xj : xi, sw ? xi : xj, sw ? qj : qi, sw ? qi : qj, sw ? bj : bi,
                    sw ? bi : bj, rsi, rsj);
-        };
+        }
         if constexpr (WAVE) if (justTest) {
-          // the resolver's justTest answer: sphereSphere tests the distance
-          // (narrow_phase.dart:737-739), every other resolver whether it would create a contact
-          bool hit;
-          if (W.si_type[sa] == CHP_SHAPE_SPHERE && W.si_type[sb] == CHP_SHAPE_SPHERE) {
-            const R dx = ld<R>(xi.x) - ld<R>(xj.x), dy = ld<R>(xi.y) - ld<R>(xj.y), dz = ld<R>(xi.z) - ld<R>(xj.z);
-            const R rr = W.si_radius[sa] + W.si_radius[sb];
-            hit = dx * dx + dy * dy + dz * dz < rr * rr;
-          } else {
-            Sink<R, WAVE> probe{nullptr, 0, 0, 0};   // counts, stores nothing
-            Sink<R, WAVE>* keep = sink;
-            sink = &probe;
-            ordered();
-            sink = keep;
-            hit = probe.n > 0;
-          }
+          if (resolve) hit = sink->n > 0;
+          *sink = held;
           if (hit && (threadIdx.x & 63) == 0) {   // Narrowphase.getContacts :712-716
             const int k = atomicAdd(&W.ev_ctl[EV_JT], 1);
             if (k < W.pair_cap) W.ev_jt[k] = make_int4(bi, bj, sa, sb);
           }
-          continue;
         }
-        ordered();
       }
     }
   }
@@ -955,9 +1135,15 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
       sphereHeightfield(W.si_radius[A], W.si_bsr[A], W.si_hf[B], xa, xb, qb, ba, bb, ra, rb);
     else if ((KINDS & NK_PC) && ta == CHP_SHAPE_PLANE && (tb == CHP_SHAPE_BOX || tb == CHP_SHAPE_CONVEX))
       planeConvex(hull_view(W, W.si_hull[B]), xa, xb, qa, qb, ba, bb, ra, rb, rsi, rsj);
-    else if ((KINDS & NK_CC) && convA && (tb == CHP_SHAPE_BOX || tb == CHP_SHAPE_CONVEX))
+    else if (WAVE && (KINDS & NK_CC) && (KINDS & NK_HC) && convA &&
+             (tb == CHP_SHAPE_BOX || tb == CHP_SHAPE_CONVEX || tb == CHP_SHAPE_HEIGHTFIELD)) {
+      if constexpr (WAVE)
+        hullPairsWave(hull_view(W, W.si_hull[A]), ra, tb == CHP_SHAPE_HEIGHTFIELD ? W.si_hf[B] : -1, W.si_hull[B], rb, xa, xb,
+                      qa, qb, ba, bb, rsi, rsj);
+    }
+    else if (!WAVE && (KINDS & NK_CC) && convA && (tb == CHP_SHAPE_BOX || tb == CHP_SHAPE_CONVEX))
       convexConvex(hull_view(W, W.si_hull[A]), ra, hull_view(W, W.si_hull[B]), rb, xa, xb, qa, qb, ba, bb, rsi, rsj, false);
-    else if ((KINDS & NK_HC) && convA && tb == CHP_SHAPE_HEIGHTFIELD)
+    else if (!WAVE && (KINDS & NK_HC) && convA && tb == CHP_SHAPE_HEIGHTFIELD)
       heightfieldConvex(hull_view(W, W.si_hull[A]), ra, W.si_hf[B], B, xa, xb, qa, qb, ba, bb);
     // other combinations have no resolver in the covered set (narrow_phase.dart:699-700 skips)
   }

@@ -859,44 +859,68 @@ constexpr int WAVE_KMAX = 64;
 // falling clear of a heightfield against one resting on a dozen pillars).  Waves numbered at or
 // beyond the queue's length leave at once, so an empty or short queue costs few atomics on the
 // one counter.
+// A pair is a chain of latencies, its instructions among them: a launch of a few hundred pairs
+// runs most of its code for the first time.  So each resolver is compiled once (46 KB; 198 KB when
+// the retry, the overlap probe and both users of convexConvex had copies of their own), the pair's
+// data are uniform, hulls are read from LDS through LDS pointers, and what follows the axis search
+// takes a lane per face, vertex, plane and contact (300-body pile 39 -> 19 us, 157 bodies in double
+// 48 -> 21 us, 24 terrains of 16 to 1024 bodies 553 -> 448 us a launch).
 // (ws: the wave's LDS workspace; loc: its LDS contact buffer of kmax records; clip_cap: points a
 // clip polygon may have)
 template <typename R, unsigned KINDS>
-__device__ void st_narrow_wave(const DevWorld<R>* worlds, const int2* queue, int cnt, int* ticket, R dt, f3* ws,
+__device__ __forceinline__ void st_narrow_wave(const DevWorld<R>* worlds, const int2* queue, int cnt, int* ticket, R dt, f3* ws,
                                ContactRec<R>* loc, int kmax, int clip_cap) {
   const int lane = threadIdx.x & 63;
   if ((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6) >= cnt) return;
   for (;;) {
     int i = 0;
     if (lane == 0) i = atomicAdd(ticket, 1);
-    i = __shfl(i, 0, 64);
+    i = uni(i);
     if (i >= cnt) break;
     const int2 q = queue[i];
-    const DevWorld<R>& W = worlds[q.x];
-    const int p = q.y;
-    const int bi = W.pair_i[p], bj = W.pair_j[p];
+    const DevWorld<R>& W = worlds[uni(q.x)];
+    const int p = uni(q.y);
+    const int bi = uni(W.pair_i[p]), bj = uni(W.pair_j[p]);
     Sink<R, true> s{loc, kmax, 0, 0};
     NPCtx<R, true, KINDS> ctx(W, dt, &s, ws);
     ctx.clip_cap = clip_cap;
-    ctx.pair(bi, bj);
-    int n = s.n, base = 0;
+    int n, base = 0;
+    for (;;) {   // (one call, so that the resolvers are compiled once)
+      ctx.pair(bi, bj);
+      NPCtx<R, true, KINDS>::wave_fence();   // the lanes' records
+      n = s.n;
+      if (s.buf != loc) break;
+      if (lane == 0) {
+        if (ctx.status) ws_fail(W.counters, ctx.status);
+        if (n > 0) base = atomicAdd(&W.counters[C_STAGING], n);
+      }
+      base = uni(base);
+      if (n > 0 && base + n > W.contact_cap) {
+        if (lane == 0) ws_fail(W.counters, WS_CONTACTS);
+        n = 0;
+      }
+      if (n <= kmax) break;
+      s = Sink<R, true>{W.contacts + base, n, 0, 0};   // more contacts than the local buffer: again into the slab
+    }
+    if (n <= kmax) {
+      const int* src = (const int*)loc;
+      int* dst = (int*)(W.contacts + base);
+      for (int w = lane; w < n * (int)(sizeof(ContactRec<R>) / 4); w += 64) dst[w] = src[w];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");   // (the lanes read each other's records)
+    const ContactRec<R>* rec = n > kmax ? (const ContactRec<R>*)W.contacts + base : loc;
+    int nc = 0, nf = 0;
+    for (int k0 = 0; k0 < n; k0 += 64) {
+      const int fl = k0 + lane < n ? rec[k0 + lane].flags : 0;
+      nc += __popcll(__ballot(fl & 1));
+      nf += 2 * __popcll(__ballot((fl & 3) == 3));
+    }
     if (lane == 0) {
-      if (ctx.status) ws_fail(W.counters, ctx.status);
-      if (n > 0) base = atomicAdd(&W.counters[C_STAGING], n);
+      W.pc_cnt[p] = n;
+      W.pc_base[p] = base;
+      W.pf_cnt[p] = nf;
+      W.pc_off[p] = nc;
     }
-    base = __shfl(base, 0, 64);
-    if (n > 0 && base + n > W.contact_cap) {
-      if (lane == 0) ws_fail(W.counters, WS_CONTACTS);
-      n = 0;
-    } else if (n > kmax) {  // more contacts than the local buffer: run the pair again into the slab
-      Sink<R, true> s2{W.contacts + base, n, 0, 0};
-      NPCtx<R, true, KINDS> ctx2(W, dt, &s2, ws);
-      ctx2.clip_cap = clip_cap;
-      ctx2.pair(bi, bj);
-    } else if (lane == 0) {
-      for (int k = 0; k < n; k++) W.contacts[base + k] = loc[k];
-    }
-    if (lane == 0) pair_counts(W, p, n, base);
     // the next pair reuses the workspace and the buffer
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -1757,15 +1781,7 @@ template <typename R> __device__ __forceinline__ R gs_row(const GsRow<R>& cr, fl
 }
 
 // values of the other lanes of a row's four (CTRL: a DPP quad permutation)
-template <int CTRL> __device__ __forceinline__ float quad(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
-}
-template <int CTRL> __device__ __forceinline__ double quad(double v) {
-  const long long x = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
+template <int CTRL, typename T> __device__ __forceinline__ T quad(T v) { return dpp<CTRL>(v); }
 constexpr int QP_SWAP1 = 0xB1, QP_SWAP2 = 0x4E;   // [1,0,3,2] [2,3,0,1]
 constexpr int QP_LANE0 = 0x00, QP_LANE1 = 0x55, QP_LANE3 = 0xFF, QP_LANES0033 = 0xF0;   // [0,..] [1,..] [3,..] [0,0,3,3]
 // v with its sign flipped where the top bit of m is set
