@@ -875,18 +875,7 @@ static int upload_list(chp_ctx* ctx, const std::vector<int>& list) {
   }
   ctx->h_list = list;
   HIPCHK(ctx, hipMemcpyAsync(ctx->d_list, ctx->h_list.data(), n * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-  {  // lists are sorted by body count, largest first (or hold one world)
-    auto lead = [&](int nb_over) {
-      size_t k = 0;
-      while (k < n && (int)ctx->worlds[list[k]].nb > nb_over) k++;
-      return (int)k;
-    };
-    GsSegs& g = ctx->gsg;
-    g.blk = lead(GS_SUB_MAX_NB);
-    g.wave = lead(GS_WAVE_NB);
-    g.nb_sub = g.wave > g.blk ? ctx->worlds[list[g.blk]].nb : 0;
-    g.nb_wave = (int)n > g.wave ? ctx->worlds[list[g.wave]].nb : 0;
-  }
+  ctx->gsg = gs_segs((int)n, [&](int k) { return (int)ctx->worlds[list[k]].nb; });
   std::vector<int> spans, tiles, bigw;
   int max_tiles = 1;
   size_t bodies = 0;
@@ -1395,10 +1384,7 @@ template <typename R> static int step_noalloc_t(chp_ctx* ctx, uint32_t id, doubl
   V.n_joints = S.joints ? 1 : 0;
   V.classes = step_classes(S);
   V.few = S.nb <= NP_FEW_BODIES;
-  V.gsg.blk = S.nb > GS_SUB_MAX_NB ? 1 : 0;
-  V.gsg.wave = S.nb > GS_WAVE_NB ? 1 : 0;
-  V.gsg.nb_sub = V.gsg.wave > V.gsg.blk ? S.nb : 0;
-  V.gsg.nb_wave = V.gsg.wave ? 0 : S.nb;
+  V.gsg = gs_segs(1, [&](int) { return (int)S.nb; });
   V.qcls = (int*)(base + o_qcls);
   V.q = (int2*)(base + o_q);
   V.qcap = (size_t)S.pair_cap;

@@ -278,7 +278,13 @@ __global__ __launch_bounds__(64) void k_joint_rows(const DevWorld<R>* __restrict
 // at most GS_SUB_MAX_NB one per workgroup of four waves, all of them in one launch; larger ones
 // one per workgroup of their own launch.  vlambda / wlambda and the step tables live in LDS where
 // they fit.
-constexpr int GS_SUB_MAX_NB = 512, GS_WAVE_NB = 128;
+// Worlds of at most GS_ONE_NB join the second launch while there is a CU for each of its workgroups:
+// a list on both sides of GS_SUB_MAX_NB then waits for one launch, not two in turn (24 terrains of
+// 16 to 1024 bodies 287 us for 333 + 213), and four waves wait less at a step's barrier than eight
+// (600 bodies 137 -> 110 us, 900 159 -> 140, 1000 in double 678 -> 474, a 3000-body pile 914 -> 668;
+// of a lattice of 3000 spheres, whose levels are wide, 1186 -> 1230).  At 16,384 bodies, whose
+// velocities are not in LDS, eight are better (3.5 ms, four 3.9).
+constexpr int GS_SUB_MAX_NB = 512, GS_WAVE_NB = 128, GS_ONE_NB = 4096, GS_ONE_WGS = 256;
 constexpr int GS_SS_WAVE = 1024, GS_SS_SUB = 2048, GS_SS_BIG = 4096;   // step table entries in LDS
 // ring depth: FP32 4, 6 and 8 measured 1188, 1165 and 1186 us on 1024 chains, 338, 329 and 324 us
 // on half a batch of 2048 piles, 60, 62 and 66 us on one 217-body world
@@ -286,11 +292,27 @@ template <typename R> constexpr int gs_depth() { return sizeof(R) == 4 ? 6 : 2; 
 
 // the list positions of a list sorted by body count (largest first): [0, blk) over
 // GS_SUB_MAX_NB bodies, [blk, wave) a workgroup each, [wave, n) a wave each; and the largest body
-// count of the last two
+// count of the last two; one: the worlds over GS_ONE_NB, nb_one: the next world's body count
 struct GsSegs {
-  int blk = 0, wave = 0;
-  int nb_sub = 0, nb_wave = 0;
+  int blk = 0, wave = 0, one = 0;
+  int nb_sub = 0, nb_wave = 0, nb_one = 0;
 };
+// nb(k): body count of the k-th of n worlds
+template <class NB> static GsSegs gs_segs(int n, NB nb) {
+  auto lead = [&](int nb_over) {
+    int k = 0;
+    while (k < n && nb(k) > nb_over) k++;
+    return k;
+  };
+  GsSegs g;
+  g.one = lead(GS_ONE_NB);
+  g.blk = lead(GS_SUB_MAX_NB);
+  g.wave = lead(GS_WAVE_NB);
+  g.nb_one = g.one < n ? nb(g.one) : 0;
+  g.nb_sub = g.wave > g.blk ? nb(g.blk) : 0;
+  g.nb_wave = g.wave < n ? nb(g.wave) : 0;
+  return g;
+}
 static size_t lds_gs_sub(const GsSegs& g) {
   const size_t sub = (size_t)(g.nb_sub + 1) * 8 * sizeof(float) + GS_SS_SUB * sizeof(int);
   const size_t wave = (size_t)(g.nb_wave + 1) * 8 * sizeof(float) + GS_SS_WAVE * sizeof(int);
@@ -424,8 +446,14 @@ __global__ __launch_bounds__(64 * NW) void k_gs(const DevWorld<R>* __restrict__ 
 // large world runs at a time (64, 128 or 256: four lanes each).  SELF: the rows may hold one whose
 // two bodies are one (the Solver slot)
 template <typename R, bool SELF = false>
-static void launch_gs(const DevWorld<R>* dw, const int* d_list, int n, const GsSegs& g, int max_nb, size_t max_lds, int rows,
+static void launch_gs(const DevWorld<R>* dw, const int* d_list, int n, const GsSegs& segs, int max_nb, size_t max_lds, int rows,
                       int keep, hipStream_t st) {
+  GsSegs g = segs;
+  if (g.blk > g.one && (g.wave - g.one) + (n - g.wave + 3) / 4 <= GS_ONE_WGS &&
+      (size_t)(g.nb_one + 1) * 8 * sizeof(float) + GS_SS_SUB * sizeof(int) + 4096 <= max_lds) {
+    g.blk = g.one;
+    g.nb_sub = g.nb_one;
+  }
   if (g.blk) {
     const int cap = big_lds_cap(max_nb, max_lds);
     const size_t lds = GS_SS_BIG * sizeof(int) + (size_t)(cap + 1) * 8 * sizeof(float);

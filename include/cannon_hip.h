@@ -282,8 +282,9 @@ int chp_sync(chp_ctx* ctx);
 int chp_last_step_ms(chp_ctx* ctx, double* ms);
 /* launch shape of the GS and level stages: workgroup sizes (64, 128 or 256; 0 keeps).  The level
  * stage gives a world of over 128 bodies a workgroup and smaller worlds one wave each; the GS
- * stage gives a world of over 512 bodies a workgroup (solve_block threads) and smaller worlds
- * 16, 32 or 64 lanes each (fixed).  Results do not depend on the choice (the GS schedule is exact
+ * stage runs a world of over 512 bodies (over 4096 while the list's other worlds leave CUs free)
+ * solve_block rows at a time, four lanes a row, and smaller worlds by four waves or, to 128 bodies,
+ * one (fixed).  Results do not depend on the choice (the GS schedule is exact
  * whatever the grouping). */
 int chp_ctx_set_tuning(chp_ctx* ctx, int solve_block, int levels_block);
 /* Autotuner: the next waited chp_step runs the level and GS stages of its first step once per
