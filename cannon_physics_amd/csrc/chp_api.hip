@@ -290,7 +290,7 @@ struct chp_ctx {
   struct StepGraph {
     bool valid = false;
     std::vector<int> list;
-    int nbig = 0, max_nb = 0, bl = 0, bg = 0;
+    int max_nb = 0, bl = 0, bg = 0;
     bool keep = false;
     double dt = 0;
     const void *dq = nullptr, *dqcls = nullptr, *dlist = nullptr, *dworlds = nullptr, *dbig = nullptr;
@@ -324,7 +324,6 @@ struct chp_ctx {
   std::deque<uint64_t> queue;      // waiting for admission, in arrival order
   std::vector<uint64_t> running;
   uint64_t next_ticket = 1;
-  int lds_cap_bodies = 2048;
 };
 
 // the context's list state <-> the second stream's
@@ -1030,7 +1029,7 @@ static const int kTuneBlocks[3] = {64, 128, 256};
 // the stage kernels of one step.  tune: the level and GS stages run once per candidate
 // workgroup size, timed by ctx->tev (they rebuild the same schedule from the same rows, so every
 // run leaves the same result)
-template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, int n, int nbig, int max_nb, double dt,
+template <typename R> static int launch_step(chp_ctx* ctx, const StepView& V, int n, int max_nb, double dt,
                                              hipEvent_t* ev, bool tune = false) {
   const DevWorld<R>* dw = (const DevWorld<R>*)V.worlds;
   const int* d_list = V.list;
@@ -1116,18 +1115,18 @@ static std::array<int, 11> step_shape(const chp_ctx* ctx) {
 // the captured step for this configuration (captured anew when anything baked into its kernel
 // arguments changed)
 template <typename R>
-static int step_graph(chp_ctx* ctx, const std::vector<int>& list, int nbig, int max_nb, double dt, bool may_capture,
+static int step_graph(chp_ctx* ctx, const std::vector<int>& list, int max_nb, double dt, bool may_capture,
                       hipGraphExec_t* out) {
   chp_ctx::StepGraph& g = ctx->sg;
   *out = nullptr;
-  if (!(g.valid && g.list == list && g.nbig == nbig && g.max_nb == max_nb && g.dt == dt && g.bl == ctx->levels_block && g.keep == ctx->keep_rows &&
+  if (!(g.valid && g.list == list && g.max_nb == max_nb && g.dt == dt && g.bl == ctx->levels_block && g.keep == ctx->keep_rows &&
         g.bg == ctx->solve_block && g.dq == ctx->d_q && g.dqcls == ctx->d_qcls && g.dlist == ctx->d_list &&
         g.dbig == ctx->d_big && g.big == step_shape(ctx) &&
         g.dworlds == ctx->d_worlds)) {
     if (!may_capture) return CHP_OK;
     drop_graph(ctx);
     HIPCHK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed));
-    int r = launch_step<R>(ctx, ctx_view(ctx), (int)list.size(), nbig, max_nb, dt, nullptr);
+    int r = launch_step<R>(ctx, ctx_view(ctx), (int)list.size(), max_nb, dt, nullptr);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(ctx->stream, &graph);
     if (r != CHP_OK) { if (graph) (void)hipGraphDestroy(graph); return r; }
@@ -1138,7 +1137,7 @@ static int step_graph(chp_ctx* ctx, const std::vector<int>& list, int nbig, int 
       (void)hipGraphDestroy(graph);
       return fail(ctx, CHP_E_HIP, std::string("step graph: ") + hipGetErrorString(e));
     }
-    g.valid = true; g.list = list; g.nbig = nbig; g.max_nb = max_nb; g.dt = dt;
+    g.valid = true; g.list = list; g.max_nb = max_nb; g.dt = dt;
     g.bl = ctx->levels_block; g.bg = ctx->solve_block; g.keep = ctx->keep_rows;
     g.dq = ctx->d_q; g.dqcls = ctx->d_qcls; g.dlist = ctx->d_list; g.dworlds = ctx->d_worlds;
     g.dbig = ctx->d_big; g.big = step_shape(ctx);
@@ -1173,10 +1172,8 @@ static int run_split(chp_ctx* ctx, const std::vector<int>& list, double dt, int 
                      const uint32_t* ids, uint32_t n, std::vector<int>* status) {
   std::vector<int> part[2];
   for (size_t k = 0; k < list.size(); k++) part[k & 1].push_back(list[k]);
-  int nbig[2], max_nb[2];
+  int max_nb[2];
   for (int h = 0; h < 2; h++) {
-    nbig[h] = 0;
-    while (nbig[h] < (int)part[h].size() && ctx->worlds[part[h][nbig[h]]].nb > SMALL_NB) nbig[h]++;
     max_nb[h] = ctx->worlds[part[h][0]].nb;
     std::vector<uint32_t> pid(part[h].begin(), part[h].end());
     if (h) swap_lists(ctx);
@@ -1191,10 +1188,10 @@ static int run_split(chp_ctx* ctx, const std::vector<int>& list, double dt, int 
   HIPCHK(ctx, hipEventRecord(ctx->ev_fork, ctx->stream));
   HIPCHK(ctx, hipStreamWaitEvent(ctx->second.stream, ctx->ev_fork, 0));
   for (int s = 0; s < nsteps; s++) {
-    int r = launch_step<R>(ctx, ctx_view(ctx), (int)part[0].size(), nbig[0], max_nb[0], dt, nullptr);
+    int r = launch_step<R>(ctx, ctx_view(ctx), (int)part[0].size(), max_nb[0], dt, nullptr);
     if (r != CHP_OK) return r;
     swap_lists(ctx);
-    r = launch_step<R>(ctx, ctx_view(ctx), (int)part[1].size(), nbig[1], max_nb[1], dt, nullptr);
+    r = launch_step<R>(ctx, ctx_view(ctx), (int)part[1].size(), max_nb[1], dt, nullptr);
     swap_lists(ctx);
     if (r != CHP_OK) return r;
   }
@@ -1221,8 +1218,6 @@ template <typename R> static int run_steps(chp_ctx* ctx, const uint32_t* ids, ui
     return run_split<R>(ctx, list, dt, nsteps, wait, ids, n, status);
   r = ensure_queue(ctx, ids, n);
   if (r != CHP_OK) return r;
-  int nbig = 0;
-  while (nbig < (int)n && ctx->worlds[list[nbig]].nb > SMALL_NB) nbig++;
   r = upload_list(ctx, list);
   if (r != CHP_OK) return r;
   size_t nev = ctx->profile ? (size_t)nsteps * (K_NSTAGE + 1) : 0;
@@ -1246,7 +1241,7 @@ template <typename R> static int run_steps(chp_ctx* ctx, const uint32_t* ids, ui
   ctx->prev_list = list;
   ctx->prev_dt = dt;
   if (ctx->use_graphs && !ctx->profile && nsteps > 1) {
-    r = step_graph<R>(ctx, list, nbig, max_nb, dt, stable || nsteps >= 16, &exec);
+    r = step_graph<R>(ctx, list, max_nb, dt, stable || nsteps >= 16, &exec);
     if (r != CHP_OK) return r;
   }
   HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
@@ -1255,7 +1250,7 @@ template <typename R> static int run_steps(chp_ctx* ctx, const uint32_t* ids, ui
       HIPCHK(ctx, hipGraphLaunch(exec, ctx->stream));
       continue;
     }
-    r = launch_step<R>(ctx, ctx_view(ctx), (int)n, nbig, max_nb, dt,
+    r = launch_step<R>(ctx, ctx_view(ctx), (int)n, max_nb, dt,
                        ctx->profile ? &ctx->sev[s * (K_NSTAGE + 1)] : nullptr, tune && s == 0);
     if (r != CHP_OK) return r;
   }
@@ -1301,7 +1296,7 @@ template <typename R> static int step_plain_t(chp_ctx* ctx, uint32_t id, double 
   if (r != CHP_OK) return r;
   HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
   for (int s = 0; s < nsteps; s++) {
-    r = launch_step<R>(ctx, ctx_view(ctx), 1, ctx->worlds[id].nb > SMALL_NB ? 1 : 0, ctx->worlds[id].nb, dt, nullptr);
+    r = launch_step<R>(ctx, ctx_view(ctx), 1, ctx->worlds[id].nb, dt, nullptr);
     if (r != CHP_OK) return r;
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // the slot-by-slot drop-in hands back each step
   }
@@ -1391,7 +1386,7 @@ template <typename R> static int step_noalloc_t(chp_ctx* ctx, uint32_t id, doubl
   k_queue_clear<<<1, 64, 0, ctx->stream>>>(V.qcls);
   HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
   for (int s = 0; s < nsteps; s++) {
-    r = launch_step<R>(ctx, V, 1, S.nb > SMALL_NB ? 1 : 0, S.nb, dt, nullptr);
+    r = launch_step<R>(ctx, V, 1, S.nb, dt, nullptr);
     if (r != CHP_OK) return r;
   }
   HIPCHK(ctx, hipEventRecord(ctx->ev1, ctx->stream));

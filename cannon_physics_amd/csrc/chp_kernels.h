@@ -330,7 +330,6 @@ static int big_lds_cap(int max_nb, size_t max_lds) {
 // (up to LV_ROWS_WAVE / LV_ROWS_SUB rows: 217 bodies 31 -> 12 us, half a batch of 2048 worlds
 // 149 -> 51 us); larger ones in a workgroup of 1024 threads of their own launch, whose passes over
 // the rows are what takes the time (16,384 bodies 2.35 -> 0.75 ms, with 256 threads before).
-constexpr int SMALL_NB = GS_WAVE_NB;
 constexpr int LV_ROWS_WAVE = 1024, LV_ROWS_SUB = 6144, LV_TB_SUB = 512, LV_TB_BIG = 1024;
 constexpr int LV_HIST_BIG = 4096;                // of a large world's level histogram in LDS
 static size_t lds_levels_sub(const GsSegs& g, int bd) {

@@ -136,8 +136,9 @@ struct Poly {
 enum : unsigned { NK_SS = 1, NK_SP = 2, NK_SB = 4, NK_SC = 8, NK_SH = 16, NK_PC = 32, NK_CC = 64, NK_HC = 128,
                   NK_ALL = 255 };
 
-// A resolver context.  WAVE: a whole wave runs one pair, every lane on the same data unless said otherwise (so every
-// branch is uniform), and the separating-axis search splits its axes over the lanes.
+// A resolver context.  WAVE: a whole wave runs one pair, every lane on the same data where not said
+// otherwise (so every branch is uniform), and the separating-axis search splits its axes over the
+// lanes.
 template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
   const DevWorld<R>& W;
   R dt;

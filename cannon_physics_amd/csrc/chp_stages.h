@@ -9,7 +9,6 @@
 
 namespace chp {
 
-#define CHP_BLOCK 256
 #define CHP_KMAX 8
 
 enum { C_STATUS = 0, C_PAIRS = 1, C_CONTACTS = 2, C_ROWS = 3, C_ITERS = 4, C_LEVELS = 5, C_STAGING = 6,
@@ -21,22 +20,6 @@ __device__ __forceinline__ void ws_fail(int* counters, int bit) { atomicOr(&coun
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// exclusive scan of one value per thread; sh needs blockDim.x ints
-__device__ __forceinline__ int block_exscan(int v, int* sh, int* total) {
-  int t = threadIdx.x, n = blockDim.x;
-  sh[t] = v;
-  __syncthreads();
-  for (int off = 1; off < n; off <<= 1) {
-    int x = t >= off ? sh[t - off] : 0;
-    __syncthreads();
-    sh[t] += x;
-    __syncthreads();
-  }
-  int incl = sh[t];
-  *total = sh[n - 1];
-  __syncthreads();
-  return incl - v;
-}
 // in-place exclusive scan of data[0..n); returns the total (same value in every thread).  Each
 // wave scans a contiguous segment in coalesced rounds of 64 (a shuffle scan per round, a
 // running carry); a pass of wave sums ahead gives every segment its offset.  sh needs
