@@ -287,8 +287,10 @@ __global__ __launch_bounds__(64) void k_joint_rows(const DevWorld<R>* __restrict
 constexpr int GS_SUB_MAX_NB = 512, GS_WAVE_NB = 128, GS_ONE_NB = 4096, GS_ONE_WGS = 256;
 constexpr int GS_SS_WAVE = 1024, GS_SS_SUB = 2048, GS_SS_BIG = 4096;   // step table entries in LDS
 // ring depth: FP32 4, 6 and 8 measured 1188, 1165 and 1186 us on 1024 chains, 338, 329 and 324 us
-// on half a batch of 2048 piles, 60, 62 and 66 us on one 217-body world
-template <typename R> constexpr int gs_depth() { return sizeof(R) == 4 ? 6 : 2; }
+// on half a batch of 2048 piles, 60, 62 and 66 us on one 217-body world; FP64 2, 3 and 4 measured
+// 251, 211 and 213 us on a 157-body world, 474, 397 and 398 us on 1000 bodies, 645, 398 and 395 us
+// on half a batch of 512 piles
+template <typename R> constexpr int gs_depth() { return sizeof(R) == 4 ? 6 : 4; }
 
 // the list positions of a list sorted by body count (largest first): [0, blk) over
 // GS_SUB_MAX_NB bodies, [blk, wave) a workgroup each, [wave, n) a wave each; and the largest body
