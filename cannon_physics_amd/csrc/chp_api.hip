@@ -294,7 +294,7 @@ struct chp_ctx {
     bool keep = false;
     double dt = 0;
     const void *dq = nullptr, *dqcls = nullptr, *dlist = nullptr, *dworlds = nullptr, *dbig = nullptr;
-    std::array<int, 11> big{};
+    std::array<int, 17> big{};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
   } sg;
@@ -1106,10 +1106,13 @@ static void drop_graph(chp_ctx* ctx) {
   ctx->sg = chp_ctx::StepGraph();
 }
 
-// what of the list decides which kernels a step launches, and their grids
-static std::array<int, 11> step_shape(const chp_ctx* ctx) {
+// what of the list decides which kernels a step launches, their grids, their LDS and the segments
+// they are given.  The ids of the list do not: a destroyed world's id goes to the next one created,
+// whatever its size
+static std::array<int, 17> step_shape(const chp_ctx* ctx) {
+  const GsSegs& g = ctx->gsg;
   return {ctx->big_nspans, ctx->big_ntiles, ctx->big_nw, ctx->big_rounds, ctx->n_sap, ctx->n_sleep, ctx->n_events, ctx->n_split,
-          ctx->n_joints, (int)ctx->classes, ctx->few ? 1 : 0};
+          ctx->n_joints, (int)ctx->classes, ctx->few ? 1 : 0, g.blk, g.wave, g.one, g.nb_sub, g.nb_wave, g.nb_one};
 }
 
 // the captured step for this configuration (captured anew when anything baked into its kernel
