@@ -1262,14 +1262,15 @@ template <typename R> static int run_steps(chp_ctx* ctx, const uint32_t* ids, ui
   ctx->stage_ms.assign(K_NSTAGE, 0.0);
   if (!wait && !ctx->profile) return CHP_OK;
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  if (tune) {  // keep the fastest workgroup size of each stage
+  if (tune) {  // keep the fastest workgroup size of each stage (of the sweeps', where some world's depends on it)
+    const bool sized = gs_launch_segs(ctx->gsg, (int)n, ctx->max_lds).blk > 0;
     float bestl = 1e30f, bestg = 1e30f;
     for (int c = 0; c < 3; c++) {
       float tl = 0, tg = 0;
       HIPCHK(ctx, hipEventElapsedTime(&tl, ctx->tev[3 * c], ctx->tev[3 * c + 1]));
       HIPCHK(ctx, hipEventElapsedTime(&tg, ctx->tev[3 * c + 1], ctx->tev[3 * c + 2]));
       if (tl < bestl) { bestl = tl; ctx->levels_block = kTuneBlocks[c]; }
-      if (tg < bestg) { bestg = tg; ctx->solve_block = kTuneBlocks[c]; }
+      if (sized && tg < bestg) { bestg = tg; ctx->solve_block = kTuneBlocks[c]; }
     }
     ctx->tune_pending = false;
   }

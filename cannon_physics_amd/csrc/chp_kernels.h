@@ -443,18 +443,23 @@ __global__ __launch_bounds__(64 * NW) void k_gs(const DevWorld<R>* __restrict__ 
     st_gs<R, NW, D, false, SELF, false>(W, W.vw, ss, shd, sh, keep != 0);
 }
 
+// the segments the sweeps are launched by: worlds of at most GS_ONE_NB bodies join the small ones'
+// launch by the rule above.  What is left in [0, blk) is what launch_gs' `rows` applies to
+static GsSegs gs_launch_segs(GsSegs g, int n, size_t max_lds) {
+  if (g.blk > g.one && (g.wave - g.one) + (n - g.wave + 3) / 4 <= GS_ONE_WGS &&
+      (size_t)(g.nb_one + 1) * 8 * sizeof(float) + GS_SS_SUB * sizeof(int) + 4096 <= max_lds) {
+    g.blk = g.one;
+    g.nb_sub = g.nb_one;
+  }
+  return g;
+}
 // the GS stage of a list (the level schedule and the GS records are in place).  rows: rows a
 // large world runs at a time (64, 128 or 256: four lanes each).  SELF: the rows may hold one whose
 // two bodies are one (the Solver slot)
 template <typename R, bool SELF = false>
 static void launch_gs(const DevWorld<R>* dw, const int* d_list, int n, const GsSegs& segs, int max_nb, size_t max_lds, int rows,
                       int keep, hipStream_t st) {
-  GsSegs g = segs;
-  if (g.blk > g.one && (g.wave - g.one) + (n - g.wave + 3) / 4 <= GS_ONE_WGS &&
-      (size_t)(g.nb_one + 1) * 8 * sizeof(float) + GS_SS_SUB * sizeof(int) + 4096 <= max_lds) {
-    g.blk = g.one;
-    g.nb_sub = g.nb_one;
-  }
+  const GsSegs g = gs_launch_segs(segs, n, max_lds);
   if (g.blk) {
     const int cap = big_lds_cap(max_nb, max_lds);
     const size_t lds = GS_SS_BIG * sizeof(int) + (size_t)(cap + 1) * 8 * sizeof(float);

@@ -289,7 +289,8 @@ int chp_last_step_ms(chp_ctx* ctx, double* ms);
 int chp_ctx_set_tuning(chp_ctx* ctx, int solve_block, int levels_block);
 /* Autotuner: the next waited chp_step runs the level and GS stages of its first step once per
  * workgroup size (64, 128, 256), times them with HIP events and keeps the fastest of each
- * (every run leaves the same result, so the step is the step chp_step would take). */
+ * (every run leaves the same result, so the step is the step chp_step would take).  solve_block
+ * stays as it is when no listed world's GS stage takes it. */
 int chp_ctx_autotune(chp_ctx* ctx);
 int chp_ctx_get_tuning(chp_ctx* ctx, int* solve_block, int* levels_block);
 /* on: chp_step with nsteps > 1 captures one step's kernels in a hipGraph and replays it for each

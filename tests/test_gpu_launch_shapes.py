@@ -119,3 +119,18 @@ def test_slots_of_large_worlds(bodies, side, mode):
         assert it == oit and np.array_equal(bits(mult), bits(omult)) and same(c, wid, ow)
     finally:
         c.close()
+
+
+# the autotuner leaves the sweeps' size alone where no sweep of the list depends on it
+@pytest.mark.parametrize("bodies", [40, 600])
+def test_autotune_of_lists_without_sized_sweeps(bodies):
+    c = Context(device=0)
+    try:
+        ids = [create(c, heap(bodies, 0.9 * bodies ** (1 / 3))) for _ in range(3)]
+        for solve in (64, 128, 256):
+            c.set_tuning(solve_block=solve, levels_block=128)
+            c.autotune()
+            c.step(ids, DT, 2)
+            assert c.tuning()["solve_block"] == solve
+    finally:
+        c.close()
