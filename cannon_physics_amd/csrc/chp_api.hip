@@ -283,7 +283,8 @@ struct chp_ctx {
   bool profile = false;                      // per-stage events in chp_step
   std::vector<hipEvent_t> sev;               // 7 events per step
   std::vector<double> stage_ms;              // accumulated per stage over the last chp_step
-  // workgroup sizes of k_levels / k_gs: one large world, or blockDim/64 small ones, per workgroup
+  // levels_block: threads of a k_levels_sub workgroup, a quarter of a k_levels one's; solve_block:
+  // rows k_gs runs at a time (four lanes each)
   int levels_block = 256, solve_block = 128;
   bool tune_pending = false;                 // time the candidates in the next waited step
   // hipGraph of one step of the last batched configuration, replayed once per step
@@ -496,7 +497,6 @@ static int build_slot(chp_ctx* ctx, WorldSlot& S, const HostWorld<R>& H, int pai
   while (np2 < nb) np2 <<= 1;
   SCR(pair_i, int, pair_cap); SCR(pair_j, int, pair_cap); SCR(cnt, int, nb); SCR(tmp, int, nb);
   SCR(pc_cnt, int, pair_cap); SCR(pc_base, int, pair_cap); SCR(pf_cnt, int, pair_cap); SCR(pc_off, int, pair_cap);
-  SCR(pf_off, int, 1);
   SCR(contacts, ContactRec<R>, contact_cap);
   SCR(rows, RowRec<R>, row_cap);
   SCR(level, int, row_cap); SCR(sched, int, row_cap); SCR(lvl_start, int, row_cap + 2);

@@ -527,8 +527,8 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     depth = d0 < d1 ? d0 : d1;
     return true;
   }
-  // findSeparatingAxis (:232-356); face0_only: faceListA = [0].  Hulls of at most 8 vertices are
-  // projected from registers.
+  // findSeparatingAxis (:232-356); face0_only: faceListA = [0] (heightfield pillars, which are wave
+  // pairs).  A thread projects hulls of at most 8 vertices from registers.
   CHP_HD static bool findSepAxis(const HullView<R>& A, const HullView<R>& B, f3 pa, f4 qa, f3 pb, f4 qb, bool face0_only,
                                  f3& target) {
     if constexpr (WAVE) {
@@ -537,20 +537,19 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     } else {
       if (A.nv <= 8 && B.nv <= 8) {
         const HullVerts8 va = verts8(A), vb = verts8(B);
-        return findSepAxisT(A, va, B, vb, pa, qa, pb, qb, face0_only, target);
+        return findSepAxisT(A, va, B, vb, pa, qa, pb, qb, target);
       }
-      return findSepAxisT(A, A, B, B, pa, qa, pb, qb, face0_only, target);
+      return findSepAxisT(A, A, B, B, pa, qa, pb, qb, target);
     }
   }
   template <class VS>
   CHP_HD static bool findSepAxisT(const HullView<R>& A, const VS& vA, const HullView<R>& B, const VS& vB, f3 pa, f4 qa,
-                                  f3 pb, f4 qb, bool face0_only, f3& target) {
+                                  f3 pb, f4 qb, f3& target) {
     R dmin = (R)__builtin_huge_val();
     const f3 zero = mk3(0.f, 0.f, 0.f);
     f3 loA = point_to_local<R>(pa, qa, zero), loB = point_to_local<R>(pb, qb, zero);
     if (A.axes) {
-      int nA = face0_only ? 1 : A.nf;
-      for (int i = 0; i < nA; i++) {
+      for (int i = 0; i < A.nf; i++) {
         f3 n = qrot<R>(qa, A.fn[i]);
         R d;
         if (!testSepAxis(vA, n, vB, loA, qa, loB, qb, d)) return false;
@@ -980,7 +979,8 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
         if (sink->n - before > 2) return;
       }
   }
-  // heightfieldConvex and convexConvex by a wave: the second shape is the heightfield hf (hf >= 0), whose
+  // heightfieldConvex (:2044-2178: convexConvex against each pillar with faceListA = [0]; wave pairs
+  // only) and convexConvex by a wave: the second shape is the heightfield hf (hf >= 0), whose
   // pillars near the hull are taken in turn, or the hull hullB.  One loop and one call for both:
   // the resolvers' code, not their data, is what a launch of a few thousand pairs waits for
   __device__ void hullPairsWave(const HullView<R>& A, SRef siRef, int hf, int hullB, SRef sjRef, f3 xi, f3 xj, f4 qi, f4 qj,
@@ -1040,25 +1040,6 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
         convexConvex(A, siRef, H, field ? pref : sjRef, xi, wpo, qi, qj, bi, bj, field ? siRef : rsi, field ? pref : rsj, field);
       }
     }
-  }
-  // heightfieldConvex (:2044-2178): convexConvex against each pillar with faceListA = [0]
-  CHP_HD void heightfieldConvex(const HullView<R>& A, SRef siRef, int hf, int hfId, f3 xi, f3 xj, f4 qi, f4 qj, int bi,
-                                int bj) {
-    f3 local = point_to_local<R>(xj, qj, xi);
-    int x0, x1, y0, y1;
-    R mn, mx;
-    R radius = A.bsr;
-    if (!hfWindow(hf, local, radius, x0, x1, y0, y1, mn, mx)) return;
-    if (ld<R>(local.z) - radius > mx || ld<R>(local.z) + radius < mn) return;
-    SRef pref{1, -1, hfId};   // the pillar hull; its contacts name the heightfield
-    for (int i = x0; i < x1; i++)
-      for (int j = y0; j < y1; j++)
-        for (int up = 0; up < 2; up++) {
-          int h = pillarHull(hf, i, j, up);
-          HullView<R> H = hull_view(W, h);
-          f3 wpo = point_to_world<R>(xj, qj, pillarOff(hf, i, j, up));
-          if (dist3<R>(xi, wpo) < H.bsr + A.bsr) convexConvex(A, siRef, H, pref, xi, wpo, qi, qj, bi, bj, siRef, pref, true);
-        }
   }
 
   // Narrowphase.getContacts for one broadphase pair (narrow_phase.dart:654-719)
@@ -1144,8 +1125,6 @@ template <typename R, bool WAVE = false, unsigned KINDS = NK_ALL> struct NPCtx {
     }
     else if (!WAVE && (KINDS & NK_CC) && convA && (tb == CHP_SHAPE_BOX || tb == CHP_SHAPE_CONVEX))
       convexConvex(hull_view(W, W.si_hull[A]), ra, hull_view(W, W.si_hull[B]), rb, xa, xb, qa, qb, ba, bb, rsi, rsj, false);
-    else if (!WAVE && (KINDS & NK_HC) && convA && tb == CHP_SHAPE_HEIGHTFIELD)
-      heightfieldConvex(hull_view(W, W.si_hull[A]), ra, W.si_hf[B], B, xa, xb, qa, qb, ba, bb);
     // other combinations have no resolver in the covered set (narrow_phase.dart:699-700 skips)
   }
 };

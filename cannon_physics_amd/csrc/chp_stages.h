@@ -76,18 +76,6 @@ __device__ __forceinline__ int array_exscan(int* data, int n, int* sh) {
   __syncthreads();
   return tot;
 }
-template <typename R> __device__ __forceinline__ R block_sum(R v, R* sh) {
-  int t = threadIdx.x;
-  sh[t] = v;
-  __syncthreads();
-  for (int off = blockDim.x >> 1; off > 0; off >>= 1) {
-    if (t < off) sh[t] = sh[t] + sh[t + off];
-    __syncthreads();
-  }
-  R r = sh[0];
-  __syncthreads();
-  return r;
-}
 // flag bits of the body indices in the solver's row records
 enum : unsigned { GS_DYN = 0x80000000u, GS_IDX = 0x3fffffffu };
 
@@ -1255,9 +1243,8 @@ template <typename R> __device__ __forceinline__ void solve_finish_body(const De
 // bodies and run in parallel, and every row sees exactly the values it sees in the
 // sequential order.
 //
-// A world's levels and sweeps run on one group: a whole workgroup for a large world, a single
-// wave for a small one (four small worlds share a workgroup, one per wave, and never meet at a
-// workgroup barrier).
+// A world's levels run on one group: a whole workgroup for a large world, a single wave for a small
+// one (four small worlds share a workgroup, one per wave, and never meet at a workgroup barrier).
 
 // a whole workgroup on one world
 struct GBlock {
@@ -1265,17 +1252,6 @@ struct GBlock {
   __device__ GBlock() : tid(threadIdx.x), n(blockDim.x) {}
   __device__ void sync() const { __syncthreads(); }
   __device__ void lds_sync() const { lds_barrier(); }
-  __device__ double sum(double v, double* shd) const {
-    shd[tid] = v;
-    lds_barrier();
-    for (int off = n >> 1; off > 0; off >>= 1) {
-      if (tid < off) shd[tid] = shd[tid] + shd[tid + off];
-      lds_barrier();
-    }
-    double r = shd[0];
-    lds_barrier();
-    return r;
-  }
   __device__ int imax(int v, int* sh) const {
     __syncthreads();
     if (tid == 0) sh[0] = 0;
@@ -1286,16 +1262,7 @@ struct GBlock {
     __syncthreads();
     return r;
   }
-  __device__ int bcast0(int v, int* sh) const {
-    lds_barrier();
-    if (tid == 0) sh[0] = v;
-    lds_barrier();
-    int r = sh[0];
-    lds_barrier();
-    return r;
-  }
   __device__ int exscan(int* data, int cnt, int* sh) const { return array_exscan(data, cnt, sh); }
-  __device__ int uni(int v) const { return __builtin_amdgcn_readfirstlane(v); }
 };
 // one wave on one world: LDS and memory accesses of a wave are issued in program order, so a
 // fence that waits for them replaces the barrier
@@ -1304,16 +1271,10 @@ struct GWave {
   __device__ GWave() : tid(threadIdx.x & 63), n(64) {}
   __device__ void sync() const { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup"); }
   __device__ void lds_sync() const { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local"); }
-  __device__ double sum(double v, double*) const {
-    // fixed butterfly: every lane ends with the same value
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-  }
   __device__ int imax(int v, int*) const {
     for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
     return v;
   }
-  __device__ int bcast0(int v, int*) const { return __shfl(v, 0, 64); }
   __device__ int exscan(int* data, int cnt, int*) const {
     int carry = 0;
     for (int base = 0; base < cnt; base += 64) {
@@ -1329,7 +1290,6 @@ struct GWave {
     sync();
     return carry;
   }
-  __device__ int uni(int v) const { return __builtin_amdgcn_readfirstlane(v); }
 };
 // GS record: 6 groups of 4 words, row position k at words [k * 24, k * 24 + 24)
 //   g0 sa.x sa.y sa.z ima  | g1 ra.x ra.y ra.z B    | g2 rb.x rb.y rb.z invC
@@ -1872,7 +1832,9 @@ __device__ __forceinline__ void st_gs(const DevWorld<R>& W, float* vw, int* ss, 
     // permutations more), or all of it in each lane.  The word wins where the loads are what the
     // steps wait for and loses where one world's four waves wait for each other: half a batch
     // of 1024 chains 1167 -> 1063 us, of 2048 piles 334 -> 322, a 16,384-body world 4.01 -> 3.74 ms,
-    // a 300-body pile in double 290 -> 253, but in single 83 -> 92
+    // a 300-body pile in double 290 -> 253, but in single 83 -> 92.  Four waves in single take the
+    // whole group however many of their workgroups there are: the word was measured there on one
+    // world and on the piles' mixture, not on hundreds of worlds of four waves each
     constexpr bool WORD = sizeof(R) == 8 || NW != 4;
     GsQuad<R> qc[WORD ? 1 : D];
     WT qw[WORD ? D : 1];

@@ -125,7 +125,7 @@ template <typename R> struct DevWorld {
   CHP_G(float) feff, vl, wl, iiws;
   CHP_G(R) ims;
   CHP_G(int) pair_i, pair_j, cnt, tmp;
-  CHP_G(int) pc_cnt, pc_base, pf_cnt, pc_off, pf_off;
+  CHP_G(int) pc_cnt, pc_base, pf_cnt, pc_off;
   CHP_G(ContactRec<R>) contacts;
   CHP_G(RowRec<R>) rows;
   CHP_G(int) level, sched, lvl_start, last_level, row_ab, rpos;
